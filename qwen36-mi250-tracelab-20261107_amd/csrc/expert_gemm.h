@@ -40,6 +40,9 @@ struct GemmArgs {
   int topk, P, E, T;
   int nrb;           // weight-row blocks per tile (set by the launcher)
   int MTgrid;        // tiles the grid covers (set by the launcher)
+  int bm, nsub, nblk;  // rows per table tile, parts a tile is taken in, row blocks per
+                       // workgroup (set by the launchers)
+  unsigned in_bytes[2], out_bytes[2];  // of each operand's input and output (set by the launcher)
   int shared_first;  // the table's last shared_first tiles run first (set by the launcher)
 };
 
@@ -52,9 +55,27 @@ bool mixed_enabled();
 hipError_t launch_expert_gemm(int mode, int role, int bm, const GemmArgs& a, int max_tiles,
                               hipStream_t st);
 
-// Prefill tiles (prefill_gemm.hip): 256 sorted rows x 256 weight rows per workgroup, bf16.
+// Where the prefill kernels start their walk over the nch = K / 64 chunks of expert e's weight
+// rows (it wraps around). Workgroups run nearly in step, and weight rows lie a power of two
+// apart: all reading the same columns at once keeps few memory channels busy (streaming gate_up
+// at T = 777 / 1111, H = 2048: 199 / 211 us against 238 / 243 with one start for all). The start
+// is the weights' own and the same in every kernel that runs a projection, so that a row's
+// result does not depend on its batch.
+__host__ __device__ inline int prefill_start_chunk(int e, int nch) {
+  return nch % 4 ? 0 : e % (nch / 4) * 4;
+}
+
+// Prefill batches. launch_prefill_gemm (prefill_gemm.hip) takes tables of bm <= 256 sorted rows
+// per tile (prefill_tile_rows() for the grouped operations, prefill_block_rows for the fused
+// entry points) and passes what prefill_stream.hip does better on to it.
+constexpr int kStreamRowsSmall = 64, kStreamRowsLarge = 160;  // tiles of prefill_stream.hip
 int prefill_tile_rows();
+int prefill_block_rows(long long pairs, int experts, bool fp8);
 bool prefill_fits(int mode, const GemmOperand& op);
-hipError_t launch_prefill_gemm(int mode, const GemmArgs& a, int max_tiles, hipStream_t st);
+hipError_t launch_prefill_gemm(int mode, const GemmArgs& a, int max_tiles, int bm, hipStream_t st);
+// Whether the routed operand's shape and table suit the pipelined form of the streaming kernel.
+bool stream_takes(const GemmArgs& a, int bm);
+// a.bm and a.shared_first set; one weight type; prefill_fits operands.
+hipError_t launch_prefill_stream(int mode, const GemmArgs& a, int max_tiles, hipStream_t st);
 
 }  // namespace moe

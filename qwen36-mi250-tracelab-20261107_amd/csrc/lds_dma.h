@@ -56,6 +56,14 @@ __device__ __forceinline__ void dma16(const void* g, void* lds) {
   __builtin_amdgcn_global_load_lds(g, lds, 16, 0, 0);
 }
 
+// The same in buffer form: 16 bytes at byte offset voff (per lane) + soff (wave-uniform) of
+// the buffer. Loads past the buffer's end give zeros.
+__device__ __forceinline__ void dma16_buffer(__amdgpu_buffer_rsrc_t buf, void* lds, uint32_t voff,
+                                             uint32_t soff) {
+  typedef __attribute__((address_space(3))) void lds_void;
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, (lds_void*)lds, 16, voff, soff, 0, 0);
+}
+
 // The LDS byte address of a __shared__ / dynamic-shared pointer.
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
   typedef __attribute__((address_space(3))) const char lds_char;

@@ -1,4 +1,6 @@
-// Grouped MFMA GEMM for prefill-sized batches on gfx950 (subsystems a8, a9, a6).
+// Grouped MFMA GEMM for prefill-sized batches on gfx950, bf16 weights (subsystems a8, a9, a6).
+// prefill_stream.hip has the e4m3 form and the bf16 gate_up of batches with fewer rows per
+// expert.
 //
 // Same contract as k_expert_gemm (expert_gemm.hip) and the reference's grouped kernels
 // (engine/fast/moe_prefill.py:156-257): for a tile of up to 256 sorted rows of ONE expert,
@@ -125,9 +127,9 @@ __global__ __launch_bounds__(kThreads, 1) void k_prefill_gemm(GemmArgs args) {
     }
     e = args.table[tile];
     r0 = args.table[args.MT + tile];
-    // the table holds the expert's end row; this tile is its next PBM rows at most (the
-    // token-row ring stages hold PBM rows)
-    r1 = min(args.table[2 * args.MT + tile], r0 + PBM);
+    // the table holds the expert's end row; this tile is its next bm rows at most (bm <= PBM:
+    // the token-row ring stages hold PBM rows)
+    r1 = min(args.table[2 * args.MT + tile], r0 + args.bm);
   } else {
     e = args.E;
     r0 = args.P + tile * PBM;
@@ -182,8 +184,13 @@ __global__ __launch_bounds__(kThreads, 1) void k_prefill_gemm(GemmArgs args) {
   }
   char* lds = reinterpret_cast<char*>(smem);
   char* bring_lds = lds + kStagesA * kOpStage;
+  const int nd = op.K / DKC;
+  // gate_up's K order is the streaming kernel's (down runs here alone)
+  const int rot = MODE == kModeSwiglu && routed ? prefill_start_chunk(e, nd) : 0;
+  auto chunk = [&](int d) { return d + rot < nd ? d + rot : d + rot - nd; };
   auto issue_a = [&](int d) {
     char* st = lds + (d % kStagesA) * kOpStage;
+    d = chunk(d);
 #pragma unroll
     for (int i = 0; i < kLoadsPerWave; ++i)
       __builtin_amdgcn_global_load_lds(srca[i] + d * DKC, st + (wave + 8 * i) * 1024, 16, 0,
@@ -195,6 +202,7 @@ __global__ __launch_bounds__(kThreads, 1) void k_prefill_gemm(GemmArgs args) {
       min(kLoadsPerWave, max(0, ((r1 - r0 + 7) / 8 - wave + 7) / 8)));
   auto issue_b = [&](int d) {
     char* st = bring_lds + (d % kStagesB) * kOpStage;
+    d = chunk(d);
 #pragma unroll
     for (int i = 0; i < kLoadsPerWave; ++i)
       if (i < nb_loads)
@@ -221,7 +229,6 @@ __global__ __launch_bounds__(kThreads, 1) void k_prefill_gemm(GemmArgs args) {
   // rows are requested three chunks before use, token rows two. The prologue issues A(0),
   // B(0), A(1), B(1), A(2) — the order the steps would have — so the loads younger than a
   // chunk's B load are exactly the next A load.
-  const int nd = op.K / DKC;
   const int nk = 2 * nd;
   issue_a(0);
   if (nd > 0) issue_b(0);
@@ -299,299 +306,16 @@ __global__ __launch_bounds__(kThreads, 1) void k_prefill_gemm(GemmArgs args) {
   }
 }
 
-// ---------------------------------------------------------------- fp8-e4m3 weights
-//
-// The same tiles (256 weight rows x up to 256 sorted rows) with e4m3 weight bytes and
-// per-output-row fp32 scales on the fp32 accumulator. A DMA chunk is 64 k as in the bf16
-// kernel, so the token-row stages are the bf16 kernel's (256 rows x 128 bytes), while a
-// weight stage is 256 rows x 64 bytes (16 KiB): the ring holds five of them (four chunks
-// requested ahead, 144 KiB of LDS in all). A weight DMA load of a wave fills 16 rows x 64
-// bytes; lane l writes physical 16-byte unit l & 3 of row l >> 2 of its group, holding
-// logical unit (l & 3) ^ ((row >> 1) & 3), which keeps the fragment reads (8 rows of one
-// 16-byte read group) conflict-free.
-//
-// The weight loads use the default cache policy: unlike the bf16 kernel's, the non-temporal
-// one measured slower here (grouped gate_up / down at 4096 tokens 261 / 189 against 248 /
-// 181 µs). A deeper or shallower weight ring (6 or 4 stages) changed little.
-//
-// The chunk's k order is permuted the same way in both operands (the same products are
-// summed): lane group kq reads weight unit kq (16 e4m3 bytes, one ds_read_b128) once per
-// chunk and feeds its first 8 bytes to the chunk's k-step 0 and its last 8 to k-step 1,
-// against token units 2 kq and 2 kq + 1. The weights are widened to bf16 in registers
-// (gfx950's scaled conversion, scale 1: exact) just before their MFMAs.
-namespace {
-constexpr int F8RowBytes = DKC;                   // weight bytes of a row per chunk: 64
-constexpr int F8Stage = 256 * F8RowBytes;         // 16 KiB
-constexpr int F8StagesA = 5, F8AheadA = 4;
-constexpr int F8ALoads = 256 / 16 / 8;            // weight DMA loads per wave per chunk: 2
-constexpr int F8LdsBytes = F8StagesA * F8Stage + kStagesB * kOpStage;  // 144 KiB
-static_assert(F8AheadA == F8StagesA - 1, "weight ring: chunk d + S - 1 into chunk d - 1's stage");
-}  // namespace
-
-// 8 e4m3 bytes -> bf16x8 (exact)
-__device__ __forceinline__ u32x4v widen8(uint32_t lo, uint32_t hi) {
-  u32x4v r;
-  r.x = fp8x2_to_bf16x2<false>(lo);
-  r.y = fp8x2_to_bf16x2<true>(lo);
-  r.z = fp8x2_to_bf16x2<false>(hi);
-  r.w = fp8x2_to_bf16x2<true>(hi);
-  return r;
-}
-// Token fragments of one k-step (the wave's 8 blocks 2 b + wn) from the B stage at bstage.
-__device__ __forceinline__ void read_bfrags(uint32_t bstage, u32x4v (&b)[8]) {
-  b[0] = lds_read_frag<0 * kBlkBytes>(bstage);
-  b[1] = lds_read_frag<2 * kBlkBytes>(bstage);
-  b[2] = lds_read_frag<4 * kBlkBytes>(bstage);
-  b[3] = lds_read_frag<6 * kBlkBytes>(bstage);
-  b[4] = lds_read_frag<8 * kBlkBytes>(bstage);
-  b[5] = lds_read_frag<10 * kBlkBytes>(bstage);
-  b[6] = lds_read_frag<12 * kBlkBytes>(bstage);
-  b[7] = lds_read_frag<14 * kBlkBytes>(bstage);
-}
-// Weight fragments of one chunk (4 row blocks of 16 rows, 16 bytes per lane).
-__device__ __forceinline__ void read_afrags8(uint32_t astage, u32x4v (&a)[4]) {
-  a[0] = lds_read_frag<0 * 16 * F8RowBytes>(astage);
-  a[1] = lds_read_frag<1 * 16 * F8RowBytes>(astage);
-  a[2] = lds_read_frag<2 * 16 * F8RowBytes>(astage);
-  a[3] = lds_read_frag<3 * 16 * F8RowBytes>(astage);
-}
-template <int N>
-__device__ __forceinline__ void tie(u32x4v (&v)[N]) {
-#pragma unroll
-  for (int i = 0; i < N; ++i) after_wait(v[i]);
-}
-// k-step h of a chunk: weight halves h of a[], token fragments b[], first nb blocks.
-__device__ __forceinline__ void mma8(const u32x4v (&a)[4], int h, const u32x4v (&b)[8], int nb,
-                                     f32x4_t (&acc)[4][8]) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const u32x4v w = h ? widen8(a[i].z, a[i].w) : widen8(a[i].x, a[i].y);
-#pragma unroll
-    for (int bb = 0; bb < 8; ++bb) {
-      if (bb >= nb) break;
-      acc[i][bb] = mfma_frag(w, b[bb], acc[i][bb]);
-    }
-  }
-}
-
-template <int MODE>
-__global__ __launch_bounds__(kThreads, 1) void k_prefill_gemm_f8(GemmArgs args) {
-  extern __shared__ uint4 smem[];  // A ring [F8StagesA][16 KiB], B ring [kStagesB][32 KiB]
-
-  // tile / row-block order, table lookup and bounds: as k_prefill_gemm
-  const int nrb = args.nrb;
-  const int xcd = blockIdx.x & (kXcds - 1);
-  const int j = blockIdx.x / kXcds;
-  int tile = (j / nrb) * kXcds + xcd;
-  const int rb = j - (j / nrb) * nrb;
-  if (tile >= args.MTgrid) return;
-  int e, r0, r1;
-  if (args.table) {
-    const int ntiles = args.table[3 * args.MT];
-    if (tile >= ntiles) return;
-    if (args.shared_first > 0) {
-      const int ns = min(args.shared_first, ntiles);
-      tile = tile < ns ? ntiles - ns + tile : tile - ns;
-    }
-    e = args.table[tile];
-    r0 = args.table[args.MT + tile];
-    r1 = min(args.table[2 * args.MT + tile], r0 + PBM);
-  } else {
-    e = args.E;
-    r0 = args.P + tile * PBM;
-    if (r0 >= args.P + args.T) return;
-    r1 = min(r0 + PBM, args.P + args.T);
-  }
-  const bool routed = e < args.E;
-  const GemmOperand& op = routed ? args.op[0] : args.op[1];
-  constexpr int kOutPerWG = MODE == kModeSwiglu ? PBN / 2 : PBN;
-  if (rb * kOutPerWG >= op.N) return;
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave & 3;   // weight-row group (64 rows)
-  const int wn = wave >> 2;  // token-block parity
-  const int lr = lane & 15;
-  const int kq = lane >> 4;
-  const int ntok = r1 - r0;
-
-  // ---- DMA sources: weights (load i of the wave: 16-row group wave + 8 i), token rows (as
-  // k_prefill_gemm: 8-row group wave + 8 i, 128 bytes of each row)
-  const uint8_t* __restrict__ srca[F8ALoads];
-  const uint16_t* __restrict__ srcb[kLoadsPerWave];
-  {
-    const uint8_t* __restrict__ wbase =
-        reinterpret_cast<const uint8_t*>(op.w) + (long long)(routed ? e : 0) * op.estride;
-    const int arow = lane >> 2;
-#pragma unroll
-    for (int i = 0; i < F8ALoads; ++i) {
-      const int row = (wave + 8 * i) * 16 + arow;  // 0..255
-      const int unit = (lane & 3) ^ ((row >> 1) & 3);
-      long long wrow;
-      if (MODE == kModeSwiglu) {
-        const int g = rb * (PBN / 2) + (row >> 6) * 32 + (row & 31);
-        wrow = (long long)g * op.ldw + (((row >> 5) & 1) ? op.up_off : 0);
-      } else {
-        wrow = (long long)min(rb * PBN + row, op.N - 1) * op.ldw;
-      }
-      srca[i] = wbase + wrow + unit * 16;
-    }
-    // token rows: physical unit q = (l & 7) ^ row holds logical unit 2 (q & 3) + (q >> 2), so
-    // that the units 2 kq + h that k-step h reads sit where the bf16 kernel's k-step reads
-    // them (physical (4 h + kq) ^ row): that pattern is conflict-free, 2 kq + h at the
-    // physical unit was not (3.2 bank-conflict cycles per LDS instruction)
-    const int grow = lane >> 3;
-    const int bq = (lane & 7) ^ grow;
-    const int bunit = 2 * (bq & 3) + (bq >> 2);
-#pragma unroll
-    for (int i = 0; i < kLoadsPerWave; ++i) {
-      const int row = (wave + 8 * i) * 8 + grow;
-      const int r = min(r0 + row, r1 - 1);
-      long long src;
-      if (!routed)
-        src = r - args.P;
-      else if (op.in_map)
-        src = args.order[r] / args.topk;
-      else
-        src = r;
-      srcb[i] = op.in + src * op.ld_in + bunit * 8;
-    }
-  }
-  char* lds = reinterpret_cast<char*>(smem);
-  char* bring_lds = lds + F8StagesA * F8Stage;
-  auto issue_a = [&](int d) {
-    char* st = lds + (d % F8StagesA) * F8Stage;
-#pragma unroll
-    for (int i = 0; i < F8ALoads; ++i)
-      __builtin_amdgcn_global_load_lds(srca[i] + d * F8RowBytes, st + (wave + 8 * i) * 1024, 16,
-                                       0, 0);
-  };
-  const int nb_loads = __builtin_amdgcn_readfirstlane(
-      min(kLoadsPerWave, max(0, ((r1 - r0 + 7) / 8 - wave + 7) / 8)));
-  auto issue_b = [&](int d) {
-    char* st = bring_lds + (d % kStagesB) * kOpStage;
-#pragma unroll
-    for (int i = 0; i < kLoadsPerWave; ++i)
-      if (i < nb_loads)
-        __builtin_amdgcn_global_load_lds(srcb[i] + d * DKC, st + (wave + 8 * i) * 1024, 16, 0, 0);
-  };
-  typedef __attribute__((address_space(3))) char lds_char;
-  const uint32_t lds_base = (uint32_t)(uintptr_t)(lds_char*)lds;
-  // weight fragment: row lr of a 16-row block, logical unit kq; token fragment of k-step h:
-  // row lr, logical unit 2 kq + h (stored at physical (4 h + kq) ^ row)
-  const uint32_t ra = (uint32_t)(wm * 64 * F8RowBytes + lr * F8RowBytes +
-                                 ((kq ^ ((lr >> 1) & 3)) * 16));
-  const uint32_t rbo0 = (uint32_t)(wn * kBlkBytes + lr * kRowBytes + ((kq ^ (lr & 7)) * 16));
-  const uint32_t rbo1 = (uint32_t)(wn * kBlkBytes + lr * kRowBytes + (((4 + kq) ^ (lr & 7)) * 16));
-
-  f32x4_t acc[4][8];
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int b = 0; b < 8; ++b) acc[a][b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-  const int nblk = (ntok + 15) >> 4;
-  const int nb = __builtin_amdgcn_readfirstlane(min(8, (nblk - wn + 1) >> 1));
-
-  // Pipeline: chunk d's weight fragments are read at its k-step 0 and kept for k-step 1;
-  // the token fragments of each k-step are read while the previous one is multiplied. Load
-  // order: A(0 .. S - 3), B(0), A(S - 2), B(1), A(S - 1), then at chunk d + 1's first k-step
-  // B(d + 2), A(d + S), so that the loads younger than B(d) are exactly A(d + S - 2).
-  const int nd = op.K / DKC;
-  const int nk = 2 * nd;
-  for (int d = 0; d < F8AheadA - 1; ++d)
-    if (d < nd) issue_a(d);
-  if (nd > 0) issue_b(0);
-  if (F8AheadA - 1 < nd) issue_a(F8AheadA - 1);
-  if (nd > 1) issue_b(1);
-  if (F8AheadA < nd) issue_a(F8AheadA);
-  // younger than B(0): A(S - 2), B(1), A(S - 1)
-  wait_loads(F8ALoads * (F8AheadA - 1 < nd) + nb_loads * (nd > 1) + F8ALoads * (F8AheadA < nd));
-  __builtin_amdgcn_s_barrier();
-  u32x4v acur[4], anxt[4], b0[8], b1[8];
-  read_afrags8(lds_base + ra, acur);
-  read_bfrags(lds_base + F8StagesA * F8Stage + rbo0, b0);
-  lds_frags_ready();
-  tie(acur);
-  tie(b0);
-  for (int d = 0; d < nd; ++d) {
-    const uint32_t bst = lds_base + F8StagesA * F8Stage + (d % kStagesB) * kOpStage;
-    // k-step 0 of chunk d (weights acur, tokens b0) while k-step 1's tokens are read
-    read_bfrags(bst + rbo1, b1);
-    mma8(acur, 0, b0, nb, acc);
-    lds_frags_ready();
-    tie(b1);
-    // k-step 1 while chunk d + 1's weights and k-step-0 tokens are read
-    const bool more = d + 1 < nd;
-    if (more) {
-      wait_loads(F8ALoads * (d + F8AheadA < nd));
-      __builtin_amdgcn_s_barrier();
-      if (d + 2 < nd) issue_b(d + 2);
-      if (d + 1 + F8AheadA < nd) issue_a(d + 1 + F8AheadA);
-      read_afrags8(lds_base + ((d + 1) % F8StagesA) * F8Stage + ra, anxt);
-      read_bfrags(lds_base + F8StagesA * F8Stage + ((d + 1) % kStagesB) * kOpStage + rbo0, b0);
-    }
-    mma8(acur, 1, b1, nb, acc);
-    if (more) {
-      lds_frags_ready();
-      tie(anxt);
-      tie(b0);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acur[i] = anxt[i];
-    }
-  }
-
-  // ---- epilogue (k_prefill_gemm's), the row scales requested together first
-  const float* sc = op.scale ? op.scale + (long long)(routed ? e : 0) * op.sstride : nullptr;
-  float scl[4][4];
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      int n;
-      if (MODE == kModeSwiglu)  // blocks 0-1 gate rows, 2-3 the matching up rows
-        n = rb * (PBN / 2) + wm * 32 + (a & 1) * 16 + 4 * kq + i + ((a >> 1) ? (int)op.s_up_off : 0);
-      else
-        n = min(rb * PBN + wm * 64 + a * 16 + 4 * kq + i, op.N - 1);
-      scl[a][i] = sc ? sc[n] : 1.f;
-    }
-#pragma unroll
-  for (int b = 0; b < 8; ++b) {
-    if (b >= nb) break;
-    const int rr = r0 + (2 * b + wn) * 16 + lr;
-    if (rr >= r1) continue;
-    const long long orow = routed ? (op.out_map ? args.order[rr] : rr) : rr - args.P;
-    if (MODE == kModeSwiglu) {
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int n = rb * (PBN / 2) + wm * 32 + h * 16 + 4 * kq;
-        float o[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float g = rbf(acc[h][b][i] * scl[h][i]);
-          float u = rbf(acc[2 + h][b][i] * scl[2 + h][i]);
-          o[i] = rbf(siluf_(g)) * u;
-        }
-        *reinterpret_cast<uint2*>(op.out + orow * op.ld_out + n) =
-            make_uint2(pack_bf2(o[0], o[1]), pack_bf2(o[2], o[3]));
-      }
-    } else {
-#pragma unroll
-      for (int a = 0; a < 4; ++a) {
-        const int n = rb * PBN + wm * 64 + a * 16 + 4 * kq;
-        if (n >= op.N) break;
-        float o[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o[i] = acc[a][b][i] * scl[a][i];
-        *reinterpret_cast<uint2*>(op.out + orow * op.ld_out + n) =
-            make_uint2(pack_bf2(o[0], o[1]), pack_bf2(o[2], o[3]));
-      }
-    }
-  }
-}
-
 int prefill_tile_rows() { return PBM; }
+
+// Sorted rows per tile of the block's own tables: what the launches of its projections take at
+// best. e4m3 experts: 64 rows where the experts' average share is at most 44 rows, else 160.
+// bf16 ones alike up to 96 rows on average, where gate_up runs on the streaming kernel; above
+// that this file's 256-row tiles do both projections.
+int prefill_block_rows(long long pairs, int experts, bool fp8) {
+  if (!fp8 && pairs > 96LL * experts) return PBM;
+  return pairs <= 44LL * experts ? kStreamRowsSmall : kStreamRowsLarge;
+}
 
 bool prefill_fits(int mode, const GemmOperand& op) {
   if (op.N <= 0) return true;
@@ -602,10 +326,10 @@ bool prefill_fits(int mode, const GemmOperand& op) {
 }
 
 namespace {
-// The kernels' dynamic LDS above the default limit, allowed once per device and mode.
+// The kernel's dynamic LDS above the default limit, allowed once per device and mode.
 hipError_t allow_lds(const void* fn, int mode, int bytes) {
   static std::mutex mu;
-  static uint64_t done[4] = {0, 0, 0, 0};  // [kernel], bit d: device d
+  static uint64_t done[2] = {0, 0};  // [mode], bit d: device d
   int dev = 0;
   hipError_t err = hipGetDevice(&dev);
   if (err != hipSuccess) return err;
@@ -618,8 +342,10 @@ hipError_t allow_lds(const void* fn, int mode, int bytes) {
 }
 }  // namespace
 
-hipError_t launch_prefill_gemm(int mode, const GemmArgs& a_in, int max_tiles, hipStream_t st) {
+hipError_t launch_prefill_gemm(int mode, const GemmArgs& a_in, int max_tiles, int bm,
+                               hipStream_t st) {
   GemmArgs a = a_in;
+  if (bm > PBM) return hipErrorInvalidValue;
   if (!prefill_fits(mode, a.op[0]) || !prefill_fits(mode, a.op[1])) return hipErrorInvalidValue;
   const bool has0 = a.op[0].N > 0, has1 = a.op[1].N > 0;
   if (has0 && has1 && a.op[0].fp8 != a.op[1].fp8) {
@@ -628,42 +354,40 @@ hipError_t launch_prefill_gemm(int mode, const GemmArgs& a_in, int max_tiles, hi
     GemmArgs r = a, v = a;
     r.op[1].N = 0;
     v.op[0].N = 0;
-    hipError_t err = launch_prefill_gemm(mode, r, max_tiles, st);
-    return err != hipSuccess ? err : launch_prefill_gemm(mode, v, max_tiles, st);
+    hipError_t err = launch_prefill_gemm(mode, r, max_tiles, bm, st);
+    return err != hipSuccess ? err : launch_prefill_gemm(mode, v, max_tiles, bm, st);
   }
   const bool f8 = (has0 && a.op[0].fp8) || (has1 && a.op[1].fp8);
+  if (max_tiles <= 0 || (!has0 && !has1)) return hipSuccess;
+  a.bm = bm;
+  a.shared_first = 0;
+  if (a.table && has0 && has1) {
+    const char* env = knob(kKnobPrefillSharedFirst);
+    if (!(env && env[0] == '0')) a.shared_first = (a.T + bm - 1) / bm;
+  }
+  // The streaming kernel's: e4m3 weights, and the routed bf16 gate_up on its own tile sizes
+  // (µs against this file's kernel, H = 2048, I = 512, E = 256, top-8: gate_up at
+  // T = 777 / 1111 / 2048 199 / 211 / 225 against 252 / 251 / 259, at 4096 290 against 280;
+  // down 125 / 131 / 142 / 180 against 113 / 118 / 134 / 167, so bf16 down stays here).
+  if (f8 || (mode == kModeSwiglu && has0 && !has1 && stream_takes(a, bm)))
+    return launch_prefill_stream(mode, a, max_tiles, st);
   const int out_per_wg = mode == kModeSwiglu ? PBN / 2 : PBN;
   const int nmax = a.op[0].N > a.op[1].N ? a.op[0].N : a.op[1].N;
   a.nrb = (nmax + out_per_wg - 1) / out_per_wg;
-  if (a.nrb <= 0 || max_tiles <= 0) return hipSuccess;
-  const size_t lds = (size_t)kLdsBytes;
+  if (!a.table) max_tiles = (a.T + PBM - 1) / PBM;  // the shared rows in whole tiles
   a.MTgrid = max_tiles;
-  a.shared_first = 0;
-  if (a.table && a.op[0].N > 0 && a.op[1].N > 0) {
-    const char* env = knob(kKnobPrefillSharedFirst);
-    if (!(env && env[0] == '0')) a.shared_first = (a.T + PBM - 1) / PBM;
-  }
   const long long grid = (long long)((max_tiles + kXcds - 1) / kXcds) * kXcds * a.nrb;
   if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
-  const size_t lds_k = f8 ? (size_t)F8LdsBytes : lds;
-  const void* fn = mode == kModeSwiglu
-                       ? (f8 ? reinterpret_cast<const void*>(&k_prefill_gemm_f8<kModeSwiglu>)
-                             : reinterpret_cast<const void*>(&k_prefill_gemm<kModeSwiglu>))
-                       : (f8 ? reinterpret_cast<const void*>(&k_prefill_gemm_f8<kModePlain>)
-                             : reinterpret_cast<const void*>(&k_prefill_gemm<kModePlain>));
-  hipError_t err = allow_lds(fn, mode + (f8 ? 2 : 0), (int)lds_k);
+  const void* fn = mode == kModeSwiglu ? reinterpret_cast<const void*>(&k_prefill_gemm<kModeSwiglu>)
+                                       : reinterpret_cast<const void*>(&k_prefill_gemm<kModePlain>);
+  hipError_t err = allow_lds(fn, mode, kLdsBytes);
   if (err != hipSuccess) return err;
-  if (f8) {
-    if (mode == kModeSwiglu)
-      hipLaunchKernelGGL(k_prefill_gemm_f8<kModeSwiglu>, dim3((unsigned)grid), dim3(kThreads), lds_k, st, a);
-    else
-      hipLaunchKernelGGL(k_prefill_gemm_f8<kModePlain>, dim3((unsigned)grid), dim3(kThreads), lds_k, st, a);
-    return hipGetLastError();
-  }
   if (mode == kModeSwiglu)
-    hipLaunchKernelGGL(k_prefill_gemm<kModeSwiglu>, dim3((unsigned)grid), dim3(kThreads), lds, st, a);
+    hipLaunchKernelGGL(k_prefill_gemm<kModeSwiglu>, dim3((unsigned)grid), dim3(kThreads),
+                       (size_t)kLdsBytes, st, a);
   else
-    hipLaunchKernelGGL(k_prefill_gemm<kModePlain>, dim3((unsigned)grid), dim3(kThreads), lds, st, a);
+    hipLaunchKernelGGL(k_prefill_gemm<kModePlain>, dim3((unsigned)grid), dim3(kThreads),
+                       (size_t)kLdsBytes, st, a);
   return hipGetLastError();
 }
 

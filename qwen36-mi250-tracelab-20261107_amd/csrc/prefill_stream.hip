@@ -1,0 +1,652 @@
+// Grouped MFMA GEMM for prefill-sized batches on gfx950 (subsystems a8, a9, a6).
+//
+// Same contract as k_expert_gemm (expert_gemm.hip) and the reference's grouped kernels
+// (engine/fast/moe_prefill.py:156-257): for the sorted rows of ONE expert in a tile,
+//   SWIGLU: act[r, n]       = bf16(bf16(silu(bf16 g)) * bf16 u)
+//   PLAIN:  out[orow(r), n] = bf16(act_or_x[r] . W[e, n])
+// with bf16 or e4m3 weights (per-output-row fp32 scales on the fp32 accumulator).
+//
+// Split. A workgroup of 4 waves takes 128 weight rows and up to 16 * MAXB token rows of a
+// tile; wave w owns 32 weight rows (two 16-row MFMA blocks; SWIGLU: 16 gate rows and the
+// matching 16 up rows, paired in registers by the epilogue) against every token row.
+// * A weight row is used by one wave only, so weights go from HBM straight into that wave's
+//   registers in the MFMA A layout (lane: row l % 16, 16 bytes at 16 (l / 16); 64 contiguous
+//   bytes of each of 16 rows per load), a ring of R chunks of 64 k. The launch is bound by
+//   this stream, and registers hold more of it in flight than LDS could.
+// * Token rows are used by all four waves: global -> LDS DMA (no registers on the way) into R
+//   stages of 64 k (128 bytes of each row), requested R - 1 chunks ahead.
+// vmcnt retires in order, so a chunk's token rows are requested beside the weights of about
+// the same chunk: waiting for them never drains younger weight loads.
+//
+// LDS layout of a stage: row r's 128 bytes at 128 r; 16-byte unit q holds logical unit
+// q ^ (r & 7), so the fragment reads (16 rows, one unit) are bank-conflict free. With e4m3
+// weights a lane's 16 weight bytes are k = 16 kq .. + 15, fed as two k-steps of 8 bytes, so
+// the token units are permuted alike: k-step h's lane group kq reads logical unit 2 kq + h,
+// stored where the bf16 form's k-step h reads.
+//
+// The body is compiled per number of 16-token blocks (NB), so that a part-filled tile loads,
+// reads and multiplies only the blocks it has and every wait count is a constant.
+#include <stdint.h>
+#include <stdlib.h>
+
+#include <mutex>
+
+#include "moe_common.h"
+#include "expert_gemm.h"
+#include "lds_dma.h"
+
+namespace moe {
+
+namespace {
+constexpr int kPKC = 64;            // k per chunk
+constexpr int kPRowBytes = kPKC * 2;             // bytes of a staged token row
+constexpr int kPBlkBytes = 16 * kPRowBytes;      // a 16-token block of a stage: 2 KiB
+// Cache policy of the results' stores. gate_up's go through the L2 at once (sc1): the launch
+// ends with little left to write back (T = 1111: 226 -> 215 us). down's rows are completed in
+// the L2 by two waves each and stay there until then (156 against 170 us at T = 4096 with sc1,
+// 232 non-temporal).
+template <int MODE>
+constexpr int kStorePolicy = MODE == kModeSwiglu ? 16 : 0;
+constexpr int kXcds = 8;            // XCDs of an MI355X (round-robin dispatch)
+constexpr int kPBlocksLarge = kStreamRowsLarge / 16;  // MAXB
+constexpr int kPBlocksSmall = kStreamRowsSmall / 16;
+}  // namespace
+
+// The NB token fragments (16 rows each, 2 KiB apart) at LDS byte address addr, waited for.
+// One asm block, so no fragment register is visible before its data has arrived.
+template <int NB>
+struct TokenFrags;
+template <>
+struct TokenFrags<2> {
+  static __device__ __forceinline__ void read(uint32_t addr, u32x4v (&f)[2]) {
+    asm volatile(
+               "ds_read_b128 %0, %2 offset:0\n\t"
+               "ds_read_b128 %1, %2 offset:2048\n\t"
+               "s_waitcnt lgkmcnt(0)"
+               : "=&v"(f[0]), "=&v"(f[1])
+               : "v"(addr));
+  }
+};
+template <>
+struct TokenFrags<4> {
+  static __device__ __forceinline__ void read(uint32_t addr, u32x4v (&f)[4]) {
+    asm volatile(
+               "ds_read_b128 %0, %4 offset:0\n\t"
+               "ds_read_b128 %1, %4 offset:2048\n\t"
+               "ds_read_b128 %2, %4 offset:4096\n\t"
+               "ds_read_b128 %3, %4 offset:6144\n\t"
+               "s_waitcnt lgkmcnt(0)"
+               : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]), "=&v"(f[3])
+               : "v"(addr));
+  }
+};
+template <>
+struct TokenFrags<6> {
+  static __device__ __forceinline__ void read(uint32_t addr, u32x4v (&f)[6]) {
+    asm volatile(
+               "ds_read_b128 %0, %6 offset:0\n\t"
+               "ds_read_b128 %1, %6 offset:2048\n\t"
+               "ds_read_b128 %2, %6 offset:4096\n\t"
+               "ds_read_b128 %3, %6 offset:6144\n\t"
+               "ds_read_b128 %4, %6 offset:8192\n\t"
+               "ds_read_b128 %5, %6 offset:10240\n\t"
+               "s_waitcnt lgkmcnt(0)"
+               : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]), "=&v"(f[3]), "=&v"(f[4]), "=&v"(f[5])
+               : "v"(addr));
+  }
+};
+template <>
+struct TokenFrags<8> {
+  static __device__ __forceinline__ void read(uint32_t addr, u32x4v (&f)[8]) {
+    asm volatile(
+               "ds_read_b128 %0, %8 offset:0\n\t"
+               "ds_read_b128 %1, %8 offset:2048\n\t"
+               "ds_read_b128 %2, %8 offset:4096\n\t"
+               "ds_read_b128 %3, %8 offset:6144\n\t"
+               "ds_read_b128 %4, %8 offset:8192\n\t"
+               "ds_read_b128 %5, %8 offset:10240\n\t"
+               "ds_read_b128 %6, %8 offset:12288\n\t"
+               "ds_read_b128 %7, %8 offset:14336\n\t"
+               "s_waitcnt lgkmcnt(0)"
+               : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]), "=&v"(f[3]), "=&v"(f[4]), "=&v"(f[5]), "=&v"(f[6]), "=&v"(f[7])
+               : "v"(addr));
+  }
+};
+template <>
+struct TokenFrags<10> {
+  static __device__ __forceinline__ void read(uint32_t addr, u32x4v (&f)[10]) {
+    asm volatile(
+               "ds_read_b128 %0, %10 offset:0\n\t"
+               "ds_read_b128 %1, %10 offset:2048\n\t"
+               "ds_read_b128 %2, %10 offset:4096\n\t"
+               "ds_read_b128 %3, %10 offset:6144\n\t"
+               "ds_read_b128 %4, %10 offset:8192\n\t"
+               "ds_read_b128 %5, %10 offset:10240\n\t"
+               "ds_read_b128 %6, %10 offset:12288\n\t"
+               "ds_read_b128 %7, %10 offset:14336\n\t"
+               "ds_read_b128 %8, %10 offset:16384\n\t"
+               "ds_read_b128 %9, %10 offset:18432\n\t"
+               "s_waitcnt lgkmcnt(0)"
+               : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]), "=&v"(f[3]), "=&v"(f[4]), "=&v"(f[5]), "=&v"(f[6]), "=&v"(f[7]), "=&v"(f[8]), "=&v"(f[9])
+               : "v"(addr));
+  }
+};
+
+// Wait until at most N of this wave's loads are in flight, then the workgroup's barrier.
+template <int N>
+__device__ __forceinline__ void wait_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+// Keeps the loads before it ahead of those after it: the waits count them in issue order.
+__device__ __forceinline__ void issue_fence() { asm volatile("" ::: "memory"); }
+
+// 8 e4m3 bytes -> bf16x8 (exact)
+__device__ __forceinline__ u32x4v widen8(uint32_t lo, uint32_t hi) {
+  u32x4v r;
+  r.x = fp8x2_to_bf16x2<false>(lo);
+  r.y = fp8x2_to_bf16x2<true>(lo);
+  r.z = fp8x2_to_bf16x2<false>(hi);
+  r.w = fp8x2_to_bf16x2<true>(hi);
+  return r;
+}
+
+__device__ __forceinline__ u32x4v ld_weight(const char* p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const u32x4v*>(p));
+}
+
+// Stores a block's results: lane (kq, lr) holds rows 4 kq .. + 3 of token column lr of each
+// 16-token block.
+// WIDE: two token blocks at a time, exchanged between lane rows so that a lane holds 8
+// consecutive results of one token (16-byte stores, half as many), always all of them: those
+// of rows past the tile or the weights go past the buffer's end, where they are dropped. The
+// weights of the next block are in flight meanwhile, and their waits count the stores.
+template <int MODE, bool FP8, int NB, int W, bool WIDE, class OutRow>
+__device__ __forceinline__ void prefill_epilogue(const GemmArgs& args, const GemmOperand& op,
+                                                 bool routed, int e, int r0, int r1, int rb,
+                                                 int wave, int lr, int kq,
+                                                 OutRow out_row,
+                                                 const f32x4_t (&acc)[2][NB]) {
+  constexpr int kRows = 32 * W;
+  constexpr int kA = MODE == kModeSwiglu ? 1 : 2;  // 16-row groups of results
+  const float* sc = FP8 && op.scale ? op.scale + (long long)(routed ? e : 0) * op.sstride : nullptr;
+  const int nw = MODE == kModeSwiglu ? rb * (kRows / 2) + wave * 16 : rb * kRows + wave * 32;
+  const int n0 = nw + 4 * kq;
+  float scl[2][4] = {{1.f, 1.f, 1.f, 1.f}, {1.f, 1.f, 1.f, 1.f}};
+  if (sc) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        scl[a][i] = sc[MODE == kModeSwiglu ? n0 + i + (a ? (int)op.s_up_off : 0)
+                                           : min(n0 + a * 16 + i, op.N - 1)];
+  }
+  // the lane's 4 results of group a and block b, as two pairs
+  auto results = [&](int a, int b, uint32_t (&o)[2]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 4; i += 2) {
+      if (MODE == kModeSwiglu) {
+        const uint32_t g = pack_bf2_rne(acc[0][b][i] * scl[0][i], acc[0][b][i + 1] * scl[0][i + 1]);
+        const uint32_t u = pack_bf2_rne(acc[1][b][i] * scl[1][i], acc[1][b][i + 1] * scl[1][i + 1]);
+        const uint32_t s = pack_bf2_rne(silu_fast(bf_lo(g)), silu_fast(bf_hi(g)));
+        o[i / 2] = pack_bf2_rne(bf_lo(s) * bf_lo(u), bf_hi(s) * bf_hi(u));
+      } else {
+        o[i / 2] = pack_bf2_rne(acc[a][b][i] * scl[a][i], acc[a][b][i + 1] * scl[a][i + 1]);
+      }
+    }
+  };
+  if constexpr (WIDE) {
+    const __amdgpu_buffer_rsrc_t obuf = __builtin_amdgcn_make_buffer_rsrc(
+        op.out, 0, args.out_bytes[routed ? 0 : 1], 0x00020000);
+    const uint32_t ld = (uint32_t)(op.ld_out * 2);
+#pragma unroll
+    for (int b = 0; b < NB; b += 2) {
+      __builtin_amdgcn_sched_barrier(0);  // one pair's results live at a time
+      const int blk = b + (kq & 1);
+      const int row = out_row(blk, b);
+      const bool live = r0 + blk * 16 + lr < r1;
+#pragma unroll
+      for (int a = 0; a < kA; ++a) {
+        uint32_t p[2], q[2];
+        results(a, b, p);
+        results(a, b + 1, q);
+        u32x4v v;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const auto x = __builtin_amdgcn_permlane16_swap(p[i], q[i], false, false);
+          v[i] = x[0];
+          v[i + 2] = x[1];
+        }
+        const int n = nw + a * 16 + (kq >> 1) * 8;
+        const uint32_t off = (uint32_t)row * ld + (uint32_t)n * 2;
+        __builtin_amdgcn_raw_buffer_store_b128(v, obuf, live && n < op.N ? off : 0xfffffff0u, 0,
+                                               kStorePolicy<MODE>);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      __builtin_amdgcn_sched_barrier(0);
+      const int row = out_row(b, b);
+      if (r0 + b * 16 + lr >= r1) continue;
+      uint16_t* out = op.out + (long long)row * op.ld_out + n0;
+#pragma unroll
+      for (int a = 0; a < kA; ++a) {
+        if (n0 + a * 16 >= op.N) break;  // N is a multiple of 16: n < N covers n + 3
+        uint32_t o[2];
+        results(a, b, o);
+        *reinterpret_cast<uint2*>(out + a * 16) = make_uint2(o[0], o[1]);
+      }
+    }
+  }
+}
+
+// One workgroup's product: weight rows of blocks rb .. rb + nblk - 1 (expert e) against sorted
+// rows [r0, r1), r1 - r0 <= 16 NB. R: chunks per phase and ring depth; K / 64 is a multiple of
+// R (R = 1: any K, multiple of 32).
+template <int MODE, bool FP8, int NB, int W, int R, bool RES>
+__device__ __forceinline__ void prefill_body(const GemmArgs& args, const GemmOperand& op,
+                                             bool routed, int e, int r0, int r1, int rb0, int nblk,
+                                             char* lds) {
+  constexpr int kCB = FP8 ? kPKC : 2 * kPKC;  // weight bytes of a row per chunk
+  constexpr int kLS = FP8 ? 1 : 2;            // weight loads per row block and chunk
+  constexpr int kLA = 2 * kLS;                // weight loads per chunk
+  constexpr int kLB = 2 * NB * R / W;         // token DMA loads of a wave per phase
+  constexpr int kSub = NB * kPBlkBytes;       // a chunk of the token rows in LDS
+  constexpr int kStage = R * kSub;            // a phase
+  constexpr int kRows = 32 * W;               // weight rows per block
+  static_assert(kLB * W == 2 * NB * R && W % R == 0, "whole DMA groups per wave");
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 15;
+  const int kq = lane >> 4;
+
+  // ---- token rows of this wave's DMA loads: chunk wave % R of the phase, 8-row groups
+  // wave / R + (W / R) i. The order lookups go first, the weights (which need no lookup)
+  // right behind them.
+  const int sub = wave % R;
+  const int grow = lane >> 3;
+  const int pq = (lane & 7) ^ grow;
+  const int unit = FP8 ? 2 * (pq & 3) + (pq >> 2) : pq;
+  int trow[kLB];
+#pragma unroll
+  for (int i = 0; i < kLB; ++i)
+    trow[i] = min(r0 + (wave / R + (W / R) * i) * 8 + grow, r1 - 1);
+  // gate_up rows are pairs in sorted order, whose tokens order gives; down rows are sorted rows
+  const bool lookup = MODE == kModeSwiglu && routed;
+  if (lookup) {
+#pragma unroll
+    for (int i = 0; i < kLB; ++i) trow[i] = args.order[trow[i]];
+  }
+  const int row_base = routed ? 0 : args.P;
+  const int row_div = lookup ? args.topk : 1;
+
+  // The output rows. Down's pairs are looked up once: lane 16 m + l holds row l of 16-row
+  // block 4 i + m.
+  int orow[(NB + 3) / 4];
+  if (MODE == kModePlain && routed) {
+#pragma unroll
+    for (int i = 0; i < (NB + 3) / 4; ++i) orow[i] = args.order[min(r0 + i * 64 + lane, r1 - 1)];
+  }
+  // of row lr of block b, one of the constant group of four blocks that holds b0
+  auto out_row = [&](int b, int b0) __attribute__((always_inline)) {
+    const int row = r0 + b * 16 + lr;
+    if (MODE == kModeSwiglu) return row - row_base;
+    const int looked = __shfl(orow[b0 / 4], (b & 3) * 16 + lr);
+    return routed ? looked : row - row_base;
+  };
+
+  // ---- this lane's two weight rows of a block: wave-uniform bases, 32-bit lane offsets (the
+  // launcher checks that an expert's rows span less than 2 GiB)
+  constexpr int kEB = FP8 ? 1 : 2;
+  const char* const wbase =
+      reinterpret_cast<const char*>(op.w) + (long long)(routed ? e : 0) * op.estride * kEB;
+  const char* const wbase1 = wbase + (MODE == kModeSwiglu ? op.up_off * kEB : 0);
+  uint32_t woff[2];
+  auto weight_rows = [&](int rb) __attribute__((always_inline)) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      int row;
+      if (MODE == kModeSwiglu)
+        row = rb * (kRows / 2) + wave * 16 + lr;
+      else  // the last block may be partial
+        row = min(rb * kRows + wave * 32 + a * 16 + lr, op.N - 1);
+      woff[a] = rb < 0 ? 0u : (uint32_t)row * (uint32_t)(op.ldw * kEB) + (uint32_t)(kq * 16);
+    }
+  };
+  const int nch = op.K / kPKC;
+  u32x4v ring[R][2][kLS];
+  auto issue_a = [&](int slot, int c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int s = 0; s < kLS; ++s)
+        ring[slot][a][s] = ld_weight((a ? wbase1 : wbase) + c * kCB + s * 64 + woff[a]);
+    issue_fence();
+  };
+  // The DMA is the buffer form: its counter is one the compiler can count loads in order with
+  // (after a global -> LDS load it waits for every load in flight before it uses any of the
+  // weight registers). 32-bit offsets: the launcher checks the input's size.
+  uint32_t toff[kLB];
+  auto issue_b = [&](int stage, int phase, bool any) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t tbuf = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(op.in), 0, any ? args.in_bytes[routed ? 0 : 1] : 0, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < kLB; ++i)
+      dma16_buffer(tbuf,
+                   lds + stage * kStage + sub * kSub + (wave / R + (W / R) * i) * 1024, toff[i],
+                   (phase * R + sub) * kPRowBytes);
+    issue_fence();
+  };
+
+  f32x4_t acc[2][NB];
+  auto clear = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < NB; ++b) acc[a][b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  };
+  // fragment read offsets of k-steps 0 and 1: row lr of a block, logical unit 4 h + kq (bf16)
+  const uint32_t lbase = lds_addr(lds) + (uint32_t)(lr * kPRowBytes);
+  const uint32_t roff[2] = {lbase + (uint32_t)((kq ^ (lr & 7)) * 16),
+                            lbase + (uint32_t)(((4 + kq) ^ (lr & 7)) * 16)};
+  auto mma = [&](int slot, uint32_t at, int steps) __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if (h >= steps) break;
+      u32x4v f[NB];
+      TokenFrags<NB>::read(roff[h] + at, f);
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        u32x4v w;
+        if constexpr (FP8)
+          w = h ? widen8(ring[slot][a][0].z, ring[slot][a][0].w)
+                : widen8(ring[slot][a][0].x, ring[slot][a][0].y);
+        else
+          w = ring[slot][a][h];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) acc[a][b] = mfma_frag(w, f[b], acc[a][b]);
+      }
+      // the products stay ahead of the requests that refill their weight registers
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  auto epilogue = [&](int rb) __attribute__((always_inline)) {
+    prefill_epilogue<MODE, FP8, NB, W, (R > 1)>(args, op, routed, e, r0, r1, rb, wave, lr, kq,
+                                                out_row, acc);
+  };
+
+  weight_rows(rb0);
+  clear();
+  if constexpr (R > 1) {
+    const int nph = nch / R;
+    const int rot = routed ? prefill_start_chunk(e, nch) / R : 0;  // whole phases: R divides 4
+    auto phase_of = [&](int p) __attribute__((always_inline)) {  // p < nph
+      p += rot;
+      return p >= nph ? p - nph : p;
+    };
+    const int ph0 = phase_of(0);
+    issue_a(0, ph0 * R);
+#pragma unroll
+    for (int i = 0; i < kLB; ++i)
+      toff[i] = (uint32_t)((trow[i] - row_base) / row_div) * (uint32_t)(op.ld_in * 2) +
+                (uint32_t)(unit * 16);
+    issue_b(0, ph0, true);
+#pragma unroll
+    for (int c = 1; c < R; ++c) issue_a(c, ph0 * R + c);
+    if constexpr (RES) {
+      issue_b(1, phase_of(1), true);
+      wait_barrier<(R - 1) * kLA + kLB>();
+    } else {
+      wait_barrier<(R - 1) * kLA>();
+    }
+    // A phase multiplies the R chunks at LDS offset `at` and requests the next phase's
+    // operands, so that the counts are the same in every phase; the walk's last phase requests
+    // nothing from the buffer and one line of the weights. At its end the next phase's token
+    // rows have landed (younger: this phase's weight requests) and every wave is past this one.
+    auto phase = [&](int at, int stage, int next, bool more, bool sync) __attribute__((always_inline)) {
+      if constexpr (!RES) issue_b(stage, next, more);
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        mma(q, at + q * kSub, 2);
+        issue_a(q, next * R + q);
+      }
+      if (sync) wait_barrier<R * kLA>();
+    };
+    // Phase f of the walk: token stage f & 1 (RES: the two stages hold all of K, requested
+    // once). A block's first phase follows the stores of the block before it, whose number is
+    // a constant: hence the code of its own (the first block's is before the loop).
+    int f = 0;
+    phase(0, 1, phase_of(1), true, true);
+    for (int rb = rb0;;) {
+      for (int p = 1; p + 1 < nph; ++p) {
+        ++f;
+        phase((f & 1) * kStage, (f + 1) & 1, phase_of(p + 1), true, !RES);
+      }
+      const bool more = rb + 1 < rb0 + nblk;
+      weight_rows(more ? rb + 1 : -1);
+      ++f;
+      phase((RES ? 1 : f & 1) * kStage, (f + 1) & 1, ph0, more, !RES);
+      epilogue(rb);
+      if (!more) break;
+      ++rb;
+      clear();
+      ++f;
+      phase((RES ? 0 : f & 1) * kStage, (f + 1) & 1, phase_of(1), true, !RES);
+    }
+  } else {
+    // K of any multiple of 32: one chunk at a time; a last half chunk reads its first half
+    // twice instead of running past the rows
+    const char* tsrc[kLB];
+#pragma unroll
+    for (int i = 0; i < kLB; ++i) {
+      const long long src = (trow[i] - row_base) / row_div;
+      tsrc[i] = reinterpret_cast<const char*>(op.in + src * op.ld_in) + unit * 16;
+    }
+    const int all = (op.K + kPKC - 1) / kPKC;
+    const int rot = routed && op.K % kPKC == 0 ? prefill_start_chunk(e, all) : 0;
+    for (int j = 0; j < nblk; ++j) {
+      weight_rows(rb0 + j);
+      clear();
+      for (int c = 0; c < all; ++c) {
+        const int k0 = (c + rot < all ? c + rot : c + rot - all) * kPKC;
+        const bool half = op.K - k0 < kPKC;
+        wait_barrier<0>();  // every wave is past the previous chunk's stage
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+          for (int s = 0; s < kLS; ++s)
+            ring[0][a][s] =
+                ld_weight((a ? wbase1 : wbase) + k0 * kEB + (half ? 0 : s * 64) + woff[a]);
+#pragma unroll
+        for (int i = 0; i < kLB; ++i)
+          dma16(tsrc[i] + (long long)k0 * 2 - (half && unit >= 4 ? 64 : 0),
+                lds + (wave + W * i) * 1024);
+        wait_barrier<0>();
+        mma(0, 0, half ? 1 : 2);
+      }
+      epilogue(rb0 + j);
+    }
+  }
+}
+
+template <int MODE, bool FP8, int MAXB, int W, int R, bool RES>
+__global__ __launch_bounds__(64 * W)
+__attribute__((amdgpu_waves_per_eu(MAXB <= 4 ? 3 : 2))) void k_prefill_stream(GemmArgs args) {
+  extern __shared__ uint4 smem[];  // two phases (R = 1: one) of up to MAXB 16-token blocks
+
+  // XCD-aware order: workgroup b runs on XCD b % 8, so the workgroups of one tile get ids 8
+  // apart (same XCD, dispatched together) and share the tile's token rows in that XCD's L2
+  // instead of fetching them once per XCD.
+  const int ng = (args.nrb + args.nblk - 1) / args.nblk;  // workgroups per tile
+  const int xcd = blockIdx.x & (kXcds - 1);
+  const int j = blockIdx.x / kXcds;
+  int tile = (j / ng) * kXcds + xcd;
+  const int rb = (j - (j / ng) * ng) * args.nblk;
+  int e, r0, r1;
+  if (args.table) {
+    // nsub parts of 16 MAXB rows per table tile
+    const int sub = tile % args.nsub;
+    tile /= args.nsub;
+    const int ntiles = args.table[3 * args.MT];
+    if (tile >= ntiles) return;
+    if (args.shared_first > 0) {
+      // the shared expert's tiles (the table's last ones, all full: the longest workgroups)
+      // are dispatched first, the routed tiles fill in behind them
+      const int ns = min(args.shared_first, ntiles);
+      tile = tile < ns ? ntiles - ns + tile : tile - ns;
+    }
+    e = args.table[tile];
+    r0 = args.table[args.MT + tile];
+    // the table holds the expert's end row
+    r1 = min(args.table[2 * args.MT + tile], r0 + args.bm);
+    r0 += sub * 16 * MAXB;
+    r1 = min(r1, r0 + 16 * MAXB);
+  } else {
+    e = args.E;
+    r0 = args.P + tile * 16 * MAXB;
+    r1 = min(r0 + 16 * MAXB, args.P + args.T);
+  }
+  if (r0 >= r1) return;
+  const bool routed = e < args.E;
+  const GemmOperand& op = routed ? args.op[0] : args.op[1];
+  constexpr int kOut = MODE == kModeSwiglu ? 16 * W : 32 * W;  // output rows per block
+  const int nblk = min(args.nblk, (op.N + kOut - 1) / kOut - rb);
+  if (nblk <= 0) return;
+  char* lds = reinterpret_cast<char*>(smem);
+  const int nb = (r1 - r0 + 15) >> 4;
+#define NB_CASE(NB)                                                                    \
+  if (NB == MAXB || nb <= NB) {                                                        \
+    prefill_body<MODE, FP8, NB, W, R, RES>(args, op, routed, e, r0, r1, rb, nblk, lds);     \
+    return;                                                                            \
+  }
+  if constexpr (MAXB == 4) {
+    NB_CASE(2)
+    NB_CASE(4)
+  } else {
+    NB_CASE(4)
+    NB_CASE(6)
+    NB_CASE(8)
+    NB_CASE(10)
+  }
+#undef NB_CASE
+}
+
+namespace {
+
+// The kernel's dynamic LDS above the default limit, allowed once per device and kernel.
+hipError_t allow_lds(const void* fn, int which, int bytes) {
+  static std::mutex mu;
+  static uint64_t done[32] = {};  // [kernel], bit d: device d
+  int dev = 0;
+  hipError_t err = hipGetDevice(&dev);
+  if (err != hipSuccess) return err;
+  if (dev < 0 || dev >= 64) return hipErrorInvalidDevice;
+  std::lock_guard<std::mutex> lock(mu);
+  if (done[which] >> dev & 1) return hipSuccess;
+  err = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  if (err == hipSuccess) done[which] |= uint64_t(1) << dev;
+  return err;
+}
+
+template <int MODE, bool FP8, int MAXB, int W, int R, bool RES = false>
+hipError_t launch_one(GemmArgs a, int tiles, hipStream_t st) {
+  constexpr int bytes = (R > 1 ? 2 * R : 1) * MAXB * kPBlkBytes;
+  constexpr int kOut = MODE == kModeSwiglu ? 16 * W : 32 * W;
+  const int nmax = a.op[0].N > a.op[1].N ? a.op[0].N : a.op[1].N;
+  a.nrb = (nmax + kOut - 1) / kOut;
+  // Row blocks per workgroup: down's token rows are staged once for all of them and the next
+  // block's weights stream through the epilogue of one (T = 777 / 1111 / 2048 / 4096, e4m3: 75 /
+  // 81 / 93 / 146 µs with 4, 77 / 82 / 96 / 132 with 2, 81 / 87 / 102 / 139 with 1). gate_up
+  // gains nothing that the coarser work units do not cost (144 / 206 against 138 / 223 with 2).
+  a.nblk = MODE == kModePlain ? (MAXB == kPBlocksSmall ? 4 : 2) : 1;
+  const long long ng = (a.nrb + a.nblk - 1) / a.nblk;
+  const long long grid = (long long)((tiles + kXcds - 1) / kXcds) * kXcds * ng;
+  if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
+  const auto fn = &k_prefill_stream<MODE, FP8, MAXB, W, R, RES>;
+  const int which = (MODE * 2 + (FP8 ? 1 : 0)) * 8 + (MAXB == kPBlocksSmall ? 0 : 4) + (RES ? 3 : R / 2);
+  const hipError_t err = allow_lds(reinterpret_cast<const void*>(fn), which, bytes);
+  if (err != hipSuccess) return err;
+  hipLaunchKernelGGL((k_prefill_stream<MODE, FP8, MAXB, W, R, RES>), dim3((unsigned)grid), dim3(64 * W),
+                     bytes, st, a);
+  return hipGetLastError();
+}
+
+// The ring an operand's shape allows: phases of 4 or 2 chunks, at least two per block, 32-bit
+// offsets into its tensors; 1: the one-chunk form, which takes any shape.
+int ring_of(const GemmArgs& a, int i) {
+  const GemmOperand& o = a.op[i];
+  const long long in = (i == 0 && !o.in_map ? (long long)a.P : a.T) * o.ld_in * 2;
+  const long long out = (i == 0 ? (long long)a.P : a.T) * o.ld_out * 2;
+  if (in > 0xffffff00LL || out > 0xffffff00LL || (long long)o.N * o.ldw * 2 > 0x7fffffffLL) return 1;
+  if (o.K % (2 * kPKC) || o.K < 4 * kPKC) return 1;
+  return o.K % (4 * kPKC) || o.K < 8 * kPKC ? 2 : 4;
+}
+
+// gate_up's 64-row tiles take short phases: T = 777 / 1111 210 / 225 µs against 215 / 228 in
+// phases of 4 chunks (e4m3 131 / 145 against 140 / 157).
+hipError_t launch_gate_up(const GemmArgs& a, bool f8, bool small, int ring, int tiles,
+                          hipStream_t st) {
+  constexpr int S = kPBlocksSmall, L = kPBlocksLarge;
+  constexpr int M = kModeSwiglu;
+  if (ring == 1) {
+    if (!f8) return hipErrorInvalidValue;
+    return small ? launch_one<M, true, S, 4, 1>(a, tiles, st)
+                 : launch_one<M, true, L, 4, 1>(a, tiles, st);
+  }
+  if (small)
+    return f8 ? launch_one<M, true, S, 8, 2>(a, tiles, st) : launch_one<M, false, S, 8, 2>(a, tiles, st);
+  if (ring == 2)
+    return f8 ? launch_one<M, true, L, 8, 2>(a, tiles, st) : launch_one<M, false, L, 8, 2>(a, tiles, st);
+  return f8 ? launch_one<M, true, L, 8, 4>(a, tiles, st) : launch_one<M, false, L, 8, 4>(a, tiles, st);
+}
+
+// e4m3 down; res: two phases hold all of K.
+hipError_t launch_down(const GemmArgs& a, bool small, int ring, bool res, int tiles,
+                       hipStream_t st) {
+  constexpr int S = kPBlocksSmall, L = kPBlocksLarge;
+  constexpr int M = kModePlain;
+  if (ring == 1)
+    return small ? launch_one<M, true, S, 4, 1>(a, tiles, st)
+                 : launch_one<M, true, L, 4, 1>(a, tiles, st);
+  if (ring == 2)
+    return small ? launch_one<M, true, S, 8, 2>(a, tiles, st)
+                 : launch_one<M, true, L, 8, 2>(a, tiles, st);
+  if (res)
+    return small ? launch_one<M, true, S, 8, 4, true>(a, tiles, st)
+                 : launch_one<M, true, L, 8, 4, true>(a, tiles, st);
+  return small ? launch_one<M, true, S, 8, 4>(a, tiles, st)
+               : launch_one<M, true, L, 8, 4>(a, tiles, st);
+}
+
+}  // namespace
+
+bool stream_takes(const GemmArgs& a, int bm) {
+  return (bm == kStreamRowsSmall || bm == kStreamRowsLarge) && a.table && ring_of(a, 0) > 1;
+}
+
+hipError_t launch_prefill_stream(int mode, const GemmArgs& a_in, int max_tiles, hipStream_t st) {
+  GemmArgs a = a_in;
+  const bool f8 = (a.op[0].N > 0 && a.op[0].fp8) || (a.op[1].N > 0 && a.op[1].fp8);
+  const bool small = a.bm == kStreamRowsSmall;
+  const int sub = small ? kStreamRowsSmall : kStreamRowsLarge;
+  a.nsub = a.table ? (a.bm + sub - 1) / sub : 1;
+  const int tiles = a.table ? max_tiles * a.nsub : (a.T + sub - 1) / sub;
+  int ring = 4;
+  bool res = true;
+  for (int i = 0; i < 2; ++i) {
+    const GemmOperand& o = a.op[i];
+    if (o.N <= 0) continue;
+    const int r = ring_of(a, i);
+    ring = r < ring ? r : ring;
+    res = res && o.K == 8 * kPKC;
+    if (r == 1) continue;
+    a.in_bytes[i] = (unsigned)((i == 0 && !o.in_map ? (long long)a.P : a.T) * o.ld_in * 2);
+    a.out_bytes[i] = (unsigned)((i == 0 ? (long long)a.P : a.T) * o.ld_out * 2);
+  }
+  if (mode == kModeSwiglu) return launch_gate_up(a, f8, small, ring, tiles, st);
+  return f8 ? launch_down(a, small, ring, res, tiles, st) : hipErrorInvalidValue;
+}
+
+}  // namespace moe
