@@ -41,7 +41,6 @@ namespace moe {
 
 namespace {
 
-constexpr int kDecThreads = 256;  // K3 (several tokens): four waves, one row each
 constexpr int kGuWaves = 4;       // K2: waves per workgroup, one gate/up row pair each
 static_assert(kGuWaves >= kDecMaxTokens, "K2 routes one token per wave");
 
@@ -96,33 +95,33 @@ __device__ __forceinline__ float swiglu(float g, float u) {
 
 // ------------------------------------------------------------------------------- K1
 
-// grid: n_pack + IS (shared rows, when sh_gate) workgroups of one wave. The weight rows are
-// requested before the token rows so that both are in flight together. With norm_x every
-// wave normalises the token rows in registers (while its weight rows are in flight) and
-// workgroup 0 stores them.
-template <int NT, int HC>
+// grid: (n_pack + IS (shared rows, when sh_gate)) x T workgroups of one wave, one token each:
+// with the tokens of a row in one wave the norm's arithmetic was serial over the tokens (5.8 µs
+// at T = 3 against 4.5; the router rows are re-read from the L2). The weight rows are requested
+// before the token row so that both are in flight together. With norm_x every wave normalises
+// its token row in registers (while its weight rows are in flight) and the token's first
+// workgroup stores it.
+template <int HC>
 __global__ __launch_bounds__(64) void k_dec_router(DecodeArgs a) {
   const int lane = threadIdx.x;
   const int g = blockIdx.x;
+  const int t = blockIdx.y;
   const int H = HC * 512;
+  const long long tr = (long long)t * H;
   const bool router = g < a.n_pack;
   const int n = g - a.n_pack;  // shared gate/up row pair
   const uint16_t* r0 = router ? a.w_pack + (long long)g * H : a.sh_gate + (long long)n * H;
   const uint16_t* r1 = router ? r0 : a.sh_up + (long long)n * H;
   uint4 w0[HC], w1[HC];
-  uint4 xv[NT][HC];
+  uint4 xv[HC];
   if (a.norm_x) {
-    // post-attention add + RMSNorm of each token row, as k_add_rms computes it: the token
-    // rows are requested first, then the weight rows, so the norm's arithmetic runs while
-    // the weight rows are in flight
-    uint4 tot[NT][HC], hv[NT][HC], wv[HC];
+    // post-attention add + RMSNorm of the token row, as k_add_rms computes it: the token row
+    // is requested first, then the weight rows, so the norm's arithmetic runs while the
+    // weight rows are in flight
+    uint4 tot[HC], hv[HC], wv[HC];
     const bool has_h = a.norm_h != nullptr;
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const long long tr = (long long)min(t, a.T - 1) * H;
-      load_row<HC, true>(a.norm_x + tr, H, lane, tot[t]);
-      if (has_h) load_row<HC, true>(a.norm_h + tr, H, lane, hv[t]);
-    }
+    load_row<HC, true>(a.norm_x + tr, H, lane, tot);
+    if (has_h) load_row<HC, true>(a.norm_h + tr, H, lane, hv);
     load_row<HC, true>(a.norm_w, H, lane, wv);
 #pragma unroll
     for (int c = 0; c < HC; ++c) w0[c] = ld16_stream(r0 + c * 512 + lane * 8);
@@ -130,14 +129,10 @@ __global__ __launch_bounds__(64) void k_dec_router(DecodeArgs a) {
 #pragma unroll
       for (int c = 0; c < HC; ++c) w1[c] = ld16_stream(r1 + c * 512 + lane * 8);
     }
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      add_rms_compute<HC>(has_h, H, a.norm_eps, tot[t], hv[t], wv, xv[t]);
-      if (g == 0 && t < a.T) {
-        const long long tr = (long long)t * H;
-        if (has_h) store_row<HC>(a.norm_sum + tr, H, lane, tot[t]);
-        store_row<HC>(a.norm_out + tr, H, lane, xv[t]);
-      }
+    add_rms_compute<HC>(has_h, H, a.norm_eps, tot, hv, wv, xv);
+    if (g == 0) {
+      if (has_h) store_row<HC>(a.norm_sum + tr, H, lane, tot);
+      store_row<HC>(a.norm_out + tr, H, lane, xv);
     }
   } else {
 #pragma unroll
@@ -147,34 +142,20 @@ __global__ __launch_bounds__(64) void k_dec_router(DecodeArgs a) {
       for (int c = 0; c < HC; ++c) w1[c] = ld16_stream(r1 + c * 512 + lane * 8);
     }
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int c = 0; c < HC; ++c)
-        xv[t][c] = ld16(a.x + (long long)min(t, a.T - 1) * H + c * 512 + lane * 8);
+    for (int c = 0; c < HC; ++c) xv[c] = ld16(a.x + tr + c * 512 + lane * 8);
   }
+  float s0 = 0.f, s1 = 0.f;
+#pragma unroll
+  for (int c = 0; c < HC; ++c) s0 = dot8(w0[c], xv[c], s0);
+  s0 = wave_sum(s0);
   if (router) {
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      float s = 0.f;
-#pragma unroll
-      for (int c = 0; c < HC; ++c) s = dot8(w0[c], xv[t][c], s);
-      s = wave_sum(s);
-      if (lane == 0 && t < a.T) a.logits[(long long)t * a.n_pack + g] = f2bf_bits(s);
-    }
+    if (lane == 0) a.logits[(long long)t * a.n_pack + g] = f2bf_bits(s0);
     return;
   }
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    float sg = 0.f, su = 0.f;
-#pragma unroll
-    for (int c = 0; c < HC; ++c) {
-      sg = dot8(w0[c], xv[t][c], sg);
-      su = dot8(w1[c], xv[t][c], su);
-    }
-    sg = wave_sum(sg);
-    su = wave_sum(su);
-    if (lane == 0 && t < a.T) a.act_sh[(long long)t * a.IS + n] = f2bf_bits(swiglu(sg, su));
-  }
+  for (int c = 0; c < HC; ++c) s1 = dot8(w1[c], xv[c], s1);
+  s1 = wave_sum(s1);
+  if (lane == 0) a.act_sh[(long long)t * a.IS + n] = f2bf_bits(swiglu(s0, s1));
 }
 
 // ------------------------------------------------------------------------------- K2
@@ -323,37 +304,23 @@ __global__ __launch_bounds__(64 * kGuWaves) void k_dec_gate_up(DecodeArgs a) {
     pmask = __ballot(lane < P && key == e);
     request(e);
   }
-  const long long base = (long long)e * 2 * a.I;
-  float sg[NT], su[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) sg[t] = su[t] = 0.f;
-#pragma unroll
-  for (int c = 0; c < HC; ++c) {
-    const uint4 wg = decode<FP8>(fg[c]);
-    const uint4 wu = decode<FP8>(fu[c]);
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      sg[t] = dot8(wg, xv[t][c], sg[t]);
-      su[t] = dot8(wu, xv[t][c], su[t]);
-    }
-  }
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    sg[t] = wave_sum(sg[t]) * scg;
-    su[t] = wave_sum(su[t]) * scu;
-  }
-  // lane 0 writes each pair of this expert (at most one per token)
+  // each pair of this expert (at most one per token): the dot products of its token alone
   while (pmask) {
     const int p = __ffsll((long long)pmask) - 1;
     pmask &= pmask - 1;
     const int t = p / a.k;
-    float g = sg[0], u = su[0];
+    float g = 0.f, u = 0.f;
 #pragma unroll
-    for (int tt = 1; tt < NT; ++tt)
-      if (t == tt) {
-        g = sg[tt];
-        u = su[tt];
+    for (int tt = 0; tt < NT; ++tt) {
+      if (t != tt) continue;
+#pragma unroll
+      for (int c = 0; c < HC; ++c) {
+        g = dot8(decode<FP8>(fg[c]), xv[tt][c], g);
+        u = dot8(decode<FP8>(fu[c]), xv[tt][c], u);
       }
+    }
+    g = wave_sum(g) * scg;
+    u = wave_sum(u) * scu;
     if (lane == 0) a.act[(long long)p * a.I + n] = f2bf_bits(swiglu(g, u));
   }
 }
@@ -488,38 +455,24 @@ __attribute__((amdgpu_waves_per_eu(HC <= 4 ? 4 : 1))) void k_dec_gate_up_multi(D
     const int b = g & 1;
     const int n = (blk0 + g) * kGuWaves + wave;
     if (g + 1 < G) request(b ^ 1, (blk0 + g + 1) * kGuWaves + wave);
-    float sg[NT], su[NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) sg[t] = su[t] = 0.f;
-#pragma unroll
-    for (int c = 0; c < HC; ++c) {
-      const uint4 wg = decode<FP8>(fg[b][c]);
-      const uint4 wu = decode<FP8>(fu[b][c]);
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const uint4 xv = s_x[t * kRowU4 + c * 64 + lane];
-        sg[t] = dot8(wg, xv, sg[t]);
-        su[t] = dot8(wu, xv, su[t]);
-      }
-    }
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      sg[t] = wave_sum(sg[t]) * scg[b];
-      su[t] = wave_sum(su[t]) * scu[b];
-    }
-    // lane 0 writes each pair of this expert (at most one per token)
+    // each pair of this expert (at most one per token): the dot products of its token alone.
+    // An expert rarely serves more than one of four tokens; multiplying all of them for every
+    // expert made the launch VALU-bound (T = 3 e4m3 22.5 µs, now 17.2, 11 by its bytes; T = 4
+    // bf16 29.3, now 25.9).
     unsigned long long pmask = pmask0;
     while (pmask) {
       const int p = __ffsll((long long)pmask) - 1;
       pmask &= pmask - 1;
-      const int t = p / a.k;
-      float gg = sg[0], uu = su[0];
+      const uint4* xt = s_x + (p / a.k) * kRowU4 + lane;
+      float gg = 0.f, uu = 0.f;
 #pragma unroll
-      for (int tt = 1; tt < NT; ++tt)
-        if (t == tt) {
-          gg = sg[tt];
-          uu = su[tt];
-        }
+      for (int c = 0; c < HC; ++c) {
+        const uint4 xv = xt[c * 64];
+        gg = dot8(decode<FP8>(fg[b][c]), xv, gg);
+        uu = dot8(decode<FP8>(fu[b][c]), xv, uu);
+      }
+      gg = wave_sum(gg) * scg[b];
+      uu = wave_sum(uu) * scu[b];
       if (lane == 0) a.act[(long long)p * a.I + n] = f2bf_bits(swiglu(gg, uu));
     }
   }
@@ -527,101 +480,110 @@ __attribute__((amdgpu_waves_per_eu(HC <= 4 ? 4 : 1))) void k_dec_gate_up_multi(D
 
 // ------------------------------------------------------------------------------- K3
 
-// grid: H / 4 workgroups; wave w computes hidden row 4 * blockIdx.x + w of every token.
-template <int NT, int IC, bool FP8>
-__global__ __launch_bounds__(kDecThreads) void k_dec_down(DecodeArgs a) {
+// Two to four tokens. An item is a routed pair or one token's shared-expert row set; a wave
+// takes items wave, wave + nw, .. and streams kDownRows consecutive rows of an item's expert
+// (contiguous memory) against its one activation row, two items in flight. The combine runs
+// over the items' results in LDS in routing order. The kernel is bound by the latency of its
+// loads: one wave per hidden row walking all pairs in groups of eight took four dependent round
+// trips and read every activation row once per hidden row (T = 3 e4m3: 15.1 µs, now 9.9; T = 4
+// bf16 17.1, now 14.9). All of a T <= 4 launch is resident at 64 registers (e4m3 14.5 µs at 125). grid:
+// H / kDownRows workgroups of nw waves.
+constexpr int kDownRows = 4;  // one token at C2: 18.3 µs per layer against 18.8 (8 rows), 18.4 (2)
+constexpr int kDownWaves = 16;  // most waves of a several-token workgroup
+template <int IC, bool FP8>
+__global__ __launch_bounds__(64 * kDownWaves)
+__attribute__((amdgpu_waves_per_eu(IC == 1 ? 8 : 4))) void k_dec_down(DecodeArgs a) {
+  __shared__ float s_term[64 + kDecMaxTokens][kDownRows];
   const int lane = threadIdx.x & 63;
-  const int n = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nw = blockDim.x >> 6;
+  const int n0 = blockIdx.x * kDownRows;
   const int I = IC * 512;
   const int P = a.T * a.k;
   const int H = a.H;
   const bool shared = a.sh_down != nullptr;
   const int isc = a.IS / 512;
-
-  // shared row and the shared activations do not depend on the routing: request them first
-  uint4 ws[2], xs[NT][2];
-  if (shared) {
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-      if (c < isc) ws[c] = ld16_stream(a.sh_down + (long long)n * a.IS + c * 512 + lane * 8);
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int c = 0; c < 2; ++c)
-        if (c < isc)
-          xs[t][c] = ld16(a.act_sh + (long long)min(t, a.T - 1) * a.IS + c * 512 + lane * 8);
+  // the combine's other inputs, requested up front: thread 4 t + r finishes row r of token t
+  float seg_in = 0.f, res_in = 0.f;
+  const int ft = threadIdx.x / kDownRows, fr = threadIdx.x % kDownRows;
+  if (ft < a.T) {
+    if (shared) seg_in = bf_bits2f(a.logits[(long long)ft * a.n_pack + a.E]);
+    if (a.residual) res_in = bf_bits2f(a.residual[(long long)ft * H + n0 + fr]);
   }
-  // routing, shared-gate logit and residual of every token: one round trip together
-  const int kv = lane < P ? a.idx32[lane] : 0;
-  const float wv = lane < P ? bf_bits2f(a.wts[lane]) : 0.f;
-  const int tl = min(lane, a.T - 1);
-  // unconditional loads from always-valid addresses (a predicated load would be waited on
-  // before the branch around it)
-  const uint16_t* segp = shared ? a.logits + (long long)tl * a.n_pack + a.E : a.wts;
-  const uint16_t* resp = a.residual ? a.residual + (long long)tl * H + n : a.wts;
-  const float seg_l = bf_bits2f(*segp);
-  const float res_l = bf_bits2f(*resp);
-
-  float acc[NT];
+  struct Item {
+    WFrag<FP8> w[kDownRows][IC];
+    uint4 x[IC];
+    float wt;
+    int e;
+  };
+  auto request = [&](int p, Item& it) __attribute__((always_inline)) {
+    it.e = __builtin_amdgcn_readfirstlane(a.idx32[p]);
+    it.wt = bf_bits2f(a.wts[p]);
 #pragma unroll
-  for (int t = 0; t < NT; ++t) acc[t] = 0.f;
-  // pairs in groups of 8: all loads of a group are in flight before the first dot
-  for (int p0 = 0; p0 < P; p0 += 8) {
-    WFrag<FP8> wf[8][IC];
-    uint4 av[8][IC];
-    int ev[8];
-    float dsc[8];  // fp8 row scales, requested with the rows
+    for (int c = 0; c < IC; ++c) it.x[c] = ld16(a.act + (long long)p * I + c * 512 + lane * 8);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int p = min(p0 + i, P - 1);
-      ev[i] = __builtin_amdgcn_readlane(kv, p);
-      dsc[i] = a.dn_scale ? a.dn_scale[(long long)ev[i] * H + n] : 1.f;
-      const void* row = wrow<FP8>(a.down, (long long)ev[i] * H + n, I);
+    for (int r = 0; r < kDownRows; ++r) {
+      const void* row = wrow<FP8>(a.down, (long long)it.e * H + n0 + r, I);
 #pragma unroll
-      for (int c = 0; c < IC; ++c) {
-        wf[i][c] = ldraw<FP8>(row, c * 512 + lane * 8);
-        av[i][c] = ld16(a.act + (long long)p * I + c * 512 + lane * 8);
-      }
+      for (int c = 0; c < IC; ++c) it.w[r][c] = ldraw<FP8>(row, c * 512 + lane * 8);
+    }
+  };
+  auto finish = [&](int p, const Item& it, const float (&scl)[kDownRows])
+                    __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < kDownRows; ++r) {
+      float d = 0.f;
+#pragma unroll
+      for (int c = 0; c < IC; ++c) d = dot8(decode<FP8>(it.w[r][c]), it.x[c], d);
+      const float y = rbf(wave_sum(d) * scl[r]);
+      if (lane == r) s_term[p][r] = a.round_w ? rbf(it.wt * y) : it.wt * y;
+    }
+  };
+  auto scales = [&](const Item& it, float (&scl)[kDownRows]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < kDownRows; ++r)
+      scl[r] = a.dn_scale ? a.dn_scale[(long long)it.e * H + n0 + r] : 1.f;
+  };
+  for (int p = wave; p < P; p += 2 * nw) {
+    Item it0, it1;
+    float scl0[kDownRows], scl1[kDownRows];
+    request(p, it0);
+    const bool two = p + nw < P;
+    if (two) request(p + nw, it1);
+    scales(it0, scl0);
+    if (two) scales(it1, scl1);
+    finish(p, it0, scl0);
+    if (two) finish(p + nw, it1, scl1);
+  }
+  // the last waves, which have fewer pairs, take the shared expert's rows of one token each
+  for (int t = nw - 1 - wave; shared && t < a.T; t += nw) {
+    float d[kDownRows] = {0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < isc; ++c) {
+      const uint4 xs = ld16(a.act_sh + (long long)t * a.IS + c * 512 + lane * 8);
+      uint4 ws[kDownRows];
+#pragma unroll
+      for (int r = 0; r < kDownRows; ++r)
+        ws[r] = ld16(a.sh_down + (long long)(n0 + r) * a.IS + c * 512 + lane * 8);
+#pragma unroll
+      for (int r = 0; r < kDownRows; ++r) d[r] = dot8(ws[r], xs, d[r]);
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int p = p0 + i;
-      if (p >= P) break;
-      float s = 0.f;
-#pragma unroll
-      for (int c = 0; c < IC; ++c) s = dot8(decode<FP8>(wf[i][c]), av[i][c], s);
-      s = wave_sum(s);
-      s *= dsc[i];
-      const float y = rbf(s);
-      const float w = __shfl(wv, p);
-      const float term = a.round_w ? rbf(w * y) : w * y;
-      const int t = p / a.k;  // pairs run token-major, j ascending inside a token
-#pragma unroll
-      for (int tt = 0; tt < NT; ++tt)
-        if (t == tt) acc[tt] += term;
+    for (int r = 0; r < kDownRows; ++r) {
+      const float y = rbf(wave_sum(d[r]));
+      if (lane == r) s_term[P + t][r] = y;
     }
   }
-
-  float o[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) o[t] = rbf(acc[t]);
-  if (shared) {
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      float s = 0.f;
-#pragma unroll
-      for (int c = 0; c < 2; ++c)
-        if (c < isc) s = dot8(ws[c], xs[t][c], s);
-      s = wave_sum(s);
-      const float gte = rbf(sigmoidf_(__shfl(seg_l, t)));
-      o[t] = rbf(o[t] + rbf(gte * rbf(s)));
+  __syncthreads();
+  if (ft < a.T) {
+    float acc = 0.f;
+    for (int j = 0; j < a.k; ++j) acc += s_term[ft * a.k + j][fr];  // routing order j
+    float o = rbf(acc);
+    if (shared) {
+      const float gte = rbf(sigmoidf_(seg_in));
+      o = rbf(o + rbf(gte * s_term[P + ft][fr]));
     }
-  }
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    if (t >= a.T) break;
-    // lane t holds token t's residual
-    if (lane == t) a.out[(long long)t * H + n] = f2bf_bits(a.residual ? o[t] + res_l : o[t]);
+    if (a.residual) o += res_in;
+    a.out[(long long)ft * H + n0 + fr] = f2bf_bits(o);
   }
 }
 
@@ -629,7 +591,6 @@ __global__ __launch_bounds__(kDecThreads) void k_dec_down(DecodeArgs a) {
 // wave streams kDownRows consecutive rows of its expert's down projection (contiguous
 // memory) against its one activation row, and the combine runs over the waves' results in
 // LDS in routing order. grid: H / kDownRows workgroups of (k + 1) waves.
-constexpr int kDownRows = 4;  // measured at C2: 18.3 µs per layer against 18.8 (8 rows) and 18.4 (2)
 template <int IC, bool FP8>
 __global__ __launch_bounds__(1024) void k_dec_down1(DecodeArgs a) {
   __shared__ float s_term[16][kDownRows];
@@ -740,22 +701,6 @@ bool down_legacy() {
   return env && env[0] == 'r';
 }
 
-template <int NT>
-hipError_t launch_router_nt(const DecodeArgs& a, hipStream_t s) {
-  const int grid = a.n_pack + (a.sh_gate && !a.sh_in_gate_up ? a.IS : 0);
-  switch (a.H / 512) {
-#define L(HC)                                                                             \
-  case HC:                                                                                \
-    hipLaunchKernelGGL((k_dec_router<NT, HC>), dim3(grid), dim3(64), 0, s, a); \
-    break;
-    L(1) L(2) L(4) L(8)
-#undef L
-    default:
-      return hipErrorInvalidValue;
-  }
-  return hipGetLastError();
-}
-
 template <int NT, bool FP8>
 hipError_t launch_gate_up_nt(const DecodeArgs& a, hipStream_t s) {
   // three or four tokens: G row blocks per routed workgroup (I / kGuWaves is a multiple of 4)
@@ -783,35 +728,42 @@ hipError_t launch_gate_up_nt(const DecodeArgs& a, hipStream_t s) {
   return hipErrorInvalidValue;
 }
 
-template <int NT, bool FP8>
-hipError_t launch_down_nt(const DecodeArgs& a, hipStream_t s) {
-  if (NT == 1 && a.T == 1 && a.k <= 15 && a.H % kDownRows == 0 && !down_legacy()) {
-    const int grid = a.H / kDownRows;
+template <bool FP8>
+hipError_t launch_down(const DecodeArgs& a, hipStream_t s) {
+  const int grid = a.H / kDownRows;
+  if (a.I != 512 && a.I != 1024) return hipErrorInvalidValue;
+  if (a.T == 1 && a.k <= 15 && !down_legacy()) {
     const dim3 block(64 * (a.k + 1));
     if (a.I == 512)
       hipLaunchKernelGGL((k_dec_down1<1, FP8>), dim3(grid), block, 0, s, a);
-    else if (a.I == 1024)
-      hipLaunchKernelGGL((k_dec_down1<2, FP8>), dim3(grid), block, 0, s, a);
     else
-      return hipErrorInvalidValue;
+      hipLaunchKernelGGL((k_dec_down1<2, FP8>), dim3(grid), block, 0, s, a);
     return hipGetLastError();
   }
-  const int grid = a.H / 4;
+  const int items = a.T * (a.k + (a.sh_down ? 1 : 0));
+  const int nw = (items + 1) / 2 < kDownWaves ? (items + 1) / 2 : kDownWaves;
   if (a.I == 512)
-    hipLaunchKernelGGL((k_dec_down<NT, 1, FP8>), dim3(grid), dim3(kDecThreads), 0, s, a);
-  else if (a.I == 1024)
-    hipLaunchKernelGGL((k_dec_down<NT, 2, FP8>), dim3(grid), dim3(kDecThreads), 0, s, a);
+    hipLaunchKernelGGL((k_dec_down<1, FP8>), dim3(grid), dim3(64 * nw), 0, s, a);
   else
-    return hipErrorInvalidValue;
+    hipLaunchKernelGGL((k_dec_down<2, FP8>), dim3(grid), dim3(64 * nw), 0, s, a);
   return hipGetLastError();
 }
 
 }  // namespace
 
 hipError_t launch_decode_router(const DecodeArgs& a, hipStream_t s) {
-  if (a.T == 1) return launch_router_nt<1>(a, s);
-  if (a.T == 2) return launch_router_nt<2>(a, s);
-  return launch_router_nt<4>(a, s);
+  const dim3 grid(a.n_pack + (a.sh_gate && !a.sh_in_gate_up ? a.IS : 0), a.T);
+  switch (a.H / 512) {
+#define L(HC)                                                                  \
+  case HC:                                                                     \
+    hipLaunchKernelGGL((k_dec_router<HC>), grid, dim3(64), 0, s, a);           \
+    break;
+    L(1) L(2) L(4) L(8)
+#undef L
+    default:
+      return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
 }
 
 hipError_t launch_decode_gate_up(const DecodeArgs& a, hipStream_t s) {
@@ -826,14 +778,7 @@ hipError_t launch_decode_gate_up(const DecodeArgs& a, hipStream_t s) {
 }
 
 hipError_t launch_decode_down(const DecodeArgs& a, hipStream_t s) {
-  if (a.fp8) {
-    if (a.T == 1) return launch_down_nt<1, true>(a, s);
-    if (a.T == 2) return launch_down_nt<2, true>(a, s);
-    return launch_down_nt<4, true>(a, s);
-  }
-  if (a.T == 1) return launch_down_nt<1, false>(a, s);
-  if (a.T == 2) return launch_down_nt<2, false>(a, s);
-  return launch_down_nt<4, false>(a, s);
+  return a.fp8 ? launch_down<true>(a, s) : launch_down<false>(a, s);
 }
 
 }  // namespace moe

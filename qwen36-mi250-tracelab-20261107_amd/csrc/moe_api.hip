@@ -116,11 +116,14 @@ bool prefill_side_enabled() {
   return env && env[0] == '1';
 }
 
-// Block forward: the shared expert on the auxiliary stream where it runs as separate
-// launches anyway: fp8 routed experts whose bf16 shared tiles do not share the routed
-// launches (MOE_MIXED=0), or prefill tiles.
-bool block_side_enabled(bool fp8, bool prefill) {
-  return (fp8 && !mixed_enabled()) || prefill;
+// Block forward: the shared expert on the auxiliary stream where its tiles do not share the
+// routed launches: fp8 routed experts (among them the tiled ones with MOE_MIXED=0), and the
+// streaming kernel's bf16 tiles, which fill the GPU by themselves (T = 1111: 402 against 406 µs
+// in one launch). In the 256-row tiles it goes first in the routed launches: the two hops
+// between queues cost more than the overlap with the router gains (T = 4096: 502 against
+// 509 µs).
+bool block_side_enabled(bool fp8, bool prefill, int bm) {
+  return (fp8 && !mixed_enabled()) || (prefill && bm != prefill_tile_rows());
 }
 
 size_t align256(size_t n) { return (n + 255) & ~size_t(255); }
@@ -892,11 +895,12 @@ int block_forward(const void* x, int T, int H, int E, int k, int I, int IS, cons
     x = nm->out;
     residual = nm->h ? nm->total : nm->x;
   }
-  // The shared expert depends on x alone: where its projections would run as launches of
-  // their own anyway (fp8 routed experts, prefill tiles), they run on the auxiliary stream
+  // The shared expert depends on x alone: where its projections run as launches of their own
+  // (block_side_enabled), they run on the auxiliary stream
   // from the start of the block, beside the router and routing, and join before the combine.
-  AuxStream* aux = block_side_enabled(wdtype == MOE_WEIGHTS_FP8_E4M3, w.prefill) ? aux_stream(s)
-                                                                                : nullptr;
+  AuxStream* aux = block_side_enabled(wdtype == MOE_WEIGHTS_FP8_E4M3, w.prefill, w.bm)
+                       ? aux_stream(s)
+                       : nullptr;
   const int part = aux ? kRoutedOnly : kBoth;
   Fork fork(aux, s);  // joined before the combine, or on any early return
   if (aux) {

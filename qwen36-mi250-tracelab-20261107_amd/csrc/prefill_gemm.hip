@@ -369,7 +369,7 @@ hipError_t launch_prefill_gemm(int mode, const GemmArgs& a_in, int max_tiles, in
   // (µs against this file's kernel, H = 2048, I = 512, E = 256, top-8: gate_up at
   // T = 777 / 1111 / 2048 199 / 211 / 225 against 252 / 251 / 259, at 4096 290 against 280;
   // down 125 / 131 / 142 / 180 against 113 / 118 / 134 / 167, so bf16 down stays here).
-  if (f8 || (mode == kModeSwiglu && has0 && !has1 && stream_takes(a, bm)))
+  if (f8 || (mode == kModeSwiglu && stream_takes(a, bm)))
     return launch_prefill_stream(mode, a, max_tiles, st);
   const int out_per_wg = mode == kModeSwiglu ? PBN / 2 : PBN;
   const int nmax = a.op[0].N > a.op[1].N ? a.op[0].N : a.op[1].N;

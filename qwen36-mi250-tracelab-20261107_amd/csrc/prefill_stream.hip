@@ -623,7 +623,9 @@ hipError_t launch_down(const GemmArgs& a, bool small, int ring, bool res, int ti
 }  // namespace
 
 bool stream_takes(const GemmArgs& a, int bm) {
-  return (bm == kStreamRowsSmall || bm == kStreamRowsLarge) && a.table && ring_of(a, 0) > 1;
+  for (int i = 0; i < 2; ++i)
+    if (a.op[i].N > 0 && ring_of(a, i) == 1) return false;
+  return (bm == kStreamRowsSmall || bm == kStreamRowsLarge) && a.table;
 }
 
 hipError_t launch_prefill_stream(int mode, const GemmArgs& a_in, int max_tiles, hipStream_t st) {
