@@ -339,15 +339,16 @@ RCfg router_cfg(int T) {
 
 bool router_gemm_fits(int H, int n_pack) { return H % (32 * kRouterSplit) == 0 && n_pack % 16 == 0; }
 
-// The block forward's router for T tokens: k_router_part + k_route_part where the routing is
-// a launch of its own anyway (more than 16 tokens) and the split kernel has few workgroups.
+// The block forward's router for T tokens: k_router_part + k_route_part where the split kernel
+// has few workgroups. Up to 16 tokens one launch fewer (k_router_gemm, then routing and sort in
+// one workgroup) is the slower choice: at 16 tokens 7.8 + 10.6 µs against 4.8 + 5.0 + 4.8.
 // Measured per layer (8 layers cycled, uniform routing): 17 / 32 / 64 / 128 / 256 tokens
 // 154.0 / 207.8 / 263.9 / 297.8 / 318.9 µs against 155.4 / 209.8 / 265.6 / 298.8 / 320.6
 // with k_router_gemm then k_route; level at 512 tokens (372.8 against 371.9), slower at 767
 // (390.1 against 386.2). At C3 the router launch takes 4.8 µs against 7.7.
 bool router_part_takes(int T, int H, int n_pack) {
   const int nst = H / (32 * kRouterSplit);
-  return router_gemm_fits(H, n_pack) && (nst == 4 || nst == 8 || nst == 16) && T > 16 &&
+  return router_gemm_fits(H, n_pack) && (nst == 4 || nst == 8 || nst == 16) && T > 4 &&
          T <= 256;
 }
 
