@@ -808,7 +808,11 @@ BlockWs carve_block(void* base, int T, int H, int E, int k, int I, int IS, int n
   w.act_sh = c.take<uint16_t>((size_t)T * IS);
   w.y = c.take<uint16_t>((size_t)P * H);
   w.y_sh = c.take<uint16_t>((size_t)T * H);
-  w.part = router_part_takes(T, H, n_pack) ? c.take<float>(4 * (size_t)T * n_pack) : nullptr;
+  // the partial sums are read before the down projection writes y: they share its bytes
+  const size_t part = router_part_takes(T, H, n_pack) ? 4 * (size_t)T * n_pack : 0;
+  w.part = part == 0                                       ? nullptr
+           : part * sizeof(float) <= (size_t)P * H * sizeof(uint16_t) ? reinterpret_cast<float*>(w.y)
+                                                           : c.take<float>(part);
   w.bytes = c.off;
   return w;
 }

@@ -345,11 +345,12 @@ bool router_gemm_fits(int H, int n_pack) { return H % (32 * kRouterSplit) == 0 &
 // Measured per layer (8 layers cycled, uniform routing): 17 / 32 / 64 / 128 / 256 tokens
 // 154.0 / 207.8 / 263.9 / 297.8 / 318.9 µs against 155.4 / 209.8 / 265.6 / 298.8 / 320.6
 // with k_router_gemm then k_route; level at 512 tokens (372.8 against 371.9), slower at 767
-// (390.1 against 386.2). At C3 the router launch takes 4.8 µs against 7.7.
+// (390.1 against 386.2); an eager call of 300 tokens 340.8 against 346.2. At C3 the router launch
+// takes 4.8 µs against 7.7.
 bool router_part_takes(int T, int H, int n_pack) {
   const int nst = H / (32 * kRouterSplit);
   return router_gemm_fits(H, n_pack) && (nst == 4 || nst == 8 || nst == 16) && T > 4 &&
-         T <= 256;
+         T <= 384;
 }
 
 hipError_t launch_router_part(const void* x, int T, int H, const void* w_pack, int n_pack,

@@ -1,0 +1,106 @@
+"""The streaming prefill kernel (fp8 experts, and bf16 gate_up up to 96 rows per expert) at the
+edges of its tiles: every 16-token block count it is compiled for with the rows one below, at
+and one above a block boundary, parts of a larger table tile, each ring depth (K of 64, 128,
+192, 256, 384, 512, 768 and 1024) and experts without rows.
+
+Tolerance: the results are bf16 roundings of fp32 sums of K bf16 products; the reference sums
+in float64 and rounds at the same points, so a rounded value differs by one bf16 ulp (at most
+2^-7 of it) only where its sum lies within the fp32 error of a rounding boundary. Down: one such
+rounding, 2^-7. gate_up: those of gate (which silu magnifies by |1 + x (1 - sigmoid(x))|, at most
+8 for the |x| <= 9 met here), silu, up and product: 11 * 2^-7; and 2^-16 of the row's largest
+value for sums that cancel. Few values meet a boundary: the mean difference is at most 2^-11 of
+the mean value."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+BF16 = torch.bfloat16
+
+
+@pytest.fixture(scope="module")
+def pkg():
+    import __graft_entry__
+
+    return __graft_entry__.load_package()
+
+
+def _routing(counts, k):
+    """top_k_index [T, 1] giving expert e exactly counts[e] pairs, in a shuffled order."""
+    ids = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)])
+    g = torch.Generator().manual_seed(len(ids))
+    return ids[torch.randperm(len(ids), generator=g)].reshape(-1, k).long()
+
+
+def _bf(x):
+    return x.to(BF16).double()
+
+
+def _close(got, ref, rel):
+    got, ref = got.double().cpu(), ref.cpu()
+    bound = rel * ref.abs() + 2.0**-16 * ref.abs().amax(-1, keepdim=True)
+    assert torch.isfinite(got).all()
+    diff = (got - ref).abs()
+    assert (diff <= bound).all(), (diff - bound).max().item()
+    assert diff.mean() <= 2.0**-11 * ref.abs().mean()
+
+
+def _weights(E, H, I, fp8, pkg, dev):
+    g = torch.Generator().manual_seed(E + H + I)
+    gu = (torch.randn(E, 2 * I, H, generator=g) * 0.05).to(BF16)
+    dn = (torch.randn(E, H, I, generator=g) * 0.05).to(BF16)
+    if not fp8:
+        return (gu.to(dev), None, dn.to(dev), None), (gu.double(), dn.double())
+    (qg, sg), (qd, sd) = pkg.fp8.quantize_rows(gu), pkg.fp8.quantize_rows(dn)
+    deq = [q.float().double() * s.double()[..., None] for q, s in ((qg, sg), (qd, sd))]
+    return tuple(t.to(dev) for t in (qg, sg, qd, sd)), deq
+
+
+# rows per expert around the block counts (2, 4 / 4, 6, 8, 10 blocks of 16) and past a tile
+SMALL = [0, 1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 1, 130]
+LARGE = [0, 79, 80, 81, 95, 96, 97, 127, 128, 129, 159, 160, 161, 3, 320, 63]
+
+
+@pytest.mark.parametrize("counts,bm", [(SMALL, 256), (LARGE, 256), (SMALL, None), (LARGE, None)])
+@pytest.mark.parametrize("H,I,fp8", [(256, 128, True), (256, 384, True), (768, 128, True),
+                                     (1024, 256, True), (512, 512, True), (512, 128, False),
+                                     (768, 256, False), (256, 128, False)])
+def test_prefill_stream_tiles(pkg, counts, bm, H, I, fp8):
+    """bm None: the whole routed-experts call with its own tile size (more than 512 tokens);
+    256: the grouped operations on a table of 256-row tiles."""
+    print(f"prefill stream H={H} I={I} fp8={fp8} rows<= {max(counts)} bm={bm}", flush=True)
+    dev = torch.device("cuda")
+    E, T = len(counts), sum(counts)
+    (gu, gus, dn, dns), (gu64, dn64) = _weights(E, H, I, fp8, pkg, dev)
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn(T, H, generator=g).to(BF16)
+    idx = _routing(counts, 1)
+    act = torch.zeros(T, I, dtype=torch.float64)
+    y = torch.zeros(T, H, dtype=torch.float64)
+    for e in range(E):
+        t = torch.where(idx[:, 0] == e)[0]
+        gate, up = _bf(x[t].double() @ gu64[e][:I].T), _bf(x[t].double() @ gu64[e][I:].T)
+        act[t] = _bf(_bf(gate * torch.sigmoid(gate)) * up)
+        y[t] = act[t] @ dn64[e].T
+    if bm is None:
+        # weights of 1: the combine passes y through
+        out = pkg.ops.moe_prefill(x.to(dev), idx.to(dev), torch.ones(T, 1, dtype=BF16, device=dev),
+                                  gu, dn, gate_up_scale=gus, down_scale=dns)
+        torch.cuda.synchronize()
+        # act off in places as above: its effect on y is at most that share of sum |act w|
+        bound = torch.zeros(T, H, dtype=torch.float64)
+        for e in range(E):
+            t = torch.where(idx[:, 0] == e)[0]
+            bound[t] = act[t].abs() @ dn64[e].abs().T
+        diff = (out.double().cpu() - _bf(y)).abs()
+        assert (diff <= 2.0**-7 * y.abs() + 11 * 2.0**-7 * bound).all()
+        assert diff.mean() <= 2.0**-10 * y.abs().mean()
+        return
+    sp = pkg.ops.sort_pairs(idx.to(dev), E, bm=bm)
+    got = pkg.ops.grouped_gate_up(x.to(dev), 1, gu, sp, gus)
+    order = sp.order.long().cpu()
+    torch.cuda.synchronize()
+    _close(got, act[order], 11 * 2.0**-7)
+    got_y = pkg.ops.grouped_down(act[order].to(BF16).to(dev), T, 1, dn, sp, dns)
+    torch.cuda.synchronize()
+    _close(got_y, _bf(y), 2.0**-7)
