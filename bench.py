@@ -281,7 +281,7 @@ def run_config(torch, dev, name, T, layers, steps, warmup, zipf=False, fp8=False
     us_k = ms * 1000.0 / (reps * layers)
     kbytes = sum(gate_up_bytes(d, T, fp8, logits=decode) for d in Ds) / len(Ds)
     res["gate_up_kernel"] = "k_dec_gate_up" if decode else (
-        ("k_prefill_gemm_f8" if fp8 else "k_prefill_gemm") if T > 512 else "k_expert_gemm")
+        ("k_prefill_stream" if fp8 else "k_prefill_gemm") if T > 512 else "k_expert_gemm")
     res["gate_up_us"] = round(us_k, 3)
     res["gate_up_bytes"] = int(kbytes)
     res["gate_up_GBps"] = round(kbytes / (us_k * 1e-6) / 1e9, 1)

@@ -61,10 +61,11 @@ const char* moe_last_error(void);
  * another thread launches through the library. */
 void moe_reload_tuning(void);
 
-/* Sorted rows per tile (bm) the fused entry points use for T tokens: 16 for one token,
- * 32 up to 512, above that 256 (the prefill tiles, bf16 or fp8-e4m3 weights: hidden a
- * multiple of 256, intermediates of 128) or else 64. A table passed to moe_grouped_gate_up /
- * moe_grouped_down must be built with a bm of 16, 32, 64, 128 or 256. */
+/* Sorted rows per tile (bm) of a table for moe_grouped_gate_up / moe_grouped_down at T tokens:
+ * 16 for one token, 32 up to 512, above that 256 (the prefill tiles, bf16 or fp8-e4m3 weights).
+ * They take tables of 16, 32, 64, 128 or 256 rows. The fused entry points choose their own
+ * tables; above 512 tokens they take the prefill kernels where hidden is a multiple of 256 and
+ * the intermediates of 128. */
 int moe_tile_rows(int T);
 
 /* Tile-table capacity for T tokens: ceil(T*k/bm) + min(E, T*k) (+ ceil(T/bm) shared tiles). */

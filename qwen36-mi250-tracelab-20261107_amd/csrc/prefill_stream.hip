@@ -1,4 +1,6 @@
-// Grouped MFMA GEMM for prefill-sized batches on gfx950 (subsystems a8, a9, a6).
+// Grouped MFMA GEMM for prefill-sized batches on gfx950 with weights streamed through registers
+// (subsystems a8, a9, a6): e4m3 weights, and the bf16 gate_up of batches with few rows per expert
+// (prefill_gemm.hip has the rest and the rule between them).
 //
 // Same contract as k_expert_gemm (expert_gemm.hip) and the reference's grouped kernels
 // (engine/fast/moe_prefill.py:156-257): for the sorted rows of ONE expert in a tile,
@@ -6,26 +8,33 @@
 //   PLAIN:  out[orow(r), n] = bf16(act_or_x[r] . W[e, n])
 // with bf16 or e4m3 weights (per-output-row fp32 scales on the fp32 accumulator).
 //
-// Split. A workgroup of 4 waves takes 128 weight rows and up to 16 * MAXB token rows of a
-// tile; wave w owns 32 weight rows (two 16-row MFMA blocks; SWIGLU: 16 gate rows and the
-// matching 16 up rows, paired in registers by the epilogue) against every token row.
+// Split. A workgroup of W = 8 waves takes blocks of 32 W weight rows and up to 16 MAXB token rows
+// of a tile; wave w owns 32 rows of a block (two 16-row MFMA blocks; SWIGLU: 16 gate rows and
+// the matching 16 up rows, paired in registers by the epilogue) against every token row.
 // * A weight row is used by one wave only, so weights go from HBM straight into that wave's
 //   registers in the MFMA A layout (lane: row l % 16, 16 bytes at 16 (l / 16); 64 contiguous
 //   bytes of each of 16 rows per load), a ring of R chunks of 64 k. The launch is bound by
-//   this stream, and registers hold more of it in flight than LDS could.
-// * Token rows are used by all four waves: global -> LDS DMA (no registers on the way) into R
-//   stages of 64 k (128 bytes of each row), requested R - 1 chunks ahead.
-// vmcnt retires in order, so a chunk's token rows are requested beside the weights of about
-// the same chunk: waiting for them never drains younger weight loads.
+//   this stream and by the stores that share the memory with it; registers hold more of it in
+//   flight than LDS could.
+// * Token rows are used by all waves: global -> LDS DMA (no registers on the way) in phases of
+//   R chunks, two stages: the next phase is requested at the start of the current one, and one
+//   barrier separates them.
+// vmcnt retires in order; every phase issues the same loads, so every wait is a constant and
+// waiting for a phase's token rows never drains younger weight loads.
 //
-// LDS layout of a stage: row r's 128 bytes at 128 r; 16-byte unit q holds logical unit
+// Measured (H = 2048, I = 512, E = 256, top-8; µs at T = 777 / 1111 / 2048 / 4096) against the
+// kernels staged through LDS before it: e4m3 gate_up 161 / 168 / 190 / 251 -> 114 / 126 / 144 /
+// 206, e4m3 down 100 / 107 / 125 / 168 -> 75 / 81 / 93 / 132, bf16 gate_up 252 / 251 / 259 / 280
+// -> 199 / 211 / 225 / 290.
+//
+// LDS layout of a chunk: row r's 128 bytes at 128 r; 16-byte unit q holds logical unit
 // q ^ (r & 7), so the fragment reads (16 rows, one unit) are bank-conflict free. With e4m3
 // weights a lane's 16 weight bytes are k = 16 kq .. + 15, fed as two k-steps of 8 bytes, so
 // the token units are permuted alike: k-step h's lane group kq reads logical unit 2 kq + h,
 // stored where the bf16 form's k-step h reads.
 //
 // The body is compiled per number of 16-token blocks (NB), so that a part-filled tile loads,
-// reads and multiplies only the blocks it has and every wait count is a constant.
+// reads and multiplies only the blocks it has.
 #include <stdint.h>
 #include <stdlib.h>
 
@@ -241,9 +250,10 @@ __device__ __forceinline__ void prefill_epilogue(const GemmArgs& args, const Gem
   }
 }
 
-// One workgroup's product: weight rows of blocks rb .. rb + nblk - 1 (expert e) against sorted
+// One workgroup's product: weight rows of blocks rb0 .. rb0 + nblk - 1 (expert e) against sorted
 // rows [r0, r1), r1 - r0 <= 16 NB. R: chunks per phase and ring depth; K / 64 is a multiple of
-// R (R = 1: any K, multiple of 32).
+// R, at least 2 R (R = 1: any K, multiple of 32, one chunk at a time). RES: K = 128 R, both
+// phases stay in LDS for all blocks.
 template <int MODE, bool FP8, int NB, int W, int R, bool RES>
 __device__ __forceinline__ void prefill_body(const GemmArgs& args, const GemmOperand& op,
                                              bool routed, int e, int r0, int r1, int rb0, int nblk,
