@@ -65,17 +65,13 @@ __host__ __device__ inline int prefill_start_chunk(int e, int nch) {
   return nch % 4 ? 0 : e % (nch / 4) * 4;
 }
 
-// Prefill batches. launch_prefill_gemm (prefill_gemm.hip) takes tables of bm <= 256 sorted rows
-// per tile (prefill_tile_rows() for the grouped operations, prefill_block_rows for the fused
-// entry points) and passes what prefill_stream.hip does better on to it.
-constexpr int kStreamRowsSmall = 64, kStreamRowsLarge = 160;  // tiles of prefill_stream.hip
+// Prefill batches. launch_prefill_gemm (prefill_gemm.hip) takes tables of prefill_tile_rows()
+// sorted rows per tile and passes e4m3 weights on to prefill_stream.hip.
+constexpr int kStreamRowsLarge = 160;  // rows prefill_stream.hip takes of a tile at a time
 int prefill_tile_rows();
-int prefill_block_rows(long long pairs, int experts, bool fp8);
 bool prefill_fits(int mode, const GemmOperand& op);
 hipError_t launch_prefill_gemm(int mode, const GemmArgs& a, int max_tiles, int bm, hipStream_t st);
-// Whether the routed operand's shape and table suit the pipelined form of the streaming kernel.
-bool stream_takes(const GemmArgs& a, int bm);
-// a.bm and a.shared_first set; one weight type; prefill_fits operands.
+// a.bm and a.shared_first set; e4m3 weights; prefill_fits operands.
 hipError_t launch_prefill_stream(int mode, const GemmArgs& a, int max_tiles, hipStream_t st);
 
 }  // namespace moe

@@ -59,7 +59,7 @@ int tile_rows_for(int T, int k, int E, int H, int I, int IS, bool fp8) {
   // bf16 49 / 59 / 69 against 51 / 60 / 69; one token 44 against 40 (bf16)
   if (T <= 1) return 16;
   if (T <= 512) return 32;
-  return prefill_for(T, H, I, IS) ? prefill_block_rows((long long)T * k, E, fp8) : 64;
+  return prefill_for(T, H, I, IS) ? prefill_tile_rows() : 64;
 }
 
 thread_local std::string g_err;
@@ -122,8 +122,8 @@ bool prefill_side_enabled() {
 // in one launch). In the 256-row tiles it goes first in the routed launches: the two hops
 // between queues cost more than the overlap with the router gains (T = 4096: 502 against
 // 509 µs).
-bool block_side_enabled(bool fp8, bool prefill, int bm) {
-  return (fp8 && !mixed_enabled()) || (prefill && bm != prefill_tile_rows());
+bool block_side_enabled(bool fp8, bool prefill, long long P, int E) {
+  return (fp8 && !mixed_enabled()) || (prefill && (fp8 || P <= 96LL * E));
 }
 
 size_t align256(size_t n) { return (n + 255) & ~size_t(255); }
@@ -902,7 +902,7 @@ int block_forward(const void* x, int T, int H, int E, int k, int I, int IS, cons
   // The shared expert depends on x alone: where its projections run as launches of their own
   // (block_side_enabled), they run on the auxiliary stream
   // from the start of the block, beside the router and routing, and join before the combine.
-  AuxStream* aux = block_side_enabled(wdtype == MOE_WEIGHTS_FP8_E4M3, w.prefill, w.bm)
+  AuxStream* aux = block_side_enabled(wdtype == MOE_WEIGHTS_FP8_E4M3, w.prefill, (long long)T * k, E)
                        ? aux_stream(s)
                        : nullptr;
   const int part = aux ? kRoutedOnly : kBoth;

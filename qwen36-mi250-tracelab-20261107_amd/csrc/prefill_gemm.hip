@@ -1,6 +1,5 @@
 // Grouped MFMA GEMM for prefill-sized batches on gfx950, bf16 weights (subsystems a8, a9, a6).
-// prefill_stream.hip has the e4m3 form and the bf16 gate_up of batches with fewer rows per
-// expert.
+// prefill_stream.hip has the e4m3 form.
 //
 // Same contract as k_expert_gemm (expert_gemm.hip) and the reference's grouped kernels
 // (engine/fast/moe_prefill.py:156-257): for a tile of up to 256 sorted rows of ONE expert,
@@ -308,15 +307,6 @@ __global__ __launch_bounds__(kThreads, 1) void k_prefill_gemm(GemmArgs args) {
 
 int prefill_tile_rows() { return PBM; }
 
-// Sorted rows per tile of the block's own tables: what the launches of its projections take at
-// best. e4m3 experts: 64 rows where the experts' average share is at most 44 rows, else 160.
-// bf16 ones alike up to 96 rows on average, where gate_up runs on the streaming kernel; above
-// that this file's 256-row tiles do both projections.
-int prefill_block_rows(long long pairs, int experts, bool fp8) {
-  if (!fp8 && pairs > 96LL * experts) return PBM;
-  return pairs <= 44LL * experts ? kStreamRowsSmall : kStreamRowsLarge;
-}
-
 bool prefill_fits(int mode, const GemmOperand& op) {
   if (op.N <= 0) return true;
   // SWIGLU: whole 128-row gate/up blocks; PLAIN: any multiple of 16 rows (the last block of
@@ -345,7 +335,7 @@ hipError_t allow_lds(const void* fn, int mode, int bytes) {
 hipError_t launch_prefill_gemm(int mode, const GemmArgs& a_in, int max_tiles, int bm,
                                hipStream_t st) {
   GemmArgs a = a_in;
-  if (bm > PBM) return hipErrorInvalidValue;
+  if (bm != PBM) return hipErrorInvalidValue;
   if (!prefill_fits(mode, a.op[0]) || !prefill_fits(mode, a.op[1])) return hipErrorInvalidValue;
   const bool has0 = a.op[0].N > 0, has1 = a.op[1].N > 0;
   if (has0 && has1 && a.op[0].fp8 != a.op[1].fp8) {
@@ -365,11 +355,7 @@ hipError_t launch_prefill_gemm(int mode, const GemmArgs& a_in, int max_tiles, in
     const char* env = knob(kKnobPrefillSharedFirst);
     if (!(env && env[0] == '0')) a.shared_first = (a.T + bm - 1) / bm;
   }
-  // The streaming kernel's: e4m3 weights, and the routed bf16 gate_up on its own tile sizes
-  // (µs against this file's kernel, H = 2048, I = 512, E = 256, top-8: gate_up at
-  // T = 777 / 1111 / 2048 199 / 211 / 225 against 252 / 251 / 259, at 4096 290 against 280;
-  // down 125 / 131 / 142 / 180 against 113 / 118 / 134 / 167, so bf16 down stays here).
-  if (f8 || (mode == kModeSwiglu && stream_takes(a, bm)))
+  if (f8)
     return launch_prefill_stream(mode, a, max_tiles, st);
   const int out_per_wg = mode == kModeSwiglu ? PBN / 2 : PBN;
   const int nmax = a.op[0].N > a.op[1].N ? a.op[0].N : a.op[1].N;

@@ -1,6 +1,7 @@
 // Grouped MFMA GEMM for prefill-sized batches on gfx950 with weights streamed through registers
-// (subsystems a8, a9, a6): e4m3 weights, and the bf16 gate_up of batches with few rows per expert
-// (prefill_gemm.hip has the rest and the rule between them).
+// (subsystems a8, a9, a6): e4m3 weights (prefill_gemm.hip has bf16 ones, for which this form
+// measured slower where expert popularity is skewed: a block of 1111 tokens, Zipf(1.1) routing,
+// 457 against 438 µs).
 //
 // Same contract as k_expert_gemm (expert_gemm.hip) and the reference's grouped kernels
 // (engine/fast/moe_prefill.py:156-257): for the sorted rows of ONE expert in a tile,
@@ -22,10 +23,10 @@
 // vmcnt retires in order; every phase issues the same loads, so every wait is a constant and
 // waiting for a phase's token rows never drains younger weight loads.
 //
-// Measured (H = 2048, I = 512, E = 256, top-8; µs at T = 777 / 1111 / 2048 / 4096) against the
-// kernels staged through LDS before it: e4m3 gate_up 161 / 168 / 190 / 251 -> 114 / 126 / 144 /
-// 206, e4m3 down 100 / 107 / 125 / 168 -> 75 / 81 / 93 / 132, bf16 gate_up 252 / 251 / 259 / 280
-// -> 199 / 211 / 225 / 290.
+// Measured (block, H = 2048, I = 512, E = 256, top-8, µs) against the kernel staged through LDS
+// before it: 1111 / 2048 tokens 312 / 358 -> 289 / 320; Zipf(1.1) routing at 600 / 1111 / 2500 /
+// 4096 tokens 310 / 356 / 433 / 541 -> 289 / 330 / 417 / 545. 160-row tiles for every batch: 64-row
+// ones gain 3 % at 1111 tokens with uniform routing and lose 13 % with Zipf.
 //
 // LDS layout of a chunk: row r's 128 bytes at 128 r; 16-byte unit q holds logical unit
 // q ^ (r & 7), so the fragment reads (16 rows, one unit) are bank-conflict free. With e4m3
@@ -58,7 +59,6 @@ template <int MODE>
 constexpr int kStorePolicy = MODE == kModeSwiglu ? 16 : 0;
 constexpr int kXcds = 8;            // XCDs of an MI355X (round-robin dispatch)
 constexpr int kPBlocksLarge = kStreamRowsLarge / 16;  // MAXB
-constexpr int kPBlocksSmall = kStreamRowsSmall / 16;
 }  // namespace
 
 // The NB token fragments (16 rows each, 2 KiB apart) at LDS byte address addr, waited for.
@@ -496,9 +496,11 @@ __attribute__((amdgpu_waves_per_eu(MAXB <= 4 ? 3 : 2))) void k_prefill_stream(Ge
   const int rb = (j - (j / ng) * ng) * args.nblk;
   int e, r0, r1;
   if (args.table) {
-    // nsub parts of 16 MAXB rows per table tile
-    const int sub = tile % args.nsub;
-    tile /= args.nsub;
+    // nsub parts of 16 MAXB rows per table tile, all the first parts before the second ones
+    // (alternating, the parts would follow the XCDs and the rarer ones leave theirs idle)
+    const int sub = tile / args.MTgrid;
+    tile -= sub * args.MTgrid;
+    if (sub >= args.nsub) return;
     const int ntiles = args.table[3 * args.MT];
     if (tile >= ntiles) return;
     if (args.shared_first > 0) {
@@ -570,12 +572,12 @@ hipError_t launch_one(GemmArgs a, int tiles, hipStream_t st) {
   // block's weights stream through the epilogue of one (T = 777 / 1111 / 2048 / 4096, e4m3: 75 /
   // 81 / 93 / 146 µs with 4, 77 / 82 / 96 / 132 with 2, 81 / 87 / 102 / 139 with 1). gate_up
   // gains nothing that the coarser work units do not cost (144 / 206 against 138 / 223 with 2).
-  a.nblk = MODE == kModePlain ? (MAXB == kPBlocksSmall ? 4 : 2) : 1;
+  a.nblk = MODE == kModePlain ? 2 : 1;
   const long long ng = (a.nrb + a.nblk - 1) / a.nblk;
   const long long grid = (long long)((tiles + kXcds - 1) / kXcds) * kXcds * ng;
   if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
   const auto fn = &k_prefill_stream<MODE, FP8, MAXB, W, R, RES>;
-  const int which = (MODE * 2 + (FP8 ? 1 : 0)) * 8 + (MAXB == kPBlocksSmall ? 0 : 4) + (RES ? 3 : R / 2);
+  const int which = (MODE * 2 + (FP8 ? 1 : 0)) * 8 + (RES ? 3 : R / 2);
   const hipError_t err = allow_lds(reinterpret_cast<const void*>(fn), which, bytes);
   if (err != hipSuccess) return err;
   hipLaunchKernelGGL((k_prefill_stream<MODE, FP8, MAXB, W, R, RES>), dim3((unsigned)grid), dim3(64 * W),
@@ -594,56 +596,29 @@ int ring_of(const GemmArgs& a, int i) {
   return o.K % (4 * kPKC) || o.K < 8 * kPKC ? 2 : 4;
 }
 
-// gate_up's 64-row tiles take short phases: T = 777 / 1111 210 / 225 µs against 215 / 228 in
-// phases of 4 chunks (e4m3 131 / 145 against 140 / 157).
-hipError_t launch_gate_up(const GemmArgs& a, bool f8, bool small, int ring, int tiles,
-                          hipStream_t st) {
-  constexpr int S = kPBlocksSmall, L = kPBlocksLarge;
-  constexpr int M = kModeSwiglu;
-  if (ring == 1) {
-    if (!f8) return hipErrorInvalidValue;
-    return small ? launch_one<M, true, S, 4, 1>(a, tiles, st)
-                 : launch_one<M, true, L, 4, 1>(a, tiles, st);
-  }
-  if (small)
-    return f8 ? launch_one<M, true, S, 8, 2>(a, tiles, st) : launch_one<M, false, S, 8, 2>(a, tiles, st);
-  if (ring == 2)
-    return f8 ? launch_one<M, true, L, 8, 2>(a, tiles, st) : launch_one<M, false, L, 8, 2>(a, tiles, st);
-  return f8 ? launch_one<M, true, L, 8, 4>(a, tiles, st) : launch_one<M, false, L, 8, 4>(a, tiles, st);
+hipError_t launch_gate_up(const GemmArgs& a, int ring, int tiles, hipStream_t st) {
+  constexpr int L = kPBlocksLarge, M = kModeSwiglu;
+  if (ring == 1) return launch_one<M, true, L, 4, 1>(a, tiles, st);
+  if (ring == 2) return launch_one<M, true, L, 8, 2>(a, tiles, st);
+  return launch_one<M, true, L, 8, 4>(a, tiles, st);
 }
 
-// e4m3 down; res: two phases hold all of K.
-hipError_t launch_down(const GemmArgs& a, bool small, int ring, bool res, int tiles,
-                       hipStream_t st) {
-  constexpr int S = kPBlocksSmall, L = kPBlocksLarge;
-  constexpr int M = kModePlain;
-  if (ring == 1)
-    return small ? launch_one<M, true, S, 4, 1>(a, tiles, st)
-                 : launch_one<M, true, L, 4, 1>(a, tiles, st);
-  if (ring == 2)
-    return small ? launch_one<M, true, S, 8, 2>(a, tiles, st)
-                 : launch_one<M, true, L, 8, 2>(a, tiles, st);
-  if (res)
-    return small ? launch_one<M, true, S, 8, 4, true>(a, tiles, st)
-                 : launch_one<M, true, L, 8, 4, true>(a, tiles, st);
-  return small ? launch_one<M, true, S, 8, 4>(a, tiles, st)
-               : launch_one<M, true, L, 8, 4>(a, tiles, st);
+// res: two phases hold all of K.
+hipError_t launch_down(const GemmArgs& a, int ring, bool res, int tiles, hipStream_t st) {
+  constexpr int L = kPBlocksLarge, M = kModePlain;
+  if (ring == 1) return launch_one<M, true, L, 4, 1>(a, tiles, st);
+  if (ring == 2) return launch_one<M, true, L, 8, 2>(a, tiles, st);
+  if (res) return launch_one<M, true, L, 8, 4, true>(a, tiles, st);
+  return launch_one<M, true, L, 8, 4>(a, tiles, st);
 }
 
 }  // namespace
 
-bool stream_takes(const GemmArgs& a, int bm) {
-  for (int i = 0; i < 2; ++i)
-    if (a.op[i].N > 0 && ring_of(a, i) == 1) return false;
-  return (bm == kStreamRowsSmall || bm == kStreamRowsLarge) && a.table;
-}
-
 hipError_t launch_prefill_stream(int mode, const GemmArgs& a_in, int max_tiles, hipStream_t st) {
   GemmArgs a = a_in;
-  const bool f8 = (a.op[0].N > 0 && a.op[0].fp8) || (a.op[1].N > 0 && a.op[1].fp8);
-  const bool small = a.bm == kStreamRowsSmall;
-  const int sub = small ? kStreamRowsSmall : kStreamRowsLarge;
+  constexpr int sub = kStreamRowsLarge;
   a.nsub = a.table ? (a.bm + sub - 1) / sub : 1;
+  a.MTgrid = max_tiles;
   const int tiles = a.table ? max_tiles * a.nsub : (a.T + sub - 1) / sub;
   int ring = 4;
   bool res = true;
@@ -657,8 +632,8 @@ hipError_t launch_prefill_stream(int mode, const GemmArgs& a_in, int max_tiles, 
     a.in_bytes[i] = (unsigned)((i == 0 && !o.in_map ? (long long)a.P : a.T) * o.ld_in * 2);
     a.out_bytes[i] = (unsigned)((i == 0 ? (long long)a.P : a.T) * o.ld_out * 2);
   }
-  if (mode == kModeSwiglu) return launch_gate_up(a, f8, small, ring, tiles, st);
-  return f8 ? launch_down(a, small, ring, res, tiles, st) : hipErrorInvalidValue;
+  return mode == kModeSwiglu ? launch_gate_up(a, ring, tiles, st)
+                             : launch_down(a, ring, res, tiles, st);
 }
 
 }  // namespace moe
