@@ -117,11 +117,10 @@ bool prefill_side_enabled() {
 }
 
 // Block forward: the shared expert on the auxiliary stream where its tiles do not share the
-// routed launches: fp8 routed experts (among them the tiled ones with MOE_MIXED=0), and the
-// streaming kernel's bf16 tiles, which fill the GPU by themselves (T = 1111: 402 against 406 µs
-// in one launch). In the 256-row tiles it goes first in the routed launches: the two hops
-// between queues cost more than the overlap with the router gains (T = 4096: 502 against
-// 509 µs).
+// routed launches (fp8 routed experts, the tiled ones with MOE_MIXED=0), and beside bf16 prefill
+// tiles of up to 96 rows per expert on average. Above that it goes first in the routed
+// launches: the two hops between queues cost more than the overlap with the router gains
+// (T = 4096: 502 against 509 µs).
 bool block_side_enabled(bool fp8, bool prefill, long long P, int E) {
   return (fp8 && !mixed_enabled()) || (prefill && (fp8 || P <= 96LL * E));
 }

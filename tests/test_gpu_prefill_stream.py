@@ -1,4 +1,4 @@
-"""The streaming prefill kernel (fp8 experts, and bf16 gate_up up to 96 rows per expert) at the
+"""The prefill kernels (streaming e4m3, staged bf16) at the
 edges of its tiles: every 16-token block count it is compiled for with the rows one below, at
 and one above a block boundary, parts of a larger table tile, each ring depth (K of 64, 128,
 192, 256, 384, 512, 768 and 1024) and experts without rows.
