@@ -67,17 +67,21 @@ __device__ __forceinline__ float siluf_(float x) { return x / (1.0f + expf(-x));
 
 // silu with the hardware exp2 and reciprocal, each with its rounding error put back: exp(-x) as
 // exp2(t) (1 + ln2 * rest) with t + rest = -x log2(e) to about 48 bits, and one step of
-// x - q d on the quotient. Past |t| = 126 the quotient is x / 1 or x * 0 (x * 2^-126 and less)
-// and takes no corrections: they are not finite there.
+// x - q d on the quotient. From t = 64 on, numerator and denominator are scaled by 2^-64: the
+// reciprocal of a denominator above 2^126 is subnormal and comes out as 0. At |t| = 128 and more
+// (exp2 is 0 or infinite, the quotient x, -0 or NaN as siluf_'s) nothing is put back: it is not
+// finite. No bf16 x has |t| between 127.99 and 128.
 __device__ __forceinline__ float silu_fast(float x) {
   constexpr float kL2eHi = -1.44269502162933349609375f, kL2eLo = -1.92596299112661746887e-8f;
   const float t = x * kL2eHi;
-  const bool mid = fabsf(t) < 126.f;
+  const bool mid = fabsf(t) < 127.99f;
   const float rest = mid ? fmaf(x, kL2eLo, fmaf(x, kL2eHi, -t)) : 0.f;
   const float d = fmaf(__builtin_amdgcn_exp2f(t), fmaf(rest, 0.693147182464599609375f, 1.0f), 1.0f);
-  const float r = __builtin_amdgcn_rcpf(d);
-  const float q = x * r;
-  const float c = fmaf(fmaf(-q, d, x), r, q);
+  const float scale = t > 64.f ? 0x1p-64f : 1.f;
+  const float ds = d * scale, xs = x * scale;
+  const float r = __builtin_amdgcn_rcpf(ds);
+  const float q = xs * r;
+  const float c = fmaf(fmaf(-q, ds, xs), r, q);
   return mid ? c : q;
 }
 

@@ -106,34 +106,44 @@ def test_prefill_stream_tiles(pkg, counts, bm, H, I, fp8):
     _close(got_y, _bf(y), 2.0**-7)
 
 
-def test_prefill_stream_silu_range(pkg):
-    """gate_up's SiLU over its whole range: one gate value per expert, up = 1, a down row that
-    passes act[0] through. Against float64 within one bf16 ulp (2^-7 of the value); below
-    x = -87 the value is under 1e-36 and may come out as 0; infinities and NaN as torch's."""
+@pytest.mark.parametrize("fp8", [False, True])
+def test_prefill_stream_silu_range(pkg, fp8):
+    """gate_up's SiLU over its whole range: one gate value per expert (e4m3: by the row's scale),
+    up = 1, a down row that passes act[0] through. Against float64 within one bf16 ulp (2^-7 of
+    the value); below x = -88.7, where exp(-x) is past float32, the value is under 3e-37 and may
+    come out as 0; infinities and NaN as torch's."""
+    print(f"silu range fp8={fp8}", flush=True)
     dev = torch.device("cuda")
     inf = float("inf")
-    vals = [0.0, 1e-30, -1e-30, 0.5, -0.5, 1.0, -1.0, 3.0, -3.0, 7.5, -7.5, 20.0, -20.0, 60.0, -60.0,
-            -80.0, -86.0, 87.5, -87.5, 88.5, -88.5, 89.0, -95.0, 300.0, -300.0, 1e8, -1e8, 1e20,
-            -1e20, 3e38, inf, float("nan")]
+    vals = [0.0, 1e-30, -1e-30, 0.5, -0.5, 1.0, -1.0, 3.0, -3.0, 7.5, -7.5, 20.0, -20.0, 44.25, -44.5,
+            60.0, -60.0, -80.0, -86.0, -87.0, 87.5, -87.5, -88.0, 88.5, -88.5, 89.0, -89.0, -95.0,
+            300.0, -300.0, 1e8, -1e8, 1e20, -1e20, 3e38, inf, -inf, float("nan")]
     E, T, H, I = len(vals), 20 * len(vals), 256, 128
     v = torch.tensor(vals, dtype=torch.float64).to(BF16)
     gu = torch.zeros(E, 2 * I, H, dtype=BF16)
-    gu[:, 0, 0] = v
+    gu[:, 0, 0] = 1.0 if fp8 else v
     gu[:, I, 0] = 1.0
     dn = torch.zeros(E, H, I, dtype=BF16)
     dn[:, 0, 0] = 1.0
+    scales = {}
+    if fp8:
+        gu, dn = gu.to(torch.float8_e4m3fn), dn.to(torch.float8_e4m3fn)
+        gus = torch.ones(E, 2 * I)
+        gus[:, 0] = v.float()
+        scales = dict(gate_up_scale=gus.to(dev), down_scale=torch.ones(E, H, device=dev))
     x = torch.zeros(T, H, dtype=BF16)
     x[:, 0] = 1.0
     idx = _routing([20] * E, 1)
     out = pkg.ops.moe_prefill(x.to(dev), idx.to(dev), torch.ones(T, 1, dtype=BF16, device=dev),
-                              gu.to(dev), dn.to(dev))
+                              gu.to(dev), dn.to(dev), **scales)
     torch.cuda.synchronize()
     got = out[:, 0].double().cpu()
-    ref = (v.double() * torch.sigmoid(v.double()))[idx[:, 0]]
+    v64 = v.double()
+    ref = (v64 * torch.sigmoid(v64))[idx[:, 0]]
     for g, r, e in zip(got.tolist(), ref.tolist(), idx[:, 0].tolist()):
         if r != r:
             assert g != g, vals[e]
         elif r == inf:
             assert g == inf, vals[e]
         else:
-            assert abs(g - r) <= max(2.0**-7 * abs(r), 1e-36), (vals[e], g, r)
+            assert abs(g - r) <= (abs(r) if vals[e] < -88.7 else 2.0**-7 * abs(r)), (vals[e], g, r)
