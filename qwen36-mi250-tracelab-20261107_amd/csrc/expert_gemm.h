@@ -66,12 +66,20 @@ __host__ __device__ inline int prefill_start_chunk(int e, int nch) {
 }
 
 // Prefill batches. launch_prefill_gemm (prefill_gemm.hip) takes tables of prefill_tile_rows()
-// sorted rows per tile and passes e4m3 weights on to prefill_stream.hip.
+// sorted rows per tile and passes on to prefill_stream.hip the e4m3 launches that one takes.
 constexpr int kStreamRowsLarge = 160;  // rows prefill_stream.hip takes of a tile at a time
 int prefill_tile_rows();
 bool prefill_fits(int mode, const GemmOperand& op);
 hipError_t launch_prefill_gemm(int mode, const GemmArgs& a, int max_tiles, int bm, hipStream_t st);
-// a.bm and a.shared_first set; e4m3 weights; prefill_fits operands.
+// A routed e4m3 launch (a.bm set, a table, prefill_fits operands): whether it takes the streaming
+// kernel, and that kernel's launch. The streaming kernel reads a row block's weights once per
+// 160 rows of an expert, the one staged through LDS once per 256: the line is the average number
+// of rows per expert from which many experts need a second pass. A block (H = 2048, I = 512,
+// E = 256, top-8) of 3072 / 3584 / 4096 / 4608 / 5120 tokens, streaming against staged, µs: uniform
+// routing 369 / 397 / 440 / 498 / 591 against 403 / 435 / 464 / 491 / 519; Zipf(1.1) routing
+// 462 / 489 / 547 / 600 / 631 against 467 / 488 / 518 / 563 / 591.
+constexpr int kStreamRowsPerExpert = 128;
+bool prefill_stream_takes(const GemmArgs& a);
 hipError_t launch_prefill_stream(int mode, const GemmArgs& a, int max_tiles, hipStream_t st);
 
 }  // namespace moe

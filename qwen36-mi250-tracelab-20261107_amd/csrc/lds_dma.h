@@ -34,6 +34,16 @@ __device__ __forceinline__ f32x4_t mfma_frag(u32x4v a, u32x4v b, f32x4_t c) {
                                                  __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
 }
 
+// 8 e4m3 bytes -> bf16x8 (exact)
+__device__ __forceinline__ u32x4v widen8(uint32_t lo, uint32_t hi) {
+  u32x4v r;
+  r.x = fp8x2_to_bf16x2<false>(lo);
+  r.y = fp8x2_to_bf16x2<true>(lo);
+  r.z = fp8x2_to_bf16x2<false>(hi);
+  r.w = fp8x2_to_bf16x2<true>(hi);
+  return r;
+}
+
 // Wait until at most n (0..24) of this wave's DMA loads are still in flight.
 __device__ __forceinline__ void wait_loads(int n) {
   switch (n) {

@@ -1,5 +1,5 @@
-// Grouped MFMA GEMM for prefill-sized batches on gfx950, bf16 weights (subsystems a8, a9, a6).
-// prefill_stream.hip has the e4m3 form.
+// Grouped MFMA GEMM for prefill-sized batches on gfx950 (subsystems a8, a9, a6): bf16 weights, and
+// the e4m3 launches that prefill_stream.hip does not take (the second kernel below).
 //
 // Same contract as k_expert_gemm (expert_gemm.hip) and the reference's grouped kernels
 // (engine/fast/moe_prefill.py:156-257): for a tile of up to 256 sorted rows of ONE expert,
@@ -305,6 +305,271 @@ __global__ __launch_bounds__(kThreads, 1) void k_prefill_gemm(GemmArgs args) {
   }
 }
 
+// ---------------------------------------------------------------- e4m3 weights
+//
+// The same tiles (256 weight rows x up to 256 sorted rows) with e4m3 weight bytes and
+// per-output-row fp32 scales on the fp32 accumulator, for the routed launches that
+// prefill_stream.hip does not take (prefill_stream_takes). A DMA chunk is 64 k as in the bf16
+// kernel, so the token-row stages are the bf16 kernel's (256 rows x 128 bytes), while a
+// weight stage is 256 rows x 64 bytes (16 KiB): the ring holds five of them (four chunks
+// requested ahead, 144 KiB of LDS in all). A weight DMA load of a wave fills 16 rows x 64
+// bytes; lane l writes physical 16-byte unit l & 3 of row l >> 2 of its group, holding
+// logical unit (l & 3) ^ ((row >> 1) & 3), which keeps the fragment reads (8 rows of one
+// 16-byte read group) conflict-free. The weight loads use the default cache policy: the
+// non-temporal one measured slower here (gate_up / down at 4096 tokens 261 / 189 against
+// 248 / 181 µs). Each weight byte costs LDS traffic and barriers that the streaming form does
+// not have, but serves 256 rows instead of 160: at 32768 tokens (1024 rows per expert) gate_up
+// takes 1146 µs (0.96 PFLOP/s) against 1505. The walk over K starts by expert
+// (prefill_start_chunk), as the streaming form's: gate_up / down at 8192 tokens 346 / 271 µs against
+// 370 / 282 with one start for all.
+//
+// The chunk's k order is permuted the same way in both operands (the same products are
+// summed): lane group kq reads weight unit kq (16 e4m3 bytes, one ds_read_b128) once per
+// chunk and feeds its first 8 bytes to the chunk's k-step 0 and its last 8 to k-step 1,
+// against token units 2 kq and 2 kq + 1. The weights are widened to bf16 in registers
+// (gfx950's scaled conversion, scale 1: exact) just before their MFMAs. The order of the sum
+// over K and the epilogue's arithmetic are the streaming kernel's: a row has the same bits
+// whichever of the two its batch takes.
+namespace {
+constexpr int F8RowBytes = DKC;                   // weight bytes of a row per chunk: 64
+constexpr int F8Stage = 256 * F8RowBytes;         // 16 KiB
+constexpr int F8StagesA = 5, F8AheadA = 4;
+constexpr int F8ALoads = 256 / 16 / 8;            // weight DMA loads per wave per chunk: 2
+constexpr int F8LdsBytes = F8StagesA * F8Stage + kStagesB * kOpStage;  // 144 KiB
+static_assert(F8AheadA == F8StagesA - 1, "weight ring: chunk d + S - 1 into chunk d - 1's stage");
+}  // namespace
+
+// Token fragments of one k-step (the wave's 8 blocks 2 b + wn) from the B stage at bstage.
+__device__ __forceinline__ void read_bfrags(uint32_t bstage, u32x4v (&b)[8]) {
+  b[0] = lds_read_frag<0 * kBlkBytes>(bstage);
+  b[1] = lds_read_frag<2 * kBlkBytes>(bstage);
+  b[2] = lds_read_frag<4 * kBlkBytes>(bstage);
+  b[3] = lds_read_frag<6 * kBlkBytes>(bstage);
+  b[4] = lds_read_frag<8 * kBlkBytes>(bstage);
+  b[5] = lds_read_frag<10 * kBlkBytes>(bstage);
+  b[6] = lds_read_frag<12 * kBlkBytes>(bstage);
+  b[7] = lds_read_frag<14 * kBlkBytes>(bstage);
+}
+// Weight fragments of one chunk (4 row blocks of 16 rows, 16 bytes per lane).
+__device__ __forceinline__ void read_afrags8(uint32_t astage, u32x4v (&a)[4]) {
+  a[0] = lds_read_frag<0 * 16 * F8RowBytes>(astage);
+  a[1] = lds_read_frag<1 * 16 * F8RowBytes>(astage);
+  a[2] = lds_read_frag<2 * 16 * F8RowBytes>(astage);
+  a[3] = lds_read_frag<3 * 16 * F8RowBytes>(astage);
+}
+template <int N>
+__device__ __forceinline__ void tie(u32x4v (&v)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) after_wait(v[i]);
+}
+// k-step h of a chunk: weight halves h of a[], token fragments b[], first nb blocks.
+__device__ __forceinline__ void mma8(const u32x4v (&a)[4], int h, const u32x4v (&b)[8], int nb,
+                                     f32x4_t (&acc)[4][8]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const u32x4v w = h ? widen8(a[i].z, a[i].w) : widen8(a[i].x, a[i].y);
+#pragma unroll
+    for (int bb = 0; bb < 8; ++bb) {
+      if (bb >= nb) break;
+      acc[i][bb] = mfma_frag(w, b[bb], acc[i][bb]);
+    }
+  }
+}
+
+template <int MODE>
+__global__ __launch_bounds__(kThreads, 1) void k_prefill_gemm_f8(GemmArgs args) {
+  extern __shared__ uint4 smem[];  // A ring [F8StagesA][16 KiB], B ring [kStagesB][32 KiB]
+
+  // tile / row-block order and table lookup: as k_prefill_gemm, routed tiles only
+  const int nrb = args.nrb;
+  const int xcd = blockIdx.x & (kXcds - 1);
+  const int j = blockIdx.x / kXcds;
+  const int tile = (j / nrb) * kXcds + xcd;
+  const int rb = j - (j / nrb) * nrb;
+  if (tile >= args.MTgrid || tile >= args.table[3 * args.MT]) return;
+  const int e = args.table[tile];
+  if (e >= args.E) return;
+  const int r0 = args.table[args.MT + tile];
+  const int r1 = min(args.table[2 * args.MT + tile], r0 + PBM);
+  const GemmOperand& op = args.op[0];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave & 3;   // weight-row group (64 rows)
+  const int wn = wave >> 2;  // token-block parity
+  const int lr = lane & 15;
+  const int kq = lane >> 4;
+  const int ntok = r1 - r0;
+
+  // ---- DMA sources: weights (load i of the wave: 16-row group wave + 8 i), token rows (as
+  // k_prefill_gemm: 8-row group wave + 8 i, 128 bytes of each row)
+  const uint8_t* __restrict__ srca[F8ALoads];
+  const uint16_t* __restrict__ srcb[kLoadsPerWave];
+  {
+    const uint8_t* __restrict__ wbase =
+        reinterpret_cast<const uint8_t*>(op.w) + (long long)e * op.estride;
+    const int arow = lane >> 2;
+#pragma unroll
+    for (int i = 0; i < F8ALoads; ++i) {
+      const int row = (wave + 8 * i) * 16 + arow;  // 0..255
+      const int unit = (lane & 3) ^ ((row >> 1) & 3);
+      long long wrow;
+      if (MODE == kModeSwiglu) {
+        const int g = rb * (PBN / 2) + (row >> 6) * 32 + (row & 31);
+        wrow = (long long)g * op.ldw + (((row >> 5) & 1) ? op.up_off : 0);
+      } else {
+        wrow = (long long)min(rb * PBN + row, op.N - 1) * op.ldw;
+      }
+      srca[i] = wbase + wrow + unit * 16;
+    }
+    // token rows: physical unit q = (l & 7) ^ row holds logical unit 2 (q & 3) + (q >> 2), so
+    // that the units 2 kq + h that k-step h reads sit where the bf16 kernel's k-step reads
+    // them (physical (4 h + kq) ^ row): that pattern is conflict-free, 2 kq + h at the
+    // physical unit was not (3.2 bank-conflict cycles per LDS instruction)
+    const int grow = lane >> 3;
+    const int bq = (lane & 7) ^ grow;
+    const int bunit = 2 * (bq & 3) + (bq >> 2);
+#pragma unroll
+    for (int i = 0; i < kLoadsPerWave; ++i) {
+      const int row = (wave + 8 * i) * 8 + grow;
+      const int r = min(r0 + row, r1 - 1);
+      const long long src = op.in_map ? args.order[r] / args.topk : r;
+      srcb[i] = op.in + src * op.ld_in + bunit * 8;
+    }
+  }
+  char* lds = reinterpret_cast<char*>(smem);
+  char* bring_lds = lds + F8StagesA * F8Stage;
+  const int nd = op.K / DKC;
+  const int rot = prefill_start_chunk(e, nd);
+  auto chunk = [&](int d) { return d + rot < nd ? d + rot : d + rot - nd; };
+  auto issue_a = [&](int d) {
+    char* st = lds + (d % F8StagesA) * F8Stage;
+    d = chunk(d);
+#pragma unroll
+    for (int i = 0; i < F8ALoads; ++i)
+      dma16(srca[i] + d * F8RowBytes, st + (wave + 8 * i) * 1024);
+  };
+  const int nb_loads = __builtin_amdgcn_readfirstlane(
+      min(kLoadsPerWave, max(0, ((r1 - r0 + 7) / 8 - wave + 7) / 8)));
+  auto issue_b = [&](int d) {
+    char* st = bring_lds + (d % kStagesB) * kOpStage;
+    d = chunk(d);
+#pragma unroll
+    for (int i = 0; i < kLoadsPerWave; ++i)
+      if (i < nb_loads) dma16(srcb[i] + d * DKC, st + (wave + 8 * i) * 1024);
+  };
+  const uint32_t lds_base = lds_addr(lds);
+  // weight fragment: row lr of a 16-row block, logical unit kq; token fragment of k-step h:
+  // row lr, logical unit 2 kq + h (stored at physical (4 h + kq) ^ row)
+  const uint32_t ra = (uint32_t)(wm * 64 * F8RowBytes + lr * F8RowBytes +
+                                 ((kq ^ ((lr >> 1) & 3)) * 16));
+  const uint32_t rbo0 = (uint32_t)(wn * kBlkBytes + lr * kRowBytes + ((kq ^ (lr & 7)) * 16));
+  const uint32_t rbo1 = (uint32_t)(wn * kBlkBytes + lr * kRowBytes + (((4 + kq) ^ (lr & 7)) * 16));
+
+  f32x4_t acc[4][8];
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int b = 0; b < 8; ++b) acc[a][b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  const int nblk = (ntok + 15) >> 4;
+  const int nb = __builtin_amdgcn_readfirstlane(min(8, (nblk - wn + 1) >> 1));
+
+  // Pipeline: chunk d's weight fragments are read at its k-step 0 and kept for k-step 1;
+  // the token fragments of each k-step are read while the previous one is multiplied. Load
+  // order: A(0 .. S - 3), B(0), A(S - 2), B(1), A(S - 1), then at chunk d + 1's first k-step
+  // B(d + 2), A(d + S), so that the loads younger than B(d) are exactly A(d + S - 2).
+  for (int d = 0; d < F8AheadA - 1; ++d)
+    if (d < nd) issue_a(d);
+  issue_b(0);
+  if (F8AheadA - 1 < nd) issue_a(F8AheadA - 1);
+  if (nd > 1) issue_b(1);
+  if (F8AheadA < nd) issue_a(F8AheadA);
+  // younger than B(0): A(S - 2), B(1), A(S - 1)
+  wait_loads(F8ALoads * (F8AheadA - 1 < nd) + nb_loads * (nd > 1) + F8ALoads * (F8AheadA < nd));
+  __builtin_amdgcn_s_barrier();
+  u32x4v acur[4], anxt[4], b0[8], b1[8];
+  read_afrags8(lds_base + ra, acur);
+  read_bfrags(lds_base + F8StagesA * F8Stage + rbo0, b0);
+  lds_frags_ready();
+  tie(acur);
+  tie(b0);
+  for (int d = 0; d < nd; ++d) {
+    const uint32_t bst = lds_base + F8StagesA * F8Stage + (d % kStagesB) * kOpStage;
+    // k-step 0 of chunk d (weights acur, tokens b0) while k-step 1's tokens are read
+    read_bfrags(bst + rbo1, b1);
+    mma8(acur, 0, b0, nb, acc);
+    lds_frags_ready();
+    tie(b1);
+    // k-step 1 while chunk d + 1's weights and k-step-0 tokens are read
+    const bool more = d + 1 < nd;
+    if (more) {
+      wait_loads(F8ALoads * (d + F8AheadA < nd));
+      __builtin_amdgcn_s_barrier();
+      if (d + 2 < nd) issue_b(d + 2);
+      if (d + 1 + F8AheadA < nd) issue_a(d + 1 + F8AheadA);
+      read_afrags8(lds_base + ((d + 1) % F8StagesA) * F8Stage + ra, anxt);
+      read_bfrags(lds_base + F8StagesA * F8Stage + ((d + 1) % kStagesB) * kOpStage + rbo0, b0);
+    }
+    mma8(acur, 1, b1, nb, acc);
+    if (more) {
+      lds_frags_ready();
+      tie(anxt);
+      tie(b0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acur[i] = anxt[i];
+    }
+  }
+
+  // ---- epilogue (k_prefill_gemm's), the row scales requested together first
+  const float* sc = op.scale ? op.scale + (long long)e * op.sstride : nullptr;
+  float scl[4][4];
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      int n;
+      if (MODE == kModeSwiglu)  // blocks 0-1 gate rows, 2-3 the matching up rows
+        n = rb * (PBN / 2) + wm * 32 + (a & 1) * 16 + 4 * kq + i + ((a >> 1) ? (int)op.s_up_off : 0);
+      else
+        n = min(rb * PBN + wm * 64 + a * 16 + 4 * kq + i, op.N - 1);
+      scl[a][i] = sc ? sc[n] : 1.f;
+    }
+#pragma unroll
+  for (int b = 0; b < 8; ++b) {
+    if (b >= nb) break;
+    const int rr = r0 + (2 * b + wn) * 16 + lr;
+    if (rr >= r1) continue;
+    const long long orow = op.out_map ? args.order[rr] : rr;
+    if (MODE == kModeSwiglu) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int n = rb * (PBN / 2) + wm * 32 + h * 16 + 4 * kq;
+        uint32_t o[2];
+#pragma unroll
+        for (int i = 0; i < 4; i += 2) {
+          const uint32_t g = pack_bf2_rne(acc[h][b][i] * scl[h][i], acc[h][b][i + 1] * scl[h][i + 1]);
+          const uint32_t u = pack_bf2_rne(acc[2 + h][b][i] * scl[2 + h][i],
+                                          acc[2 + h][b][i + 1] * scl[2 + h][i + 1]);
+          const uint32_t s = pack_bf2_rne(silu_fast(bf_lo(g)), silu_fast(bf_hi(g)));
+          o[i / 2] = pack_bf2_rne(bf_lo(s) * bf_lo(u), bf_hi(s) * bf_hi(u));
+        }
+        *reinterpret_cast<uint2*>(op.out + orow * op.ld_out + n) = make_uint2(o[0], o[1]);
+      }
+    } else {
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {
+        const int n = rb * PBN + wm * 64 + a * 16 + 4 * kq;
+        if (n >= op.N) break;
+        *reinterpret_cast<uint2*>(op.out + orow * op.ld_out + n) =
+            make_uint2(pack_bf2_rne(acc[a][b][0] * scl[a][0], acc[a][b][1] * scl[a][1]),
+                       pack_bf2_rne(acc[a][b][2] * scl[a][2], acc[a][b][3] * scl[a][3]));
+      }
+    }
+  }
+}
+
 int prefill_tile_rows() { return PBM; }
 
 bool prefill_fits(int mode, const GemmOperand& op) {
@@ -316,18 +581,18 @@ bool prefill_fits(int mode, const GemmOperand& op) {
 }
 
 namespace {
-// The kernel's dynamic LDS above the default limit, allowed once per device and mode.
-hipError_t allow_lds(const void* fn, int mode, int bytes) {
+// The kernels' dynamic LDS above the default limit, allowed once per device and kernel.
+hipError_t allow_lds(const void* fn, int which, int bytes) {
   static std::mutex mu;
-  static uint64_t done[2] = {0, 0};  // [mode], bit d: device d
+  static uint64_t done[4] = {};  // [kernel], bit d: device d
   int dev = 0;
   hipError_t err = hipGetDevice(&dev);
   if (err != hipSuccess) return err;
   if (dev < 0 || dev >= 64) return hipErrorInvalidDevice;
   std::lock_guard<std::mutex> lock(mu);
-  if (done[mode] >> dev & 1) return hipSuccess;
+  if (done[which] >> dev & 1) return hipSuccess;
   err = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  if (err == hipSuccess) done[mode] |= uint64_t(1) << dev;
+  if (err == hipSuccess) done[which] |= uint64_t(1) << dev;
   return err;
 }
 }  // namespace
@@ -350,13 +615,16 @@ hipError_t launch_prefill_gemm(int mode, const GemmArgs& a_in, int max_tiles, in
   const bool f8 = (has0 && a.op[0].fp8) || (has1 && a.op[1].fp8);
   if (max_tiles <= 0 || (!has0 && !has1)) return hipSuccess;
   a.bm = bm;
+  if (f8) {
+    // e4m3 weights are the routed experts' only
+    if (has1 || !a.table) return hipErrorInvalidValue;
+    if (prefill_stream_takes(a)) return launch_prefill_stream(mode, a, max_tiles, st);
+  }
   a.shared_first = 0;
   if (a.table && has0 && has1) {
     const char* env = knob(kKnobPrefillSharedFirst);
     if (!(env && env[0] == '0')) a.shared_first = (a.T + bm - 1) / bm;
   }
-  if (f8)
-    return launch_prefill_stream(mode, a, max_tiles, st);
   const int out_per_wg = mode == kModeSwiglu ? PBN / 2 : PBN;
   const int nmax = a.op[0].N > a.op[1].N ? a.op[0].N : a.op[1].N;
   a.nrb = (nmax + out_per_wg - 1) / out_per_wg;
@@ -364,16 +632,14 @@ hipError_t launch_prefill_gemm(int mode, const GemmArgs& a_in, int max_tiles, in
   a.MTgrid = max_tiles;
   const long long grid = (long long)((max_tiles + kXcds - 1) / kXcds) * kXcds * a.nrb;
   if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
-  const void* fn = mode == kModeSwiglu ? reinterpret_cast<const void*>(&k_prefill_gemm<kModeSwiglu>)
-                                       : reinterpret_cast<const void*>(&k_prefill_gemm<kModePlain>);
-  hipError_t err = allow_lds(fn, mode, kLdsBytes);
+  const int which = (f8 ? 2 : 0) + (mode == kModeSwiglu ? 1 : 0);
+  void (*const kernels[4])(GemmArgs) = {
+      k_prefill_gemm<kModePlain>, k_prefill_gemm<kModeSwiglu>, k_prefill_gemm_f8<kModePlain>,
+      k_prefill_gemm_f8<kModeSwiglu>};
+  const int bytes = f8 ? F8LdsBytes : kLdsBytes;
+  hipError_t err = allow_lds(reinterpret_cast<const void*>(kernels[which]), which, bytes);
   if (err != hipSuccess) return err;
-  if (mode == kModeSwiglu)
-    hipLaunchKernelGGL(k_prefill_gemm<kModeSwiglu>, dim3((unsigned)grid), dim3(kThreads),
-                       (size_t)kLdsBytes, st, a);
-  else
-    hipLaunchKernelGGL(k_prefill_gemm<kModePlain>, dim3((unsigned)grid), dim3(kThreads),
-                       (size_t)kLdsBytes, st, a);
+  hipLaunchKernelGGL(kernels[which], dim3((unsigned)grid), dim3(kThreads), (size_t)bytes, st, a);
   return hipGetLastError();
 }
 

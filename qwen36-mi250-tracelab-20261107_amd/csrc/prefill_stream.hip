@@ -150,27 +150,17 @@ __device__ __forceinline__ void wait_barrier() {
 // Keeps the loads before it ahead of those after it: the waits count them in issue order.
 __device__ __forceinline__ void issue_fence() { asm volatile("" ::: "memory"); }
 
-// 8 e4m3 bytes -> bf16x8 (exact)
-__device__ __forceinline__ u32x4v widen8(uint32_t lo, uint32_t hi) {
-  u32x4v r;
-  r.x = fp8x2_to_bf16x2<false>(lo);
-  r.y = fp8x2_to_bf16x2<true>(lo);
-  r.z = fp8x2_to_bf16x2<false>(hi);
-  r.w = fp8x2_to_bf16x2<true>(hi);
-  return r;
-}
-
 __device__ __forceinline__ u32x4v ld_weight(const char* p) {
   return __builtin_nontemporal_load(reinterpret_cast<const u32x4v*>(p));
 }
 
 // Stores a block's results: lane (kq, lr) holds rows 4 kq .. + 3 of token column lr of each
 // 16-token block.
-// WIDE: two token blocks at a time, exchanged between lane rows so that a lane holds 8
+// Two token blocks at a time, exchanged between lane rows so that a lane holds 8
 // consecutive results of one token (16-byte stores, half as many), always all of them: those
 // of rows past the tile or the weights go past the buffer's end, where they are dropped. The
 // weights of the next block are in flight meanwhile, and their waits count the stores.
-template <int MODE, bool FP8, int NB, int W, bool WIDE, class OutRow>
+template <int MODE, bool FP8, int NB, int W, class OutRow>
 __device__ __forceinline__ void prefill_epilogue(const GemmArgs& args, const GemmOperand& op,
                                                  bool routed, int e, int r0, int r1, int rb,
                                                  int wave, int lr, int kq,
@@ -204,56 +194,38 @@ __device__ __forceinline__ void prefill_epilogue(const GemmArgs& args, const Gem
       }
     }
   };
-  if constexpr (WIDE) {
-    const __amdgpu_buffer_rsrc_t obuf = __builtin_amdgcn_make_buffer_rsrc(
-        op.out, 0, args.out_bytes[routed ? 0 : 1], 0x00020000);
-    const uint32_t ld = (uint32_t)(op.ld_out * 2);
+  const __amdgpu_buffer_rsrc_t obuf = __builtin_amdgcn_make_buffer_rsrc(
+      op.out, 0, args.out_bytes[routed ? 0 : 1], 0x00020000);
+  const uint32_t ld = (uint32_t)(op.ld_out * 2);
 #pragma unroll
-    for (int b = 0; b < NB; b += 2) {
-      __builtin_amdgcn_sched_barrier(0);  // one pair's results live at a time
-      const int blk = b + (kq & 1);
-      const int row = out_row(blk, b);
-      const bool live = r0 + blk * 16 + lr < r1;
+  for (int b = 0; b < NB; b += 2) {
+    __builtin_amdgcn_sched_barrier(0);  // one pair's results live at a time
+    const int blk = b + (kq & 1);
+    const int row = out_row(blk, b);
+    const bool live = r0 + blk * 16 + lr < r1;
 #pragma unroll
-      for (int a = 0; a < kA; ++a) {
-        uint32_t p[2], q[2];
-        results(a, b, p);
-        results(a, b + 1, q);
-        u32x4v v;
+    for (int a = 0; a < kA; ++a) {
+      uint32_t p[2], q[2];
+      results(a, b, p);
+      results(a, b + 1, q);
+      u32x4v v;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          const auto x = __builtin_amdgcn_permlane16_swap(p[i], q[i], false, false);
-          v[i] = x[0];
-          v[i + 2] = x[1];
-        }
-        const int n = nw + a * 16 + (kq >> 1) * 8;
-        const uint32_t off = (uint32_t)row * ld + (uint32_t)n * 2;
-        __builtin_amdgcn_raw_buffer_store_b128(v, obuf, live && n < op.N ? off : 0xfffffff0u, 0,
-                                               kStorePolicy<MODE>);
+      for (int i = 0; i < 2; ++i) {
+        const auto x = __builtin_amdgcn_permlane16_swap(p[i], q[i], false, false);
+        v[i] = x[0];
+        v[i + 2] = x[1];
       }
-    }
-  } else {
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      __builtin_amdgcn_sched_barrier(0);
-      const int row = out_row(b, b);
-      if (r0 + b * 16 + lr >= r1) continue;
-      uint16_t* out = op.out + (long long)row * op.ld_out + n0;
-#pragma unroll
-      for (int a = 0; a < kA; ++a) {
-        if (n0 + a * 16 >= op.N) break;  // N is a multiple of 16: n < N covers n + 3
-        uint32_t o[2];
-        results(a, b, o);
-        *reinterpret_cast<uint2*>(out + a * 16) = make_uint2(o[0], o[1]);
-      }
+      const int n = nw + a * 16 + (kq >> 1) * 8;
+      const uint32_t off = (uint32_t)row * ld + (uint32_t)n * 2;
+      __builtin_amdgcn_raw_buffer_store_b128(v, obuf, live && n < op.N ? off : 0xfffffff0u, 0,
+                                             kStorePolicy<MODE>);
     }
   }
 }
 
 // One workgroup's product: weight rows of blocks rb0 .. rb0 + nblk - 1 (expert e) against sorted
 // rows [r0, r1), r1 - r0 <= 16 NB. R: chunks per phase and ring depth; K / 64 is a multiple of
-// R, at least 2 R (R = 1: any K, multiple of 32, one chunk at a time). RES: K = 128 R, both
-// phases stay in LDS for all blocks.
+// R, at least 2 R. RES: K = 128 R, both phases stay in LDS for all blocks.
 template <int MODE, bool FP8, int NB, int W, int R, bool RES>
 __device__ __forceinline__ void prefill_body(const GemmArgs& args, const GemmOperand& op,
                                              bool routed, int e, int r0, int r1, int rb0, int nblk,
@@ -383,108 +355,73 @@ __device__ __forceinline__ void prefill_body(const GemmArgs& args, const GemmOpe
     }
   };
   auto epilogue = [&](int rb) __attribute__((always_inline)) {
-    prefill_epilogue<MODE, FP8, NB, W, (R > 1)>(args, op, routed, e, r0, r1, rb, wave, lr, kq,
+    prefill_epilogue<MODE, FP8, NB, W>(args, op, routed, e, r0, r1, rb, wave, lr, kq,
                                                 out_row, acc);
   };
 
   weight_rows(rb0);
   clear();
-  if constexpr (R > 1) {
-    const int nph = nch / R;
-    const int rot = routed ? prefill_start_chunk(e, nch) / R : 0;  // whole phases: R divides 4
-    auto phase_of = [&](int p) __attribute__((always_inline)) {  // p < nph
-      p += rot;
-      return p >= nph ? p - nph : p;
-    };
-    const int ph0 = phase_of(0);
-    issue_a(0, ph0 * R);
+  const int nph = nch / R;
+  const int rot = routed ? prefill_start_chunk(e, nch) / R : 0;  // whole phases: R divides 4
+  auto phase_of = [&](int p) __attribute__((always_inline)) {  // p < nph
+    p += rot;
+    return p >= nph ? p - nph : p;
+  };
+  const int ph0 = phase_of(0);
+  issue_a(0, ph0 * R);
 #pragma unroll
-    for (int i = 0; i < kLB; ++i)
-      toff[i] = (uint32_t)((trow[i] - row_base) / row_div) * (uint32_t)(op.ld_in * 2) +
-                (uint32_t)(unit * 16);
-    issue_b(0, ph0, true);
+  for (int i = 0; i < kLB; ++i)
+    toff[i] = (uint32_t)((trow[i] - row_base) / row_div) * (uint32_t)(op.ld_in * 2) +
+              (uint32_t)(unit * 16);
+  issue_b(0, ph0, true);
 #pragma unroll
-    for (int c = 1; c < R; ++c) issue_a(c, ph0 * R + c);
-    if constexpr (RES) {
-      issue_b(1, phase_of(1), true);
-      wait_barrier<(R - 1) * kLA + kLB>();
-    } else {
-      wait_barrier<(R - 1) * kLA>();
-    }
-    // A phase multiplies the R chunks at LDS offset `at` and requests the next phase's
-    // operands, so that the counts are the same in every phase; the walk's last phase requests
-    // nothing from the buffer and one line of the weights. At its end the next phase's token
-    // rows have landed (younger: this phase's weight requests) and every wave is past this one.
-    auto phase = [&](int at, int stage, int next, bool more, bool sync) __attribute__((always_inline)) {
-      if constexpr (!RES) issue_b(stage, next, more);
-#pragma unroll
-      for (int q = 0; q < R; ++q) {
-        mma(q, at + q * kSub, 2);
-        issue_a(q, next * R + q);
-      }
-      if (sync) wait_barrier<R * kLA>();
-    };
-    // Phase f of the walk: token stage f & 1 (RES: the two stages hold all of K, requested
-    // once). A block's first phase follows the stores of the block before it, whose number is
-    // a constant: hence the code of its own (the first block's is before the loop).
-    int f = 0;
-    phase(0, 1, phase_of(1), true, true);
-    for (int rb = rb0;;) {
-      for (int p = 1; p + 1 < nph; ++p) {
-        ++f;
-        phase((f & 1) * kStage, (f + 1) & 1, phase_of(p + 1), true, !RES);
-      }
-      const bool more = rb + 1 < rb0 + nblk;
-      weight_rows(more ? rb + 1 : -1);
-      ++f;
-      phase((RES ? 1 : f & 1) * kStage, (f + 1) & 1, ph0, more, !RES);
-      epilogue(rb);
-      if (!more) break;
-      ++rb;
-      clear();
-      ++f;
-      phase((RES ? 0 : f & 1) * kStage, (f + 1) & 1, phase_of(1), true, !RES);
-    }
+  for (int c = 1; c < R; ++c) issue_a(c, ph0 * R + c);
+  if constexpr (RES) {
+    issue_b(1, phase_of(1), true);
+    wait_barrier<(R - 1) * kLA + kLB>();
   } else {
-    // K of any multiple of 32: one chunk at a time; a last half chunk reads its first half
-    // twice instead of running past the rows
-    const char* tsrc[kLB];
+    wait_barrier<(R - 1) * kLA>();
+  }
+  // A phase multiplies the R chunks at LDS offset `at` and requests the next phase's
+  // operands, so that the counts are the same in every phase; the walk's last phase requests
+  // nothing from the buffer and one line of the weights. At its end the next phase's token
+  // rows have landed (younger: this phase's weight requests) and every wave is past this one.
+  auto phase = [&](int at, int stage, int next, bool more, bool sync) __attribute__((always_inline)) {
+    if constexpr (!RES) issue_b(stage, next, more);
 #pragma unroll
-    for (int i = 0; i < kLB; ++i) {
-      const long long src = (trow[i] - row_base) / row_div;
-      tsrc[i] = reinterpret_cast<const char*>(op.in + src * op.ld_in) + unit * 16;
+    for (int q = 0; q < R; ++q) {
+      mma(q, at + q * kSub, 2);
+      issue_a(q, next * R + q);
     }
-    const int all = (op.K + kPKC - 1) / kPKC;
-    const int rot = routed && op.K % kPKC == 0 ? prefill_start_chunk(e, all) : 0;
-    for (int j = 0; j < nblk; ++j) {
-      weight_rows(rb0 + j);
-      clear();
-      for (int c = 0; c < all; ++c) {
-        const int k0 = (c + rot < all ? c + rot : c + rot - all) * kPKC;
-        const bool half = op.K - k0 < kPKC;
-        wait_barrier<0>();  // every wave is past the previous chunk's stage
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-          for (int s = 0; s < kLS; ++s)
-            ring[0][a][s] =
-                ld_weight((a ? wbase1 : wbase) + k0 * kEB + (half ? 0 : s * 64) + woff[a]);
-#pragma unroll
-        for (int i = 0; i < kLB; ++i)
-          dma16(tsrc[i] + (long long)k0 * 2 - (half && unit >= 4 ? 64 : 0),
-                lds + (wave + W * i) * 1024);
-        wait_barrier<0>();
-        mma(0, 0, half ? 1 : 2);
-      }
-      epilogue(rb0 + j);
+    if (sync) wait_barrier<R * kLA>();
+  };
+  // Phase f of the walk: token stage f & 1 (RES: the two stages hold all of K, requested
+  // once). A block's first phase follows the stores of the block before it, whose number is
+  // a constant: hence the code of its own (the first block's is before the loop).
+  int f = 0;
+  phase(0, 1, phase_of(1), true, true);
+  for (int rb = rb0;;) {
+    for (int p = 1; p + 1 < nph; ++p) {
+      ++f;
+      phase((f & 1) * kStage, (f + 1) & 1, phase_of(p + 1), true, !RES);
     }
+    const bool more = rb + 1 < rb0 + nblk;
+    weight_rows(more ? rb + 1 : -1);
+    ++f;
+    phase((RES ? 1 : f & 1) * kStage, (f + 1) & 1, ph0, more, !RES);
+    epilogue(rb);
+    if (!more) break;
+    ++rb;
+    clear();
+    ++f;
+    phase((RES ? 0 : f & 1) * kStage, (f + 1) & 1, phase_of(1), true, !RES);
   }
 }
 
 template <int MODE, bool FP8, int MAXB, int W, int R, bool RES>
 __global__ __launch_bounds__(64 * W)
 __attribute__((amdgpu_waves_per_eu(MAXB <= 4 ? 3 : 2))) void k_prefill_stream(GemmArgs args) {
-  extern __shared__ uint4 smem[];  // two phases (R = 1: one) of up to MAXB 16-token blocks
+  extern __shared__ uint4 smem[];  // two phases of up to MAXB 16-token blocks
 
   // XCD-aware order: workgroup b runs on XCD b % 8, so the workgroups of one tile get ids 8
   // apart (same XCD, dispatched together) and share the tile's token rows in that XCD's L2
@@ -564,7 +501,7 @@ hipError_t allow_lds(const void* fn, int which, int bytes) {
 
 template <int MODE, bool FP8, int MAXB, int W, int R, bool RES = false>
 hipError_t launch_one(GemmArgs a, int tiles, hipStream_t st) {
-  constexpr int bytes = (R > 1 ? 2 * R : 1) * MAXB * kPBlkBytes;
+  constexpr int bytes = 2 * R * MAXB * kPBlkBytes;
   constexpr int kOut = MODE == kModeSwiglu ? 16 * W : 32 * W;
   const int nmax = a.op[0].N > a.op[1].N ? a.op[0].N : a.op[1].N;
   a.nrb = (nmax + kOut - 1) / kOut;
@@ -585,20 +522,8 @@ hipError_t launch_one(GemmArgs a, int tiles, hipStream_t st) {
   return hipGetLastError();
 }
 
-// The ring an operand's shape allows: phases of 4 or 2 chunks, at least two per block, 32-bit
-// offsets into its tensors; 1: the one-chunk form, which takes any shape.
-int ring_of(const GemmArgs& a, int i) {
-  const GemmOperand& o = a.op[i];
-  const long long in = (i == 0 && !o.in_map ? (long long)a.P : a.T) * o.ld_in * 2;
-  const long long out = (i == 0 ? (long long)a.P : a.T) * o.ld_out * 2;
-  if (in > 0xffffff00LL || out > 0xffffff00LL || (long long)o.N * o.ldw * 2 > 0x7fffffffLL) return 1;
-  if (o.K % (2 * kPKC) || o.K < 4 * kPKC) return 1;
-  return o.K % (4 * kPKC) || o.K < 8 * kPKC ? 2 : 4;
-}
-
 hipError_t launch_gate_up(const GemmArgs& a, int ring, int tiles, hipStream_t st) {
   constexpr int L = kPBlocksLarge, M = kModeSwiglu;
-  if (ring == 1) return launch_one<M, true, L, 4, 1>(a, tiles, st);
   if (ring == 2) return launch_one<M, true, L, 8, 2>(a, tiles, st);
   return launch_one<M, true, L, 8, 4>(a, tiles, st);
 }
@@ -606,34 +531,42 @@ hipError_t launch_gate_up(const GemmArgs& a, int ring, int tiles, hipStream_t st
 // res: two phases hold all of K.
 hipError_t launch_down(const GemmArgs& a, int ring, bool res, int tiles, hipStream_t st) {
   constexpr int L = kPBlocksLarge, M = kModePlain;
-  if (ring == 1) return launch_one<M, true, L, 4, 1>(a, tiles, st);
   if (ring == 2) return launch_one<M, true, L, 8, 2>(a, tiles, st);
   if (res) return launch_one<M, true, L, 8, 4, true>(a, tiles, st);
   return launch_one<M, true, L, 8, 4>(a, tiles, st);
 }
 
+long long in_bytes(const GemmArgs& a) { return (a.op[0].in_map ? a.T : a.P) * a.op[0].ld_in * 2; }
+long long out_bytes(const GemmArgs& a) { return a.P * a.op[0].ld_out * 2; }
+
 }  // namespace
+
+// K in whole phases, at least two per block; 32-bit offsets into the tensors; and few enough rows.
+// For other K (64, 128 and odd multiples of 64) and tensors past 4 GiB (down's from 131072 tokens
+// of the model) a form of this kernel with one chunk in flight measured slower than the staged
+// kernel: down at 777 tokens, K = 320 / 576, 85 / 138 against 75 / 103 µs; gate_up at 4096 tokens,
+// K = 128, 45 against 42; the experts at 140000 tokens 12.8 against 9.6 ms.
+bool prefill_stream_takes(const GemmArgs& a) {
+  const GemmOperand& o = a.op[0];
+  if (o.K % (2 * kPKC) || o.K < 4 * kPKC) return false;
+  if (in_bytes(a) > 0xffffff00LL || out_bytes(a) > 0xffffff00LL ||
+      (long long)o.N * o.ldw * 2 > 0x7fffffffLL)
+    return false;
+  return a.P <= (long long)kStreamRowsPerExpert * a.E;
+}
 
 hipError_t launch_prefill_stream(int mode, const GemmArgs& a_in, int max_tiles, hipStream_t st) {
   GemmArgs a = a_in;
   constexpr int sub = kStreamRowsLarge;
-  a.nsub = a.table ? (a.bm + sub - 1) / sub : 1;
+  a.nsub = (a.bm + sub - 1) / sub;
   a.MTgrid = max_tiles;
-  const int tiles = a.table ? max_tiles * a.nsub : (a.T + sub - 1) / sub;
-  int ring = 4;
-  bool res = true;
-  for (int i = 0; i < 2; ++i) {
-    const GemmOperand& o = a.op[i];
-    if (o.N <= 0) continue;
-    const int r = ring_of(a, i);
-    ring = r < ring ? r : ring;
-    res = res && o.K == 8 * kPKC;
-    if (r == 1) continue;
-    a.in_bytes[i] = (unsigned)((i == 0 && !o.in_map ? (long long)a.P : a.T) * o.ld_in * 2);
-    a.out_bytes[i] = (unsigned)((i == 0 ? (long long)a.P : a.T) * o.ld_out * 2);
-  }
+  const int tiles = max_tiles * a.nsub;
+  const int K = a.op[0].K;
+  const int ring = K % (4 * kPKC) || K < 8 * kPKC ? 2 : 4;
+  a.in_bytes[0] = (unsigned)in_bytes(a);
+  a.out_bytes[0] = (unsigned)out_bytes(a);
   return mode == kModeSwiglu ? launch_gate_up(a, ring, tiles, st)
-                             : launch_down(a, ring, res, tiles, st);
+                             : launch_down(a, ring, K == 8 * kPKC, tiles, st);
 }
 
 }  // namespace moe

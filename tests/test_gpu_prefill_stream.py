@@ -1,7 +1,8 @@
-"""The prefill kernels (streaming e4m3, staged bf16) at the
-edges of its tiles: every 16-token block count it is compiled for with the rows one below, at
-and one above a block boundary, parts of a larger table tile, each ring depth (K of 64, 128,
-192, 256, 384, 512, 768 and 1024) and experts without rows.
+"""The prefill kernels (e4m3 streaming, e4m3 and bf16 staged through LDS) at the edges of their
+tiles: every 16-token block count they are compiled for with the rows one below, at and one
+above a block boundary, parts of a larger table tile, each ring depth of the streaming kernel (K
+of 256, 384, 512, 768 and 1024), the K that the staged e4m3 kernel takes instead (64, 128, 192) and
+experts without rows; above 128 rows per expert on average the staged e4m3 kernel alone.
 
 Tolerance: the results are bf16 roundings of fp32 sums of K bf16 products; the reference sums
 in float64 and rounds at the same points, so a rounded value differs by one bf16 ulp (at most
@@ -61,11 +62,20 @@ SMALL = [0, 1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 1, 130]
 LARGE = [0, 79, 80, 81, 95, 96, 97, 127, 128, 129, 159, 160, 161, 3, 320, 63]
 
 
-@pytest.mark.parametrize("counts,bm", [(SMALL, 256), (LARGE, 256), (SMALL, None), (LARGE, None)])
-@pytest.mark.parametrize("H,I,fp8", [(256, 128, True), (256, 384, True), (768, 128, True),
-                                     (1024, 256, True), (512, 512, True), (512, 128, False),
-                                     (768, 256, False), (256, 128, False)])
-def test_prefill_stream_tiles(pkg, counts, bm, H, I, fp8):
+# more than 128 rows per expert on average: edges of whole 256-row tiles and of the last one
+MANY = [0, 255, 256, 257, 511, 512, 513, 1, 272, 290]
+
+
+SHAPES = [(256, 128, True), (256, 384, True), (768, 128, True), (1024, 256, True), (512, 512, True),
+          (512, 128, False), (768, 256, False), (256, 128, False)]
+# hidden sizes that the whole call takes on 64-row tiles
+GROUPED_ONLY = [(64, 128, True), (192, 128, True)]
+
+
+@pytest.mark.parametrize("H,I,fp8,counts,bm", [
+    (*shape, counts, bm) for bm in (256, None) for shape in SHAPES + (GROUPED_ONLY if bm else [])
+    for counts in (SMALL, LARGE, MANY)])
+def test_prefill_stream_tiles(pkg, H, I, fp8, counts, bm):
     """bm None: the whole routed-experts call with its own tile size (more than 512 tokens);
     256: the grouped operations on a table of 256-row tiles."""
     print(f"prefill stream H={H} I={I} fp8={fp8} rows<= {max(counts)} bm={bm}", flush=True)
@@ -106,19 +116,19 @@ def test_prefill_stream_tiles(pkg, counts, bm, H, I, fp8):
     _close(got_y, _bf(y), 2.0**-7)
 
 
-@pytest.mark.parametrize("fp8", [False, True])
-def test_prefill_stream_silu_range(pkg, fp8):
+@pytest.mark.parametrize("fp8,rows", [(False, 20), (True, 20), (True, 129)])
+def test_prefill_stream_silu_range(pkg, fp8, rows):
     """gate_up's SiLU over its whole range: one gate value per expert (e4m3: by the row's scale),
     up = 1, a down row that passes act[0] through. Against float64 within one bf16 ulp (2^-7 of
     the value); below x = -88.7, where exp(-x) is past float32, the value is under 3e-37 and may
     come out as 0; infinities and NaN as torch's."""
-    print(f"silu range fp8={fp8}", flush=True)
+    print(f"silu range fp8={fp8} rows={rows}", flush=True)
     dev = torch.device("cuda")
     inf = float("inf")
     vals = [0.0, 1e-30, -1e-30, 0.5, -0.5, 1.0, -1.0, 3.0, -3.0, 7.5, -7.5, 20.0, -20.0, 44.25, -44.5,
             60.0, -60.0, -80.0, -86.0, -87.0, 87.5, -87.5, -88.0, 88.5, -88.5, 89.0, -89.0, -95.0,
             300.0, -300.0, 1e8, -1e8, 1e20, -1e20, 3e38, inf, -inf, float("nan")]
-    E, T, H, I = len(vals), 20 * len(vals), 256, 128
+    E, T, H, I = len(vals), rows * len(vals), 256, 128
     v = torch.tensor(vals, dtype=torch.float64).to(BF16)
     gu = torch.zeros(E, 2 * I, H, dtype=BF16)
     gu[:, 0, 0] = 1.0 if fp8 else v
@@ -133,7 +143,7 @@ def test_prefill_stream_silu_range(pkg, fp8):
         scales = dict(gate_up_scale=gus.to(dev), down_scale=torch.ones(E, H, device=dev))
     x = torch.zeros(T, H, dtype=BF16)
     x[:, 0] = 1.0
-    idx = _routing([20] * E, 1)
+    idx = _routing([rows] * E, 1)
     out = pkg.ops.moe_prefill(x.to(dev), idx.to(dev), torch.ones(T, 1, dtype=BF16, device=dev),
                               gu.to(dev), dn.to(dev), **scales)
     torch.cuda.synchronize()

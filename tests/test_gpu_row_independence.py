@@ -57,3 +57,32 @@ def test_leading_rows_match_smaller_batch(pkg, dev, mlp, big, small, decode):
     # fp32 summation order: across that boundary only the routing is compared
     if (big > 512) == (small > 512):
         assert torch.equal(a[:small], b)
+
+
+@pytest.mark.parametrize("big,small", [(1024, 600), (1100, 900), (4096, 2048), (6000, 4096),
+                                       (8192, 5000), (132000, 4096)])
+def test_leading_rows_match_smaller_batch_fp8_prefill(pkg, dev, big, small):
+    """The e4m3 prefill kernels: a row's bits do not depend on the batch either where its rows
+    fall into another part or block count of a tile, where the batch takes the other kernel (above
+    128 rows per expert on average: 4096 tokens), or where the outputs of the experts are past
+    4 GiB (131072 tokens)."""
+    print(f"fp8 row independence {big} -> {small}", flush=True)
+    E, H, I, k = 256, 2048, 512, 8
+    g = torch.Generator(device=dev).manual_seed(big + small)
+
+    def weight(*shape):
+        return (torch.randn(*shape, generator=g, device=dev) * 100).clamp(-448, 448).to(
+            torch.float8_e4m3fn)
+
+    gu, dn = weight(E, 2 * I, H), weight(E, H, I)
+    scales = dict(gate_up_scale=torch.rand(E, 2 * I, generator=g, device=dev) * 4e-4,
+                  down_scale=torch.rand(E, H, generator=g, device=dev) * 4e-4)
+    x = torch.randn(big, H, generator=g, device=dev).to(BF16)
+    idx = torch.rand(big, E, generator=g, device=dev).topk(k, dim=1).indices
+    w = torch.full((big, k), 0.125, dtype=BF16, device=dev)
+    a = pkg.ops.moe_prefill(x, idx, w, gu, dn, **scales)[:small].clone()
+    b = pkg.ops.moe_prefill(x[:small].contiguous(), idx[:small].contiguous(),
+                            w[:small].contiguous(), gu, dn, **scales)
+    torch.cuda.synchronize()
+    assert torch.isfinite(a).all() and a.float().abs().mean() > 1e-3
+    assert torch.equal(a, b)
