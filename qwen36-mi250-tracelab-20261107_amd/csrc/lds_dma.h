@@ -65,6 +65,10 @@ __device__ __forceinline__ void wait_loads(int n) {
 __device__ __forceinline__ void dma16(const void* g, void* lds) {
   __builtin_amdgcn_global_load_lds(g, lds, 16, 0, 0);
 }
+// The same with the non-temporal cache policy.
+__device__ __forceinline__ void dma16_nt(const void* g, void* lds) {
+  __builtin_amdgcn_global_load_lds(g, lds, 16, 0, 2);
+}
 
 // The same in buffer form: 16 bytes at byte offset voff (per lane) + soff (wave-uniform) of
 // the buffer. Loads past the buffer's end give zeros.

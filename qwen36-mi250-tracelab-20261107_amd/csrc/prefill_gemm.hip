@@ -49,11 +49,6 @@ constexpr int kStagesB = 2, kAheadB = 1;          // token-row ring: chunk d + 2
 constexpr int kLdsBytes = (kStagesA + kStagesB) * kOpStage;  // 160 KiB
 constexpr int kThreads = 512;
 constexpr int kXcds = 8;                          // XCDs of an MI355X (round-robin dispatch)
-// Weight rows are read once per tile: their DMA loads are non-temporal (cache policy NT), so
-// they do not displace the token rows the tile's other workgroups read again, or the pair
-// outputs the combine reads next (C4 530 against 547 µs per layer; the token rows loaded
-// non-temporal as well measured 552).
-constexpr int kWeightCachePolicy = 2;
 constexpr int kGroups = 256 / 8;                  // 8-row DMA groups per operand and chunk
 constexpr int kLoadsPerWave = kGroups / (kThreads / 64);  // per operand and chunk: 4
 static_assert(kLoadsPerWave == 4, "wait_loads counts 4 loads per operand per chunk");
@@ -101,7 +96,9 @@ __device__ __forceinline__ void mma_frags(const Frags& f, int nb, f32x4_t (&acc)
   }
 }
 
-template <int MODE>
+// TAIL: an operand's K may be an odd multiple of 32 (a form of its own: the others' loop carries
+// no tests for it).
+template <int MODE, bool TAIL>
 __global__ __launch_bounds__(kThreads, 1) void k_prefill_gemm(GemmArgs args) {
   extern __shared__ uint4 smem[];  // A ring [kStagesA][16][1 KiB], B ring [kStagesB][16][1 KiB]
 
@@ -183,17 +180,21 @@ __global__ __launch_bounds__(kThreads, 1) void k_prefill_gemm(GemmArgs args) {
   }
   char* lds = reinterpret_cast<char*>(smem);
   char* bring_lds = lds + kStagesA * kOpStage;
-  const int nd = op.K / DKC;
-  // gate_up's K order is the streaming kernel's (down runs here alone)
-  const int rot = MODE == kModeSwiglu && routed ? prefill_start_chunk(e, nd) : 0;
+  // a last half chunk holds its 32 k twice (so that no load runs past a row) and is multiplied once
+  const bool half = TAIL && op.K % DKC != 0;
+  const int nd = TAIL ? (op.K + DKC - 1) / DKC : op.K / DKC;
+  const int rot = MODE == kModeSwiglu && routed && !half ? prefill_start_chunk(e, nd) : 0;
   auto chunk = [&](int d) { return d + rot < nd ? d + rot : d + rot - nd; };
+  auto koff = [&](int d) { return d * DKC - (half && d == nd - 1 && unit >= 4 ? PKC : 0); };
   auto issue_a = [&](int d) {
     char* st = lds + (d % kStagesA) * kOpStage;
     d = chunk(d);
+    // Weight rows are read once per tile: non-temporal, they do not displace the token rows the
+    // tile's other workgroups read again, or the pair outputs the combine reads next (C4 530
+    // against 547 µs per layer; the token rows loaded non-temporal as well measured 552)
 #pragma unroll
     for (int i = 0; i < kLoadsPerWave; ++i)
-      __builtin_amdgcn_global_load_lds(srca[i] + d * DKC, st + (wave + 8 * i) * 1024, 16, 0,
-                                       kWeightCachePolicy);
+      dma16_nt(srca[i] + koff(d), st + (wave + 8 * i) * 1024);
   };
   // token-row groups past the tile's tokens are not loaded (their LDS rows keep stale data,
   // which only reaches MFMA output columns that are never stored): nb_loads of the wave's 4
@@ -204,8 +205,7 @@ __global__ __launch_bounds__(kThreads, 1) void k_prefill_gemm(GemmArgs args) {
     d = chunk(d);
 #pragma unroll
     for (int i = 0; i < kLoadsPerWave; ++i)
-      if (i < nb_loads)
-        __builtin_amdgcn_global_load_lds(srcb[i] + d * DKC, st + (wave + 8 * i) * 1024, 16, 0, 0);
+      if (i < nb_loads) dma16(srcb[i] + koff(d), st + (wave + 8 * i) * 1024);
   };
   // fragment read offsets of this lane (row lr of a 16-row block, logical unit s * 4 + kq)
   typedef __attribute__((address_space(3))) char lds_char;
@@ -228,9 +228,9 @@ __global__ __launch_bounds__(kThreads, 1) void k_prefill_gemm(GemmArgs args) {
   // rows are requested three chunks before use, token rows two. The prologue issues A(0),
   // B(0), A(1), B(1), A(2) — the order the steps would have — so the loads younger than a
   // chunk's B load are exactly the next A load.
-  const int nk = 2 * nd;
+  const int nk = 2 * nd - (half ? 1 : 0);
   issue_a(0);
-  if (nd > 0) issue_b(0);
+  issue_b(0);
   if (nd > 1) issue_a(1);
   if (nd > 1) issue_b(1);
   if (nd > 2) issue_a(2);
@@ -260,6 +260,7 @@ __global__ __launch_bounds__(kThreads, 1) void k_prefill_gemm(GemmArgs args) {
   };
   for (int j = 0; j < nk; j += 2) {
     step(j, f0, f1);
+    if (TAIL && j + 1 >= nk) break;
     step(j + 1, f1, f0);
   }
 
@@ -575,7 +576,7 @@ int prefill_tile_rows() { return PBM; }
 bool prefill_fits(int mode, const GemmOperand& op) {
   if (op.N <= 0) return true;
   // SWIGLU: whole 128-row gate/up blocks; PLAIN: any multiple of 16 rows (the last block of
-  // 256 may be partial); K in whole chunks of the fp8 kernel
+  // 256 may be partial); K in whole k-steps, e4m3 in whole chunks
   const bool rows_ok = mode == kModeSwiglu ? op.N % (PBN / 2) == 0 : op.N % 16 == 0;
   return rows_ok && (op.fp8 ? op.K % DKC == 0 : op.K % PKC == 0);
 }
@@ -584,7 +585,7 @@ namespace {
 // The kernels' dynamic LDS above the default limit, allowed once per device and kernel.
 hipError_t allow_lds(const void* fn, int which, int bytes) {
   static std::mutex mu;
-  static uint64_t done[4] = {};  // [kernel], bit d: device d
+  static uint64_t done[6] = {};  // [kernel], bit d: device d
   int dev = 0;
   hipError_t err = hipGetDevice(&dev);
   if (err != hipSuccess) return err;
@@ -632,10 +633,12 @@ hipError_t launch_prefill_gemm(int mode, const GemmArgs& a_in, int max_tiles, in
   a.MTgrid = max_tiles;
   const long long grid = (long long)((max_tiles + kXcds - 1) / kXcds) * kXcds * a.nrb;
   if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
-  const int which = (f8 ? 2 : 0) + (mode == kModeSwiglu ? 1 : 0);
-  void (*const kernels[4])(GemmArgs) = {
-      k_prefill_gemm<kModePlain>, k_prefill_gemm<kModeSwiglu>, k_prefill_gemm_f8<kModePlain>,
-      k_prefill_gemm_f8<kModeSwiglu>};
+  const bool tail = (has0 && a.op[0].K % DKC) || (has1 && a.op[1].K % DKC);
+  const int which = (f8 ? 4 : tail ? 2 : 0) + (mode == kModeSwiglu ? 1 : 0);
+  void (*const kernels[6])(GemmArgs) = {
+      k_prefill_gemm<kModePlain, false>, k_prefill_gemm<kModeSwiglu, false>,
+      k_prefill_gemm<kModePlain, true>,  k_prefill_gemm<kModeSwiglu, true>,
+      k_prefill_gemm_f8<kModePlain>,     k_prefill_gemm_f8<kModeSwiglu>};
   const int bytes = f8 ? F8LdsBytes : kLdsBytes;
   hipError_t err = allow_lds(reinterpret_cast<const void*>(kernels[which]), which, bytes);
   if (err != hipSuccess) return err;

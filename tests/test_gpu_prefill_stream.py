@@ -116,6 +116,48 @@ def test_prefill_stream_tiles(pkg, H, I, fp8, counts, bm):
     _close(got_y, _bf(y), 2.0**-7)
 
 
+@pytest.mark.parametrize("K", [32, 96, 160, 224])
+def test_prefill_bf16_half_chunk(pkg, K):
+    """bf16 rows of an odd multiple of 32 on 256-row tiles, with a shared expert of the same and of
+    another length in the launch: K is walked in chunks of 64, whose last one is a half."""
+    print(f"prefill half chunk K={K}", flush=True)
+    dev = torch.device("cuda")
+    counts, N, IS = [0, 1, 17, 255, 256, 257, 300], 128, 128
+    E, T = len(counts), sum(counts)
+    g = torch.Generator().manual_seed(K)
+
+    def rnd(*shape):
+        return (torch.randn(*shape, generator=g) * 0.25).to(BF16)
+
+    def act(x, gate, up):
+        gt, u = _bf(x @ gate.double().T), _bf(x @ up.double().T)
+        return _bf(_bf(gt * torch.sigmoid(gt)) * u)
+
+    idx = _routing(counts, 1)
+    sp = pkg.ops.sort_pairs(idx.to(dev), E, bm=256, shared=True)
+    order = sp.order.long().cpu()
+    expert = idx[order, 0]
+    # gate_up: hidden K
+    x, gu, sg, su = rnd(T, K), rnd(E, 2 * N, K), rnd(IS, K), rnd(IS, K)
+    ref = torch.cat([act(x[order][expert == e].double(), gu[e, :N], gu[e, N:]) for e in range(E)])
+    got, got_sh = pkg.ops.grouped_gate_up(x.to(dev), 1, gu.to(dev), sp,
+                                          shared=(sg.to(dev), su.to(dev)))
+    torch.cuda.synchronize()
+    _close(got, ref, 11 * 2.0**-7)
+    _close(got_sh, act(x.double(), sg, su), 11 * 2.0**-7)
+    # down: intermediate K, the shared expert's K and 128
+    for Ks in (K, 128):
+        a, dn, sd, ash = rnd(T, K), rnd(E, N, K), rnd(N, Ks), rnd(T, Ks)
+        y = torch.empty(T, N, dtype=torch.float64)
+        for e in range(E):
+            y[order[expert == e]] = a[expert == e].double() @ dn[e].double().T
+        got, got_sh = pkg.ops.grouped_down(a.to(dev), T, 1, dn.to(dev), sp,
+                                           shared=(sd.to(dev), ash.to(dev)))
+        torch.cuda.synchronize()
+        _close(got, _bf(y), 2.0**-7)
+        _close(got_sh, _bf(ash.double() @ sd.double().T), 2.0**-7)
+
+
 @pytest.mark.parametrize("fp8,rows", [(False, 20), (True, 20), (True, 129)])
 def test_prefill_stream_silu_range(pkg, fp8, rows):
     """gate_up's SiLU over its whole range: one gate value per expert (e4m3: by the row's scale),
