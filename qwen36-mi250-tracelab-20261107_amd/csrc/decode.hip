@@ -7,10 +7,9 @@
 // every weight byte is used by at most four tokens and the block is bound by HBM latency
 // and bandwidth rather than by any arithmetic:
 //
-//   K1 k_dec_router   one wave per router row (logits[t, n] = bf16(x_t . Wpack[n])) and one
-//                     wave per shared-expert gate/up row pair (act_sh = SwiGLU). The shared
-//                     expert does not depend on the routing, so its 4 MiB stream overlaps the
-//                     router's HBM round trip instead of following it. Optionally it
+//   K1 k_dec_router   one wave per router row and token (logits[t, n] = bf16(x_t . Wpack[n]));
+//                     the stand-alone operation may add the shared expert's gate/up row pairs
+//                     (act_sh = SwiGLU), which the block gives to K2. Optionally it
 //                     first computes the layer's post-attention add + RMSNorm of the token
 //                     rows itself (every wave already reads whole rows), which removes that
 //                     launch from a decode layer.
@@ -20,9 +19,10 @@
 //                     four gate/up row pairs of it, and writes act[pair, n]. For one token
 //                     the weight rows are requested as soon as the selection has reached the
 //                     workgroup's expert, and the rest of the routing overlaps them.
-//   K3 k_dec_down     one wave per hidden row n: y_p = bf16(act_p . Wd[e_p, n]) for every
-//                     pair, the shared expert's row, and the combine of those values in the
-//                     routing order j, gated shared term and residual, written straight to out.
+//   K3 k_dec_down     four hidden rows n per workgroup, its waves over the pairs: y_p =
+//                     bf16(act_p . Wd[e_p, n]) for every pair, the shared expert's rows, and the
+//                     combine of those values in the routing order j, gated shared term and
+//                     residual, written straight to out (k_dec_down1: one token, a wave per pair).
 //
 // Every projection is a dot product over a whole weight row: lane l holds elements
 // [512 c + 8 l, 512 c + 8 l + 8) of chunk c, so one load instruction reads 1 KiB (bf16) or
@@ -58,8 +58,8 @@ __device__ __forceinline__ float dot8(uint4 w, uint4 x, float acc) {
 
 // The same product with gfx950's two-term bf16 dot product: four instructions instead of
 // sixteen unpacks and eight fmas, in the kernels that the VALU bounds at several tokens. Its
-// error against float64 over random rows is that of the fma chain (3.4e-8 against 3.6e-8
-// relative over 32 terms).
+// error against float64 is not above the fma chain's (root mean square of a row's error over
+// sum |x w|, rows of 1024: 7.6e-10 against 7.8e-10), and subnormal operands and sums count.
 __device__ __forceinline__ float dot8_pairs(uint4 w, uint4 x, float acc) {
   const uint32_t *a = &w.x, *b = &x.x;
 #pragma unroll
@@ -713,7 +713,7 @@ int gate_up_blocks() {
   return v == 1 || v == 2 ? v : 4;
 }
 
-// MOE_DECODE_DOWN=rows: the wave-per-row down kernel for one token too (comparisons).
+// MOE_DECODE_DOWN=rows: the several-token down kernel for one token too (comparisons).
 bool down_legacy() {
   const char* env = knob(kKnobDecodeDown);
   return env && env[0] == 'r';

@@ -176,8 +176,8 @@ def test_decode_stages_compose_to_block(pkg, dev, layer, shared_in):
 
 @pytest.mark.parametrize("fp8", [False, True])
 def test_decode_one_token_down_kernels_agree(pkg, dev, layer, fp8):
-    """One token: the wave-per-pair down kernel and the wave-per-row one compute the same
-    dot products in the same order, so they give the same bits."""
+    """One token: its own down kernel and the one for several tokens (MOE_DECODE_DOWN=rows) compute
+    the same dot products in the same order, so they give the same bits."""
     mlp = _mlp(layer, dev)
     if fp8:
         q, s = pkg.fp8.quantize_rows(layer["gate_up"])
@@ -220,6 +220,69 @@ def test_decode_gate_up_row_blocks_agree(pkg, dev, layer, T, routes):
     for blocks in ("4", "2"):
         for a, b in zip(got[blocks], got["1"]):
             assert torch.equal(a, b), blocks
+
+
+@pytest.mark.parametrize("T", [1, 2, 4])
+def test_decode_dot_products_keep_float32(pkg, dev, T):
+    """The sums of a projection are float32 sums: over rows whose second half undoes the first
+    the exact result is 0 and the output is the rounding error itself. A lane adds 16 terms in at
+    most 16 rounded steps, each off by at most 2^-24 of the terms so far, so no error is above
+    16 * 2^-24 of sum |x w|; the 64 lanes' errors are independent and an eighth of that share in
+    the root mean square, a lane's steps about twice one's 2^-25: 2^-27 of sum |x w|."""
+    _say("decode dot precision", T)
+    E, H, I = 16, 1024, 1024
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn(T, 512, generator=g).to(BF16)
+    x[:, 0] = 1.0
+    w = torch.randn(H, 512, generator=g).to(BF16)
+    total = x.double().abs() @ w.double().abs().T
+    xx = torch.cat([x, x], 1).to(dev)
+    rows = torch.zeros(E, H, I, dtype=BF16)
+    rows[0] = torch.cat([w, -w], 1)
+    zero = torch.zeros(T, 1, dtype=torch.long, device=dev)
+    y = pkg.ops.decode_down(xx, T, 1, rows.to(dev), zero, torch.ones(T, 1, dtype=BF16, device=dev))
+    gate_up = torch.zeros(E, 2 * I, H, dtype=BF16)
+    gate_up[0, :I, 0] = 32.0  # gate = silu(32) = 32 for x[:, 0] = 1
+    gate_up[0, I:] = rows[0]
+    act = pkg.ops.decode_gate_up(xx, gate_up.to(dev), 1, top_k_index=zero)[0]
+    torch.cuda.synchronize()
+    for err in (y.double().cpu() / total, act.double().cpu() / 32 / total):
+        assert 0 < err.abs().max() <= 2.0**-20
+        assert err.square().mean().sqrt() <= 2.0**-27
+
+
+@pytest.mark.parametrize("T", [1, 2, 3, 4])
+def test_decode_keeps_subnormal_values(pkg, dev, T):
+    """Subnormal bf16 weights (gate_up's and down's) and subnormal float32 partial sums count in
+    full: all values are powers of two, so the results are exact."""
+    _say("decode subnormals", T)
+    E, H, I = 16, 512, 512
+    idx = torch.zeros(T, 1, dtype=torch.long, device=dev)
+    one = torch.ones(T, 1, dtype=BF16, device=dev)
+
+    def out(x, gate, up, down):
+        gu, dn = torch.zeros(E, 2 * I, H), torch.zeros(E, H, I)
+        gu[0, 0], gu[0, I], dn[0, :, 0] = gate, up, down
+        return pkg.ops.moe_decode(x.to(dev), idx, one, gu.to(BF16).to(dev), dn.to(BF16).to(dev))
+
+    def unit(value, at=slice(0, 1)):
+        row = torch.zeros(H)
+        row[at] = value
+        return row
+
+    big = torch.zeros(T, H, dtype=BF16)
+    big[:, 0] = 2.0**100
+    small = torch.full((T, H), 2.0**-70, dtype=BF16)
+    small[:, 0] = 1.0
+    # gate 2^40, up 2^100 * 2^-130 (subnormal weight), down 2^-10
+    a = out(big, unit(2.0**-60), unit(2.0**-130), 2.0**-10)
+    # act 2^40 * 2^40, down 2^-130 (subnormal weight)
+    b = out(big, unit(2.0**-60), unit(2.0**-60), 2.0**-130)
+    # up: 64 products of 2^-135, each and their sum (2^-129) subnormal; gate 64, down 2^100
+    c = out(small, unit(64.0), unit(2.0**-65, slice(8, 72)), 2.0**100)
+    torch.cuda.synchronize()
+    for got, want in ((a, 1.0), (b, 2.0**-50), (c, 2.0**-23)):
+        assert (got.double() == want).all(), (got[0, 0].item(), want)
 
 
 @pytest.mark.parametrize("E,k", [(256, 8), (64, 8), (16, 4)])
