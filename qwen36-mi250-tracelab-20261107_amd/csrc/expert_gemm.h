@@ -40,9 +40,9 @@ struct GemmArgs {
   int topk, P, E, T;
   int nrb;           // weight-row blocks per tile (set by the launcher)
   int MTgrid;        // tiles the grid covers (set by the launcher)
-  int bm, nsub, nblk;  // rows per table tile, parts a tile is taken in, row blocks per
-                       // workgroup (set by the launchers)
-  unsigned in_bytes[2], out_bytes[2];  // of each operand's input and output (set by the launcher)
+  int tile_rows, nsub, nblk;  // rows per table tile, parts a tile is taken in, row blocks per
+                              // workgroup (set by the streaming kernel's launcher)
+  unsigned in_bytes, out_bytes;  // of op[0]'s input and output (set by the same)
   int shared_first;  // the table's last shared_first tiles run first (set by the launcher)
 };
 
@@ -67,11 +67,10 @@ __host__ __device__ inline int prefill_start_chunk(int e, int nch) {
 
 // Prefill batches. launch_prefill_gemm (prefill_gemm.hip) takes tables of prefill_tile_rows()
 // sorted rows per tile and passes on to prefill_stream.hip the e4m3 launches that one takes.
-constexpr int kStreamRowsLarge = 160;  // rows prefill_stream.hip takes of a tile at a time
 int prefill_tile_rows();
 bool prefill_fits(int mode, const GemmOperand& op);
-hipError_t launch_prefill_gemm(int mode, const GemmArgs& a, int max_tiles, int bm, hipStream_t st);
-// A routed e4m3 launch (a.bm set, a table, prefill_fits operands): whether it takes the streaming
+hipError_t launch_prefill_gemm(int mode, const GemmArgs& a, int max_tiles, hipStream_t st);
+// A routed e4m3 launch (op[0], a table, prefill_fits operands): whether it takes the streaming
 // kernel, and that kernel's launch. The streaming kernel reads a row block's weights once per
 // 160 rows of an expert, the one staged through LDS once per 256: the line is the average number
 // of rows per expert from which many experts need a second pass. A block (H = 2048, I = 512,

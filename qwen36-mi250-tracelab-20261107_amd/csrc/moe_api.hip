@@ -44,22 +44,17 @@ using namespace moe;
 
 namespace {
 
-// Whether T tokens run on the prefill kernel (above 512 tokens, shapes it tiles).
-bool prefill_for(int T, int H, int I, int IS) {
-  return T > 512 && H % 256 == 0 && I % 128 == 0 && IS % 128 == 0;
-}
-
 // Sorted rows per tile of the grouped GEMMs: one 16-row MFMA block for one token (K split
-// over 4 waves), two blocks up to 512 tokens, and the prefill kernel's tiles above (shapes it
-// does not tile: 64-row tiles of the expert GEMM).
-int tile_rows_for(int T, int k, int E, int H, int I, int IS, bool fp8) {
+// over 4 waves), two blocks up to 512 tokens, and the prefill kernels' tiles above (shapes they
+// do not tile: 64-row tiles of the expert GEMM).
+int tile_rows_for(int T, int H, int I, int IS) {
   // 32-row tiles from 2 tokens: per layer (12 layers cycled) 8 / 16 tokens take 81 / 113 µs
   // with fp8 experts against 128 / 213 with 16-row tiles, and 102 / 150 against 107 / 166
   // with bf16; at 2 / 3 / 4 tokens (16 layers) fp8 50 / 53 / 56 against 55 / 68 / 79 and
   // bf16 49 / 59 / 69 against 51 / 60 / 69; one token 44 against 40 (bf16)
   if (T <= 1) return 16;
   if (T <= 512) return 32;
-  return prefill_for(T, H, I, IS) ? prefill_tile_rows() : 64;
+  return H % 256 == 0 && I % 128 == 0 && IS % 128 == 0 ? prefill_tile_rows() : 64;
 }
 
 thread_local std::string g_err;
@@ -121,7 +116,8 @@ bool prefill_side_enabled() {
 // tiles of up to 96 rows per expert on average. Above that it goes first in the routed
 // launches: the two hops between queues cost more than the overlap with the router gains
 // (T = 4096: 502 against 509 µs).
-bool block_side_enabled(bool fp8, bool prefill, long long P, int E) {
+bool block_side_enabled(bool fp8, int bm, long long P, int E) {
+  const bool prefill = bm == prefill_tile_rows();
   return (fp8 && !mixed_enabled()) || (prefill && (fp8 || P <= 96LL * E));
 }
 
@@ -278,20 +274,21 @@ class Fork {
 // 4 or 8 row blocks), and the shared expert's tiles would add a last, mostly idle round; run
 // them as a second launch on the auxiliary stream instead, where they fill the gaps of the
 // routed launch.
-hipError_t launch_prefill_split(int mode, const GemmArgs& a, int MT, int bm, hipStream_t s) {
+hipError_t launch_prefill_split(int mode, const GemmArgs& a, int MT, hipStream_t s) {
   AuxStream* aux = a.op[0].N > 0 && a.op[1].N > 0 && a.table ? aux_stream(s) : nullptr;
-  if (!aux || !prefill_side_enabled()) return launch_prefill_gemm(mode, a, MT, bm, s);
+  if (!aux || !prefill_side_enabled()) return launch_prefill_gemm(mode, a, MT, s);
   GemmArgs v = a;  // no table: the prefill kernel covers the shared rows from the token count
   v.op[0].N = 0;
   v.table = nullptr;
   Fork fork(aux, s);
   hipError_t e = fork.begin();
   if (e != hipSuccess) return e;
-  e = launch_prefill_gemm(mode, v, (a.T + bm - 1) / bm, bm, fork.aux());
+  e = launch_prefill_gemm(mode, v, (a.T + prefill_tile_rows() - 1) / prefill_tile_rows(),
+                          fork.aux());
   if (e != hipSuccess) return e;
   GemmArgs r = a;
   r.op[1].N = 0;
-  e = launch_prefill_gemm(mode, r, MT, bm, s);
+  e = launch_prefill_gemm(mode, r, MT, s);
   if (e != hipSuccess) return e;
   return fork.join();
 }
@@ -324,12 +321,13 @@ hipError_t launch_split(int mode, int role, int bm, const GemmArgs& a, int MT, h
 // count alone).
 enum Part { kBoth = 0, kRoutedOnly = 1, kSharedOnly = 2 };
 
-hipError_t launch_part(int mode, int role, int bm, bool prefill, const GemmArgs& a, int MT,
-                       int part, hipStream_t s) {
+hipError_t launch_part(int mode, int role, int bm, const GemmArgs& a, int MT, int part,
+                       hipStream_t s) {
+  const bool prefill = bm == prefill_tile_rows();
   if (part == kRoutedOnly) {
     GemmArgs r = a;
     r.op[1].N = 0;
-    return prefill ? launch_prefill_gemm(mode, r, MT, bm, s)
+    return prefill ? launch_prefill_gemm(mode, r, MT, s)
                    : launch_expert_gemm(mode, role, bm, r, MT, s);
   }
   if (part == kSharedOnly) {
@@ -338,20 +336,20 @@ hipError_t launch_part(int mode, int role, int bm, bool prefill, const GemmArgs&
     const int tiles = (a.T + bm - 1) / bm;
     if (prefill) {
       v.op[0].N = 0;  // the prefill kernel covers the shared rows from the token count
-      return launch_prefill_gemm(mode, v, tiles, bm, s);
+      return launch_prefill_gemm(mode, v, tiles, s);
     }
     v.op[0] = v.op[1];  // the configuration follows op[0]'s weight type
     v.op[0].N = 0;
     return launch_expert_gemm(mode, role, bm, v, tiles, s);
   }
-  return prefill ? launch_prefill_split(mode, a, MT, bm, s)
+  return prefill ? launch_prefill_split(mode, a, MT, s)
                  : launch_split(mode, role, bm, a, MT, s);
 }
 
 int run_gate_up(const void* x, int T, int H, int E, int k, int I, const void* gate_up,
                 const float* gu_scale, int wdtype, const void* sh_gate, const void* sh_up, int IS,
-                const int* order, const int* table, int MT, int bm, bool prefill, void* act,
-                void* act_sh, hipStream_t s, int part = kBoth) {
+                const int* order, const int* table, int MT, int bm, void* act, void* act_sh,
+                hipStream_t s, int part = kBoth) {
   GemmArgs a{};
   a.op[0] = gate_up_operand(gate_up, gu_scale, H, I, x, act);
   a.op[0].fp8 = wdtype == MOE_WEIGHTS_FP8_E4M3;
@@ -377,7 +375,7 @@ int run_gate_up(const void* x, int T, int H, int E, int k, int I, const void* ga
   a.P = T * k;
   a.E = E;
   a.T = T;
-  hipError_t err = launch_part(kModeSwiglu, kRoleGateUp, bm, prefill, a, MT, sh_gate ? part : kBoth, s);
+  hipError_t err = launch_part(kModeSwiglu, kRoleGateUp, bm, a, MT, sh_gate ? part : kBoth, s);
   if (err == hipErrorInvalidValue)
     return fail(MOE_EINVAL, "gate_up: no kernel configuration for H=%d I=%d IS=%d", H, I, IS);
   return hip_check(err, "gate_up launch");
@@ -385,7 +383,7 @@ int run_gate_up(const void* x, int T, int H, int E, int k, int I, const void* ga
 
 int run_down(const void* act, int T, int H, int E, int k, int I, const void* down,
              const float* dn_scale, int wdtype, const void* sh_down, int IS, const void* act_sh,
-             const int* order, const int* table, int MT, int bm, bool prefill, void* y, void* y_sh,
+             const int* order, const int* table, int MT, int bm, void* y, void* y_sh,
              hipStream_t s, int part = kBoth) {
   GemmArgs a{};
   a.op[0] = down_operand(down, dn_scale, H, I, act, y);
@@ -411,7 +409,7 @@ int run_down(const void* act, int T, int H, int E, int k, int I, const void* dow
   a.P = T * k;
   a.E = E;
   a.T = T;
-  hipError_t err = launch_part(kModePlain, kRoleDown, bm, prefill, a, MT, sh_down ? part : kBoth, s);
+  hipError_t err = launch_part(kModePlain, kRoleDown, bm, a, MT, sh_down ? part : kBoth, s);
   if (err == hipErrorInvalidValue)
     return fail(MOE_EINVAL, "down: no kernel configuration for H=%d I=%d IS=%d", H, I, IS);
   return hip_check(err, "down launch");
@@ -456,7 +454,8 @@ void moe_reload_tuning(void) { read_knobs(); }
 
 const char* moe_last_error(void) { return g_err.c_str(); }
 
-int moe_tile_rows(int T) { return T <= 1 ? 16 : T <= 512 ? 32 : prefill_tile_rows(); }
+// for shapes that the prefill kernels tile
+int moe_tile_rows(int T) { return tile_rows_for(T, 256, 128, 128); }
 
 int moe_max_tiles(int T, int k, int E, int bm, int has_shared) {
   if (T < 0 || k < 1 || E < 1 || bm < 1) return 0;
@@ -551,8 +550,7 @@ int moe_grouped_gate_up(const void* x, int T, int H, int E, int k, int I, const 
   CHECK_ARG(bm == 16 || bm == 32 || bm == 64 || bm == 128 || bm == prefill_tile_rows(),
             "bm must be 16, 32, 64, 128 or %d (got %d)", prefill_tile_rows(), bm);
   return run_gate_up(x, T, H, E, k, I, gate_up, gu_scale, wdtype, sh_gate, sh_up, IS, order,
-                     table, max_tiles, bm, bm == prefill_tile_rows(), act, act_sh,
-                     (hipStream_t)stream);
+                     table, max_tiles, bm, act, act_sh, (hipStream_t)stream);
 }
 
 int moe_grouped_down(const void* act, int T, int H, int E, int k, int I, const void* down,
@@ -570,7 +568,7 @@ int moe_grouped_down(const void* act, int T, int H, int E, int k, int I, const v
   CHECK_ARG(bm == 16 || bm == 32 || bm == 64 || bm == 128 || bm == prefill_tile_rows(),
             "bm must be 16, 32, 64, 128 or %d (got %d)", prefill_tile_rows(), bm);
   return run_down(act, T, H, E, k, I, down, dn_scale, wdtype, sh_down, IS, act_sh, order, table,
-                  max_tiles, bm, bm == prefill_tile_rows(), y, y_sh, (hipStream_t)stream);
+                  max_tiles, bm, y, y_sh, (hipStream_t)stream);
 }
 
 int moe_combine(const void* y, const void* w, int T, int H, int k, const void* ysh,
@@ -693,14 +691,12 @@ struct ExpertsWs {
   uint16_t *act, *y;
   size_t bytes;
   int MT, bm;
-  bool prefill;
 };
-ExpertsWs carve_experts(void* base, int T, int H, int E, int k, int I, bool fp8) {
+ExpertsWs carve_experts(void* base, int T, int H, int E, int k, int I) {
   Carver c{static_cast<char*>(base)};
   ExpertsWs w{};
   const int P = T * k;
-  w.bm = tile_rows_for(T, k, E, H, I, I, fp8);
-  w.prefill = prefill_for(T, H, I, I);
+  w.bm = tile_rows_for(T, H, I, I);
   w.MT = max_tiles_of(T, k, E, w.bm, 0);
   w.idx32 = c.take<int>(P);
   w.counts = c.take<int>(E);
@@ -717,9 +713,7 @@ ExpertsWs carve_experts(void* base, int T, int H, int E, int k, int I, bool fp8)
 
 size_t moe_experts_workspace_bytes(int T, int H, int E, int k, int I) {
   if (T < 0 || k < 1 || E < 1) return 0;
-  const size_t a = carve_experts(nullptr, T, H, E, k, I, false).bytes;
-  const size_t b = carve_experts(nullptr, T, H, E, k, I, true).bytes;
-  return a > b ? a : b;
+  return carve_experts(nullptr, T, H, E, k, I).bytes;
 }
 
 int moe_experts_forward(const void* x, int T, int H, int E, int k, int I,
@@ -735,7 +729,7 @@ int moe_experts_forward(const void* x, int T, int H, int E, int k, int I,
             "bad weight dtype / missing scales");
   CHECK_ARG(x && top_k_index && top_k_weights && gate_up && down && out, "null pointer");
   if (T == 0) return MOE_OK;
-  ExpertsWs w = carve_experts(workspace, T, H, E, k, I, wdtype == MOE_WEIGHTS_FP8_E4M3);
+  ExpertsWs w = carve_experts(workspace, T, H, E, k, I);
   CHECK_ARG(workspace && workspace_bytes >= w.bytes, "workspace too small: %zu < %zu",
             workspace_bytes, w.bytes);
   hipStream_t s = (hipStream_t)stream;
@@ -760,10 +754,10 @@ int moe_experts_forward(const void* x, int T, int H, int E, int k, int I,
                             nullptr, w.counts, w.offsets, w.order, w.table, w.MT, w.scratch, s),
           "sort launch");
   rc = run_gate_up(x, T, H, E, k, I, gate_up, gu_scale, wdtype, nullptr, nullptr, 0, w.order,
-                   w.table, w.MT, w.bm, w.prefill, w.act, nullptr, s);
+                   w.table, w.MT, w.bm, w.act, nullptr, s);
   if (rc) return rc;
   rc = run_down(w.act, T, H, E, k, I, down, dn_scale, wdtype, nullptr, 0, nullptr, w.order, w.table,
-                w.MT, w.bm, w.prefill, w.y, nullptr, s);
+                w.MT, w.bm, w.y, nullptr, s);
   if (rc) return rc;
   return hip_check(launch_combine(w.y, static_cast<const uint16_t*>(top_k_weights), k, nullptr,
                                   nullptr, 0, nullptr, static_cast<uint16_t*>(out), T, H,
@@ -784,15 +778,12 @@ struct BlockWs {
   float* part;  // the router's fp32 K-quarter partial sums (router_part_takes)
   size_t bytes;
   int MT, bm;
-  bool prefill;
 };
-BlockWs carve_block(void* base, int T, int H, int E, int k, int I, int IS, int n_pack,
-                    bool fp8) {
+BlockWs carve_block(void* base, int T, int H, int E, int k, int I, int IS, int n_pack) {
   Carver c{static_cast<char*>(base)};
   BlockWs w{};
   const int P = T * k;
-  w.bm = tile_rows_for(T, k, E, H, I, IS, fp8);
-  w.prefill = prefill_for(T, H, I, IS);
+  w.bm = tile_rows_for(T, H, I, IS);
   w.MT = max_tiles_of(T, k, E, w.bm, 1);
   w.logits = c.take<uint16_t>((size_t)T * n_pack);
   w.idx64 = c.take<long long>(P);
@@ -819,9 +810,7 @@ BlockWs carve_block(void* base, int T, int H, int E, int k, int I, int IS, int n
 
 size_t moe_block_workspace_bytes(int T, int H, int E, int k, int I, int IS, int n_pack) {
   if (T < 0 || k < 1 || E < 1) return 0;
-  const size_t a = carve_block(nullptr, T, H, E, k, I, IS, n_pack, false).bytes;
-  const size_t b = carve_block(nullptr, T, H, E, k, I, IS, n_pack, true).bytes;
-  return a > b ? a : b;
+  return carve_block(nullptr, T, H, E, k, I, IS, n_pack).bytes;
 }
 
 }  // extern "C"
@@ -852,7 +841,7 @@ int block_forward(const void* x, int T, int H, int E, int k, int I, int IS, cons
   CHECK_ARG(x && w_pack && gate_up && down && sh_gate && sh_up && sh_down && out, "null pointer");
   CHECK_ARG((((intptr_t)sh_up - (intptr_t)sh_gate) & 1) == 0, "misaligned shared weights");
   if (T == 0) return MOE_OK;
-  BlockWs w = carve_block(workspace, T, H, E, k, I, IS, n_pack, wdtype == MOE_WEIGHTS_FP8_E4M3);
+  BlockWs w = carve_block(workspace, T, H, E, k, I, IS, n_pack);
   CHECK_ARG(workspace && workspace_bytes >= w.bytes, "workspace too small: %zu < %zu",
             workspace_bytes, w.bytes);
   hipStream_t s = (hipStream_t)stream;
@@ -901,7 +890,7 @@ int block_forward(const void* x, int T, int H, int E, int k, int I, int IS, cons
   // The shared expert depends on x alone: where its projections run as launches of their own
   // (block_side_enabled), they run on the auxiliary stream
   // from the start of the block, beside the router and routing, and join before the combine.
-  AuxStream* aux = block_side_enabled(wdtype == MOE_WEIGHTS_FP8_E4M3, w.prefill, (long long)T * k, E)
+  AuxStream* aux = block_side_enabled(wdtype == MOE_WEIGHTS_FP8_E4M3, w.bm, (long long)T * k, E)
                        ? aux_stream(s)
                        : nullptr;
   const int part = aux ? kRoutedOnly : kBoth;
@@ -909,10 +898,10 @@ int block_forward(const void* x, int T, int H, int E, int k, int I, int IS, cons
   if (aux) {
     HIP_TRY(fork.begin(), "fork");
     rc = run_gate_up(x, T, H, E, k, I, gate_up, gu_scale, wdtype, sh_gate, sh_up, IS, w.order,
-                     w.table, w.MT, w.bm, w.prefill, w.act, w.act_sh, fork.aux(), kSharedOnly);
+                     w.table, w.MT, w.bm, w.act, w.act_sh, fork.aux(), kSharedOnly);
     if (rc) return rc;
     rc = run_down(w.act, T, H, E, k, I, down, dn_scale, wdtype, sh_down, IS, w.act_sh, w.order,
-                  w.table, w.MT, w.bm, w.prefill, w.y, w.y_sh, fork.aux(), kSharedOnly);
+                  w.table, w.MT, w.bm, w.y, w.y_sh, fork.aux(), kSharedOnly);
     if (rc) return rc;
   }
   if (w.part) {
@@ -932,10 +921,10 @@ int block_forward(const void* x, int T, int H, int E, int k, int I, int IS, cons
             "route/sort launch");
   }
   rc = run_gate_up(x, T, H, E, k, I, gate_up, gu_scale, wdtype, sh_gate, sh_up, IS, w.order,
-                   w.table, w.MT, w.bm, w.prefill, w.act, w.act_sh, s, part);
+                   w.table, w.MT, w.bm, w.act, w.act_sh, s, part);
   if (rc) return rc;
   rc = run_down(w.act, T, H, E, k, I, down, dn_scale, wdtype, sh_down, IS, w.act_sh, w.order,
-                w.table, w.MT, w.bm, w.prefill, w.y, w.y_sh, s, part);
+                w.table, w.MT, w.bm, w.y, w.y_sh, s, part);
   if (rc) return rc;
   HIP_TRY(fork.join(), "join");
   return hip_check(launch_combine(w.y, wt, k, w.y_sh, lg + E, n_pack,

@@ -123,9 +123,9 @@ __global__ __launch_bounds__(kThreads, 1) void k_prefill_gemm(GemmArgs args) {
     }
     e = args.table[tile];
     r0 = args.table[args.MT + tile];
-    // the table holds the expert's end row; this tile is its next bm rows at most (bm <= PBM:
-    // the token-row ring stages hold PBM rows)
-    r1 = min(args.table[2 * args.MT + tile], r0 + args.bm);
+    // the table holds the expert's end row; this tile is its next PBM rows at most (the
+    // token-row ring stages hold PBM rows)
+    r1 = min(args.table[2 * args.MT + tile], r0 + PBM);
   } else {
     e = args.E;
     r0 = args.P + tile * PBM;
@@ -598,10 +598,8 @@ hipError_t allow_lds(const void* fn, int which, int bytes) {
 }
 }  // namespace
 
-hipError_t launch_prefill_gemm(int mode, const GemmArgs& a_in, int max_tiles, int bm,
-                               hipStream_t st) {
+hipError_t launch_prefill_gemm(int mode, const GemmArgs& a_in, int max_tiles, hipStream_t st) {
   GemmArgs a = a_in;
-  if (bm != PBM) return hipErrorInvalidValue;
   if (!prefill_fits(mode, a.op[0]) || !prefill_fits(mode, a.op[1])) return hipErrorInvalidValue;
   const bool has0 = a.op[0].N > 0, has1 = a.op[1].N > 0;
   if (has0 && has1 && a.op[0].fp8 != a.op[1].fp8) {
@@ -610,12 +608,11 @@ hipError_t launch_prefill_gemm(int mode, const GemmArgs& a_in, int max_tiles, in
     GemmArgs r = a, v = a;
     r.op[1].N = 0;
     v.op[0].N = 0;
-    hipError_t err = launch_prefill_gemm(mode, r, max_tiles, bm, st);
-    return err != hipSuccess ? err : launch_prefill_gemm(mode, v, max_tiles, bm, st);
+    hipError_t err = launch_prefill_gemm(mode, r, max_tiles, st);
+    return err != hipSuccess ? err : launch_prefill_gemm(mode, v, max_tiles, st);
   }
   const bool f8 = (has0 && a.op[0].fp8) || (has1 && a.op[1].fp8);
   if (max_tiles <= 0 || (!has0 && !has1)) return hipSuccess;
-  a.bm = bm;
   if (f8) {
     // e4m3 weights are the routed experts' only
     if (has1 || !a.table) return hipErrorInvalidValue;
@@ -624,7 +621,7 @@ hipError_t launch_prefill_gemm(int mode, const GemmArgs& a_in, int max_tiles, in
   a.shared_first = 0;
   if (a.table && has0 && has1) {
     const char* env = knob(kKnobPrefillSharedFirst);
-    if (!(env && env[0] == '0')) a.shared_first = (a.T + bm - 1) / bm;
+    if (!(env && env[0] == '0')) a.shared_first = (a.T + PBM - 1) / PBM;
   }
   const int out_per_wg = mode == kModeSwiglu ? PBN / 2 : PBN;
   const int nmax = a.op[0].N > a.op[1].N ? a.op[0].N : a.op[1].N;

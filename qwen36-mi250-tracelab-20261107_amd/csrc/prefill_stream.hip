@@ -1,22 +1,24 @@
-// Grouped MFMA GEMM for prefill-sized batches on gfx950 with weights streamed through registers
-// (subsystems a8, a9, a6): e4m3 weights (prefill_gemm.hip has bf16 ones, for which this form
-// measured slower where expert popularity is skewed: a block of 1111 tokens, Zipf(1.1) routing,
-// 457 against 438 µs).
+// Grouped MFMA GEMM for prefill-sized batches on gfx950 with e4m3 weights streamed through
+// registers (subsystems a8, a9, a6): the routed experts' launches that prefill_stream_takes.
+// prefill_gemm.hip has the other ones (bf16 weights, many rows per expert, other K).
 //
 // Same contract as k_expert_gemm (expert_gemm.hip) and the reference's grouped kernels
 // (engine/fast/moe_prefill.py:156-257): for the sorted rows of ONE expert in a tile,
 //   SWIGLU: act[r, n]       = bf16(bf16(silu(bf16 g)) * bf16 u)
 //   PLAIN:  out[orow(r), n] = bf16(act_or_x[r] . W[e, n])
-// with bf16 or e4m3 weights (per-output-row fp32 scales on the fp32 accumulator).
+// with e4m3 weights and per-output-row fp32 scales on the fp32 accumulator. It takes tables of
+// routed experts' tiles (op[0]; a shared expert's tiles are passed over), K a multiple of 128 from
+// 256 on, outputs in multiples of 16, tensors under 4 GiB.
 //
-// Split. A workgroup of W = 8 waves takes blocks of 32 W weight rows and up to 16 MAXB token rows
-// of a tile; wave w owns 32 rows of a block (two 16-row MFMA blocks; SWIGLU: 16 gate rows and
+// Split. A workgroup of 8 waves takes blocks of 256 weight rows and up to 160 token rows of a
+// tile; a wave owns 32 rows of a block (two 16-row MFMA blocks; SWIGLU: 16 gate rows and
 // the matching 16 up rows, paired in registers by the epilogue) against every token row.
 // * A weight row is used by one wave only, so weights go from HBM straight into that wave's
 //   registers in the MFMA A layout (lane: row l % 16, 16 bytes at 16 (l / 16); 64 contiguous
 //   bytes of each of 16 rows per load), a ring of R chunks of 64 k. The launch is bound by
 //   this stream and by the stores that share the memory with it; registers hold more of it in
-//   flight than LDS could.
+//   flight than LDS could. (bf16 weights in this form measured slower than staged where expert
+//   popularity is skewed: a block of 1111 tokens, Zipf(1.1) routing, 457 against 438 µs.)
 // * Token rows are used by all waves: global -> LDS DMA (no registers on the way) in phases of
 //   R chunks, two stages: the next phase is requested at the start of the current one, and one
 //   barrier separates them.
@@ -25,14 +27,13 @@
 //
 // Measured (block, H = 2048, I = 512, E = 256, top-8, µs) against the kernel staged through LDS
 // before it: 1111 / 2048 tokens 312 / 358 -> 289 / 320; Zipf(1.1) routing at 600 / 1111 / 2500 /
-// 4096 tokens 310 / 356 / 433 / 541 -> 289 / 330 / 417 / 545. 160-row tiles for every batch: 64-row
+// 4096 tokens 310 / 356 / 433 / 541 -> 289 / 330 / 417 / 545. 160-row parts for every batch: 64-row
 // ones gain 3 % at 1111 tokens with uniform routing and lose 13 % with Zipf.
 //
-// LDS layout of a chunk: row r's 128 bytes at 128 r; 16-byte unit q holds logical unit
-// q ^ (r & 7), so the fragment reads (16 rows, one unit) are bank-conflict free. With e4m3
-// weights a lane's 16 weight bytes are k = 16 kq .. + 15, fed as two k-steps of 8 bytes, so
-// the token units are permuted alike: k-step h's lane group kq reads logical unit 2 kq + h,
-// stored where the bf16 form's k-step h reads.
+// LDS layout of a chunk: row r's 128 bytes at 128 r; 16-byte unit q of row r sits at physical unit
+// p(q) ^ (r & 7), p(2 kq + h) = 4 h + kq: a lane's 16 weight bytes are k = 16 kq .. + 15, fed as two
+// k-steps of 8 bytes, so k-step h's lane group kq reads logical unit 2 kq + h, and its fragment
+// reads (16 rows, one unit) are bank-conflict free.
 //
 // The body is compiled per number of 16-token blocks (NB), so that a part-filled tile loads,
 // reads and multiplies only the blocks it has.
@@ -58,24 +59,19 @@ constexpr int kPBlkBytes = 16 * kPRowBytes;      // a 16-token block of a stage:
 template <int MODE>
 constexpr int kStorePolicy = MODE == kModeSwiglu ? 16 : 0;
 constexpr int kXcds = 8;            // XCDs of an MI355X (round-robin dispatch)
-constexpr int kPBlocksLarge = kStreamRowsLarge / 16;  // MAXB
+constexpr int kWaves = 8;
+constexpr int kMaxBlocks = 10;                   // 16-token blocks of a part of a tile
+constexpr int kPartRows = 16 * kMaxBlocks;
+constexpr int kRows = 32 * kWaves;               // weight rows per block
+// output rows per block
+template <int MODE>
+constexpr int kOut = MODE == kModeSwiglu ? kRows / 2 : kRows;
 }  // namespace
 
 // The NB token fragments (16 rows each, 2 KiB apart) at LDS byte address addr, waited for.
 // One asm block, so no fragment register is visible before its data has arrived.
 template <int NB>
 struct TokenFrags;
-template <>
-struct TokenFrags<2> {
-  static __device__ __forceinline__ void read(uint32_t addr, u32x4v (&f)[2]) {
-    asm volatile(
-               "ds_read_b128 %0, %2 offset:0\n\t"
-               "ds_read_b128 %1, %2 offset:2048\n\t"
-               "s_waitcnt lgkmcnt(0)"
-               : "=&v"(f[0]), "=&v"(f[1])
-               : "v"(addr));
-  }
-};
 template <>
 struct TokenFrags<4> {
   static __device__ __forceinline__ void read(uint32_t addr, u32x4v (&f)[4]) {
@@ -160,15 +156,13 @@ __device__ __forceinline__ u32x4v ld_weight(const char* p) {
 // consecutive results of one token (16-byte stores, half as many), always all of them: those
 // of rows past the tile or the weights go past the buffer's end, where they are dropped. The
 // weights of the next block are in flight meanwhile, and their waits count the stores.
-template <int MODE, bool FP8, int NB, int W, class OutRow>
-__device__ __forceinline__ void prefill_epilogue(const GemmArgs& args, const GemmOperand& op,
-                                                 bool routed, int e, int r0, int r1, int rb,
-                                                 int wave, int lr, int kq,
-                                                 OutRow out_row,
+template <int MODE, int NB, class OutRow>
+__device__ __forceinline__ void prefill_epilogue(const GemmArgs& args, int e, int r0, int r1,
+                                                 int rb, int wave, int lr, int kq, OutRow out_row,
                                                  const f32x4_t (&acc)[2][NB]) {
-  constexpr int kRows = 32 * W;
+  const GemmOperand& op = args.op[0];
   constexpr int kA = MODE == kModeSwiglu ? 1 : 2;  // 16-row groups of results
-  const float* sc = FP8 && op.scale ? op.scale + (long long)(routed ? e : 0) * op.sstride : nullptr;
+  const float* sc = op.scale ? op.scale + (long long)e * op.sstride : nullptr;
   const int nw = MODE == kModeSwiglu ? rb * (kRows / 2) + wave * 16 : rb * kRows + wave * 32;
   const int n0 = nw + 4 * kq;
   float scl[2][4] = {{1.f, 1.f, 1.f, 1.f}, {1.f, 1.f, 1.f, 1.f}};
@@ -195,7 +189,7 @@ __device__ __forceinline__ void prefill_epilogue(const GemmArgs& args, const Gem
     }
   };
   const __amdgpu_buffer_rsrc_t obuf = __builtin_amdgcn_make_buffer_rsrc(
-      op.out, 0, args.out_bytes[routed ? 0 : 1], 0x00020000);
+      op.out, 0, args.out_bytes, 0x00020000);
   const uint32_t ld = (uint32_t)(op.ld_out * 2);
 #pragma unroll
   for (int b = 0; b < NB; b += 2) {
@@ -226,18 +220,16 @@ __device__ __forceinline__ void prefill_epilogue(const GemmArgs& args, const Gem
 // One workgroup's product: weight rows of blocks rb0 .. rb0 + nblk - 1 (expert e) against sorted
 // rows [r0, r1), r1 - r0 <= 16 NB. R: chunks per phase and ring depth; K / 64 is a multiple of
 // R, at least 2 R. RES: K = 128 R, both phases stay in LDS for all blocks.
-template <int MODE, bool FP8, int NB, int W, int R, bool RES>
-__device__ __forceinline__ void prefill_body(const GemmArgs& args, const GemmOperand& op,
-                                             bool routed, int e, int r0, int r1, int rb0, int nblk,
-                                             char* lds) {
-  constexpr int kCB = FP8 ? kPKC : 2 * kPKC;  // weight bytes of a row per chunk
-  constexpr int kLS = FP8 ? 1 : 2;            // weight loads per row block and chunk
-  constexpr int kLA = 2 * kLS;                // weight loads per chunk
+template <int MODE, int NB, int R, bool RES>
+__device__ __forceinline__ void prefill_body(const GemmArgs& args, int e, int r0, int r1, int rb0,
+                                             int nblk, char* lds) {
+  constexpr int W = kWaves;
+  constexpr int kLA = 2;                      // weight loads per chunk: one per row block
   constexpr int kLB = 2 * NB * R / W;         // token DMA loads of a wave per phase
   constexpr int kSub = NB * kPBlkBytes;       // a chunk of the token rows in LDS
   constexpr int kStage = R * kSub;            // a phase
-  constexpr int kRows = 32 * W;               // weight rows per block
   static_assert(kLB * W == 2 * NB * R && W % R == 0, "whole DMA groups per wave");
+  const GemmOperand& op = args.op[0];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -250,41 +242,35 @@ __device__ __forceinline__ void prefill_body(const GemmArgs& args, const GemmOpe
   const int sub = wave % R;
   const int grow = lane >> 3;
   const int pq = (lane & 7) ^ grow;
-  const int unit = FP8 ? 2 * (pq & 3) + (pq >> 2) : pq;
+  const int unit = 2 * (pq & 3) + (pq >> 2);
   int trow[kLB];
 #pragma unroll
   for (int i = 0; i < kLB; ++i)
     trow[i] = min(r0 + (wave / R + (W / R) * i) * 8 + grow, r1 - 1);
   // gate_up rows are pairs in sorted order, whose tokens order gives; down rows are sorted rows
-  const bool lookup = MODE == kModeSwiglu && routed;
-  if (lookup) {
+  if (MODE == kModeSwiglu) {
 #pragma unroll
     for (int i = 0; i < kLB; ++i) trow[i] = args.order[trow[i]];
   }
-  const int row_base = routed ? 0 : args.P;
-  const int row_div = lookup ? args.topk : 1;
+  const int row_div = MODE == kModeSwiglu ? args.topk : 1;
 
   // The output rows. Down's pairs are looked up once: lane 16 m + l holds row l of 16-row
   // block 4 i + m.
   int orow[(NB + 3) / 4];
-  if (MODE == kModePlain && routed) {
+  if (MODE == kModePlain) {
 #pragma unroll
     for (int i = 0; i < (NB + 3) / 4; ++i) orow[i] = args.order[min(r0 + i * 64 + lane, r1 - 1)];
   }
   // of row lr of block b, one of the constant group of four blocks that holds b0
   auto out_row = [&](int b, int b0) __attribute__((always_inline)) {
-    const int row = r0 + b * 16 + lr;
-    if (MODE == kModeSwiglu) return row - row_base;
-    const int looked = __shfl(orow[b0 / 4], (b & 3) * 16 + lr);
-    return routed ? looked : row - row_base;
+    if (MODE == kModeSwiglu) return r0 + b * 16 + lr;
+    return __shfl(orow[b0 / 4], (b & 3) * 16 + lr);
   };
 
   // ---- this lane's two weight rows of a block: wave-uniform bases, 32-bit lane offsets (the
   // launcher checks that an expert's rows span less than 2 GiB)
-  constexpr int kEB = FP8 ? 1 : 2;
-  const char* const wbase =
-      reinterpret_cast<const char*>(op.w) + (long long)(routed ? e : 0) * op.estride * kEB;
-  const char* const wbase1 = wbase + (MODE == kModeSwiglu ? op.up_off * kEB : 0);
+  const char* const wbase = reinterpret_cast<const char*>(op.w) + (long long)e * op.estride;
+  const char* const wbase1 = wbase + (MODE == kModeSwiglu ? op.up_off : 0);
   uint32_t woff[2];
   auto weight_rows = [&](int rb) __attribute__((always_inline)) {
 #pragma unroll
@@ -294,17 +280,15 @@ __device__ __forceinline__ void prefill_body(const GemmArgs& args, const GemmOpe
         row = rb * (kRows / 2) + wave * 16 + lr;
       else  // the last block may be partial
         row = min(rb * kRows + wave * 32 + a * 16 + lr, op.N - 1);
-      woff[a] = rb < 0 ? 0u : (uint32_t)row * (uint32_t)(op.ldw * kEB) + (uint32_t)(kq * 16);
+      woff[a] = rb < 0 ? 0u : (uint32_t)row * (uint32_t)op.ldw + (uint32_t)(kq * 16);
     }
   };
   const int nch = op.K / kPKC;
-  u32x4v ring[R][2][kLS];
+  u32x4v ring[R][2];
   auto issue_a = [&](int slot, int c) __attribute__((always_inline)) {
 #pragma unroll
     for (int a = 0; a < 2; ++a)
-#pragma unroll
-      for (int s = 0; s < kLS; ++s)
-        ring[slot][a][s] = ld_weight((a ? wbase1 : wbase) + c * kCB + s * 64 + woff[a]);
+      ring[slot][a] = ld_weight((a ? wbase1 : wbase) + c * kPKC + woff[a]);
     issue_fence();
   };
   // The DMA is the buffer form: its counter is one the compiler can count loads in order with
@@ -313,7 +297,7 @@ __device__ __forceinline__ void prefill_body(const GemmArgs& args, const GemmOpe
   uint32_t toff[kLB];
   auto issue_b = [&](int stage, int phase, bool any) __attribute__((always_inline)) {
     const __amdgpu_buffer_rsrc_t tbuf = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(op.in), 0, any ? args.in_bytes[routed ? 0 : 1] : 0, 0x00020000);
+        const_cast<uint16_t*>(op.in), 0, any ? args.in_bytes : 0, 0x00020000);
 #pragma unroll
     for (int i = 0; i < kLB; ++i)
       dma16_buffer(tbuf,
@@ -329,24 +313,19 @@ __device__ __forceinline__ void prefill_body(const GemmArgs& args, const GemmOpe
 #pragma unroll
       for (int b = 0; b < NB; ++b) acc[a][b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   };
-  // fragment read offsets of k-steps 0 and 1: row lr of a block, logical unit 4 h + kq (bf16)
+  // fragment read offsets of k-steps 0 and 1: row lr of a block, physical unit 4 h + kq
   const uint32_t lbase = lds_addr(lds) + (uint32_t)(lr * kPRowBytes);
   const uint32_t roff[2] = {lbase + (uint32_t)((kq ^ (lr & 7)) * 16),
                             lbase + (uint32_t)(((4 + kq) ^ (lr & 7)) * 16)};
-  auto mma = [&](int slot, uint32_t at, int steps) __attribute__((always_inline)) {
+  auto mma = [&](int slot, uint32_t at) __attribute__((always_inline)) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      if (h >= steps) break;
       u32x4v f[NB];
       TokenFrags<NB>::read(roff[h] + at, f);
 #pragma unroll
       for (int a = 0; a < 2; ++a) {
-        u32x4v w;
-        if constexpr (FP8)
-          w = h ? widen8(ring[slot][a][0].z, ring[slot][a][0].w)
-                : widen8(ring[slot][a][0].x, ring[slot][a][0].y);
-        else
-          w = ring[slot][a][h];
+        const u32x4v w = h ? widen8(ring[slot][a].z, ring[slot][a].w)
+                           : widen8(ring[slot][a].x, ring[slot][a].y);
 #pragma unroll
         for (int b = 0; b < NB; ++b) acc[a][b] = mfma_frag(w, f[b], acc[a][b]);
       }
@@ -355,14 +334,13 @@ __device__ __forceinline__ void prefill_body(const GemmArgs& args, const GemmOpe
     }
   };
   auto epilogue = [&](int rb) __attribute__((always_inline)) {
-    prefill_epilogue<MODE, FP8, NB, W>(args, op, routed, e, r0, r1, rb, wave, lr, kq,
-                                                out_row, acc);
+    prefill_epilogue<MODE, NB>(args, e, r0, r1, rb, wave, lr, kq, out_row, acc);
   };
 
   weight_rows(rb0);
   clear();
   const int nph = nch / R;
-  const int rot = routed ? prefill_start_chunk(e, nch) / R : 0;  // whole phases: R divides 4
+  const int rot = prefill_start_chunk(e, nch) / R;  // whole phases: R divides 4
   auto phase_of = [&](int p) __attribute__((always_inline)) {  // p < nph
     p += rot;
     return p >= nph ? p - nph : p;
@@ -371,8 +349,7 @@ __device__ __forceinline__ void prefill_body(const GemmArgs& args, const GemmOpe
   issue_a(0, ph0 * R);
 #pragma unroll
   for (int i = 0; i < kLB; ++i)
-    toff[i] = (uint32_t)((trow[i] - row_base) / row_div) * (uint32_t)(op.ld_in * 2) +
-              (uint32_t)(unit * 16);
+    toff[i] = (uint32_t)(trow[i] / row_div) * (uint32_t)(op.ld_in * 2) + (uint32_t)(unit * 16);
   issue_b(0, ph0, true);
 #pragma unroll
   for (int c = 1; c < R; ++c) issue_a(c, ph0 * R + c);
@@ -390,7 +367,7 @@ __device__ __forceinline__ void prefill_body(const GemmArgs& args, const GemmOpe
     if constexpr (!RES) issue_b(stage, next, more);
 #pragma unroll
     for (int q = 0; q < R; ++q) {
-      mma(q, at + q * kSub, 2);
+      mma(q, at + q * kSub);
       issue_a(q, next * R + q);
     }
     if (sync) wait_barrier<R * kLA>();
@@ -418,10 +395,10 @@ __device__ __forceinline__ void prefill_body(const GemmArgs& args, const GemmOpe
   }
 }
 
-template <int MODE, bool FP8, int MAXB, int W, int R, bool RES>
-__global__ __launch_bounds__(64 * W)
-__attribute__((amdgpu_waves_per_eu(MAXB <= 4 ? 3 : 2))) void k_prefill_stream(GemmArgs args) {
-  extern __shared__ uint4 smem[];  // two phases of up to MAXB 16-token blocks
+template <int MODE, int R, bool RES>
+__global__ __launch_bounds__(64 * kWaves)
+__attribute__((amdgpu_waves_per_eu(2))) void k_prefill_stream(GemmArgs args) {
+  extern __shared__ uint4 smem[];  // two phases of up to kMaxBlocks 16-token blocks
 
   // XCD-aware order: workgroup b runs on XCD b % 8, so the workgroups of one tile get ids 8
   // apart (same XCD, dispatched together) and share the tile's token rows in that XCD's L2
@@ -431,54 +408,31 @@ __attribute__((amdgpu_waves_per_eu(MAXB <= 4 ? 3 : 2))) void k_prefill_stream(Ge
   const int j = blockIdx.x / kXcds;
   int tile = (j / ng) * kXcds + xcd;
   const int rb = (j - (j / ng) * ng) * args.nblk;
-  int e, r0, r1;
-  if (args.table) {
-    // nsub parts of 16 MAXB rows per table tile, all the first parts before the second ones
-    // (alternating, the parts would follow the XCDs and the rarer ones leave theirs idle)
-    const int sub = tile / args.MTgrid;
-    tile -= sub * args.MTgrid;
-    if (sub >= args.nsub) return;
-    const int ntiles = args.table[3 * args.MT];
-    if (tile >= ntiles) return;
-    if (args.shared_first > 0) {
-      // the shared expert's tiles (the table's last ones, all full: the longest workgroups)
-      // are dispatched first, the routed tiles fill in behind them
-      const int ns = min(args.shared_first, ntiles);
-      tile = tile < ns ? ntiles - ns + tile : tile - ns;
-    }
-    e = args.table[tile];
-    r0 = args.table[args.MT + tile];
-    // the table holds the expert's end row
-    r1 = min(args.table[2 * args.MT + tile], r0 + args.bm);
-    r0 += sub * 16 * MAXB;
-    r1 = min(r1, r0 + 16 * MAXB);
-  } else {
-    e = args.E;
-    r0 = args.P + tile * 16 * MAXB;
-    r1 = min(r0 + 16 * MAXB, args.P + args.T);
-  }
+  // nsub parts of kPartRows rows per table tile, all the first parts before the second ones
+  // (alternating, the parts would follow the XCDs and the rarer ones leave theirs idle)
+  const int sub = tile / args.MTgrid;
+  tile -= sub * args.MTgrid;
+  if (sub >= args.nsub || tile >= args.table[3 * args.MT]) return;
+  const int e = args.table[tile];
+  if (e >= args.E) return;  // a shared expert's tile
+  const int t0 = args.table[args.MT + tile];
+  // the table holds the expert's end row; this tile is its next tile_rows at most
+  const int t1 = min(args.table[2 * args.MT + tile], t0 + args.tile_rows);
+  const int r0 = t0 + sub * kPartRows;
+  const int r1 = min(t1, r0 + kPartRows);
   if (r0 >= r1) return;
-  const bool routed = e < args.E;
-  const GemmOperand& op = routed ? args.op[0] : args.op[1];
-  constexpr int kOut = MODE == kModeSwiglu ? 16 * W : 32 * W;  // output rows per block
-  const int nblk = min(args.nblk, (op.N + kOut - 1) / kOut - rb);
-  if (nblk <= 0) return;
+  const int nblk = min(args.nblk, args.nrb - rb);
   char* lds = reinterpret_cast<char*>(smem);
   const int nb = (r1 - r0 + 15) >> 4;
-#define NB_CASE(NB)                                                                    \
-  if (NB == MAXB || nb <= NB) {                                                        \
-    prefill_body<MODE, FP8, NB, W, R, RES>(args, op, routed, e, r0, r1, rb, nblk, lds);     \
-    return;                                                                            \
+#define NB_CASE(NB)                                                   \
+  if (NB == kMaxBlocks || nb <= NB) {                                 \
+    prefill_body<MODE, NB, R, RES>(args, e, r0, r1, rb, nblk, lds);   \
+    return;                                                           \
   }
-  if constexpr (MAXB == 4) {
-    NB_CASE(2)
-    NB_CASE(4)
-  } else {
-    NB_CASE(4)
-    NB_CASE(6)
-    NB_CASE(8)
-    NB_CASE(10)
-  }
+  NB_CASE(4)
+  NB_CASE(6)
+  NB_CASE(8)
+  NB_CASE(10)
 #undef NB_CASE
 }
 
@@ -487,7 +441,7 @@ namespace {
 // The kernel's dynamic LDS above the default limit, allowed once per device and kernel.
 hipError_t allow_lds(const void* fn, int which, int bytes) {
   static std::mutex mu;
-  static uint64_t done[32] = {};  // [kernel], bit d: device d
+  static uint64_t done[5] = {};  // [kernel], bit d: device d
   int dev = 0;
   hipError_t err = hipGetDevice(&dev);
   if (err != hipSuccess) return err;
@@ -499,12 +453,10 @@ hipError_t allow_lds(const void* fn, int which, int bytes) {
   return err;
 }
 
-template <int MODE, bool FP8, int MAXB, int W, int R, bool RES = false>
-hipError_t launch_one(GemmArgs a, int tiles, hipStream_t st) {
-  constexpr int bytes = 2 * R * MAXB * kPBlkBytes;
-  constexpr int kOut = MODE == kModeSwiglu ? 16 * W : 32 * W;
-  const int nmax = a.op[0].N > a.op[1].N ? a.op[0].N : a.op[1].N;
-  a.nrb = (nmax + kOut - 1) / kOut;
+template <int MODE, int R, bool RES>
+hipError_t launch_one(GemmArgs a, int tiles, int which, hipStream_t st) {
+  constexpr int bytes = 2 * R * kMaxBlocks * kPBlkBytes;
+  a.nrb = (a.op[0].N + kOut<MODE> - 1) / kOut<MODE>;
   // Row blocks per workgroup: down's token rows are staged once for all of them and the next
   // block's weights stream through the epilogue of one (T = 777 / 1111 / 2048 / 4096, e4m3: 75 /
   // 81 / 93 / 146 µs with 4, 77 / 82 / 96 / 132 with 2, 81 / 87 / 102 / 139 with 1). gate_up
@@ -513,27 +465,12 @@ hipError_t launch_one(GemmArgs a, int tiles, hipStream_t st) {
   const long long ng = (a.nrb + a.nblk - 1) / a.nblk;
   const long long grid = (long long)((tiles + kXcds - 1) / kXcds) * kXcds * ng;
   if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
-  const auto fn = &k_prefill_stream<MODE, FP8, MAXB, W, R, RES>;
-  const int which = (MODE * 2 + (FP8 ? 1 : 0)) * 8 + (RES ? 3 : R / 2);
+  const auto fn = &k_prefill_stream<MODE, R, RES>;
   const hipError_t err = allow_lds(reinterpret_cast<const void*>(fn), which, bytes);
   if (err != hipSuccess) return err;
-  hipLaunchKernelGGL((k_prefill_stream<MODE, FP8, MAXB, W, R, RES>), dim3((unsigned)grid), dim3(64 * W),
-                     bytes, st, a);
+  hipLaunchKernelGGL((k_prefill_stream<MODE, R, RES>), dim3((unsigned)grid), dim3(64 * kWaves), bytes,
+                     st, a);
   return hipGetLastError();
-}
-
-hipError_t launch_gate_up(const GemmArgs& a, int ring, int tiles, hipStream_t st) {
-  constexpr int L = kPBlocksLarge, M = kModeSwiglu;
-  if (ring == 2) return launch_one<M, true, L, 8, 2>(a, tiles, st);
-  return launch_one<M, true, L, 8, 4>(a, tiles, st);
-}
-
-// res: two phases hold all of K.
-hipError_t launch_down(const GemmArgs& a, int ring, bool res, int tiles, hipStream_t st) {
-  constexpr int L = kPBlocksLarge, M = kModePlain;
-  if (ring == 2) return launch_one<M, true, L, 8, 2>(a, tiles, st);
-  if (res) return launch_one<M, true, L, 8, 4, true>(a, tiles, st);
-  return launch_one<M, true, L, 8, 4>(a, tiles, st);
 }
 
 long long in_bytes(const GemmArgs& a) { return (a.op[0].in_map ? a.T : a.P) * a.op[0].ld_in * 2; }
@@ -557,16 +494,22 @@ bool prefill_stream_takes(const GemmArgs& a) {
 
 hipError_t launch_prefill_stream(int mode, const GemmArgs& a_in, int max_tiles, hipStream_t st) {
   GemmArgs a = a_in;
-  constexpr int sub = kStreamRowsLarge;
-  a.nsub = (a.bm + sub - 1) / sub;
+  a.tile_rows = prefill_tile_rows();
+  a.nsub = (a.tile_rows + kPartRows - 1) / kPartRows;
   a.MTgrid = max_tiles;
   const int tiles = max_tiles * a.nsub;
+  a.in_bytes = (unsigned)in_bytes(a);
+  a.out_bytes = (unsigned)out_bytes(a);
+  // phases of four chunks where K has whole ones, else of two; down with all of K in two phases
+  // (K = 512) keeps both in LDS
   const int K = a.op[0].K;
-  const int ring = K % (4 * kPKC) || K < 8 * kPKC ? 2 : 4;
-  a.in_bytes[0] = (unsigned)in_bytes(a);
-  a.out_bytes[0] = (unsigned)out_bytes(a);
-  return mode == kModeSwiglu ? launch_gate_up(a, ring, tiles, st)
-                             : launch_down(a, ring, K == 8 * kPKC, tiles, st);
+  const bool four = K % (4 * kPKC) == 0 && K >= 8 * kPKC;
+  if (mode == kModeSwiglu)
+    return four ? launch_one<kModeSwiglu, 4, false>(a, tiles, 0, st)
+                : launch_one<kModeSwiglu, 2, false>(a, tiles, 1, st);
+  if (!four) return launch_one<kModePlain, 2, false>(a, tiles, 2, st);
+  return K == 8 * kPKC ? launch_one<kModePlain, 4, true>(a, tiles, 3, st)
+                       : launch_one<kModePlain, 4, false>(a, tiles, 4, st);
 }
 
 }  // namespace moe
