@@ -104,7 +104,7 @@ bool decode_takes(int T, bool fp8) {
 // A grouped prefill launch with routed and shared tiles: one launch, the shared expert's
 // tiles dispatched first (grouped gate_up at C4 303-310 against 317 µs with the shared
 // tiles as a second launch on the auxiliary stream, 632 with them dispatched last);
-// MOE_PREFILL_SIDE=1 restores the second launch. (The block forward runs the whole shared
+// MOE_PREFILL_SIDE=1 restores the second launch. (The block forward mostly runs the whole shared
 // expert on the auxiliary stream from its start instead; see block_side_enabled.)
 bool prefill_side_enabled() {
   const char* env = knob(kKnobPrefillSide);
@@ -113,12 +113,15 @@ bool prefill_side_enabled() {
 
 // Block forward: the shared expert on the auxiliary stream where its tiles do not share the
 // routed launches (fp8 routed experts, the tiled ones with MOE_MIXED=0), and beside bf16 prefill
-// tiles of up to 96 rows per expert on average. Above that it goes first in the routed
-// launches: the two hops between queues cost more than the overlap with the router gains
-// (T = 4096: 502 against 509 µs).
+// tiles, except from 96 to 128 rows per expert on average, where it goes first in the routed
+// launches. In the routed launches / beside them, µs per block at 2048 / 2560 / 3072 / 3584 / 4096 /
+// 5120 / 6144 / 8192 / 16384 tokens: uniform routing 407 / 435 / 452 / 478 / 500 / 571 / 642 / 883 /
+// 1603 against 407 / 434 / 453 / 481 / 506 / 560 / 633 / 865 / 1608; Zipf(1.1) 456 / 490 / 527 / 558 /
+// 594 / 673 / 737 / 908 / 1597 against 451 / 487 / 538 / 561 / 592 / 666 / 729 / 889 / 1589. (Beside them it
+// overlaps the router and fills the gaps of the routed rounds, but costs two hops between queues.)
 bool block_side_enabled(bool fp8, int bm, long long P, int E) {
-  const bool prefill = bm == prefill_tile_rows();
-  return (fp8 && !mixed_enabled()) || (prefill && (fp8 || P <= 96LL * E));
+  if (bm != prefill_tile_rows()) return fp8 && !mixed_enabled();
+  return fp8 || P <= 96LL * E || P > 128LL * E;
 }
 
 size_t align256(size_t n) { return (n + 255) & ~size_t(255); }

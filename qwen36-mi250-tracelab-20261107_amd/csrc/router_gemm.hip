@@ -344,8 +344,10 @@ bool router_gemm_fits(int H, int n_pack) { return H % (32 * kRouterSplit) == 0 &
 // one workgroup) is the slower choice: at 16 tokens 7.8 + 10.6 µs against 4.8 + 5.0 + 4.8.
 // Measured per layer (8 layers cycled, uniform routing): 17 / 32 / 64 / 128 / 256 tokens
 // 154.0 / 207.8 / 263.9 / 297.8 / 318.9 µs against 155.4 / 209.8 / 265.6 / 298.8 / 320.6
-// with k_router_gemm then k_route; level at 512 tokens (372.8 against 371.9), slower at 767
-// (390.1 against 386.2); an eager call of 300 tokens 340.8 against 346.2. At C3 the router launch
+// with k_router_gemm then k_route; slower at 767 (390.1 against 386.2). A block of 300 / 350 / 384 /
+// 400 / 450 / 512 tokens: bf16 350 / 359 / 366 / 373 / 386 / 401 against 355 / 364 / 370 / 373 / 385 /
+// 400, Zipf(1.1) 347 / 367 / 380 / 388 / 405 / 423 against 351 / 372 / 383 / 388 / 404 / 423, e4m3 230 /
+// 236 / 243 / 248 / 258 / 268 against 235 / 241 / 246 / 248 / 256 / 267. At C3 the router launch
 // takes 4.8 µs against 7.7.
 bool router_part_takes(int T, int H, int n_pack) {
   const int nst = H / (32 * kRouterSplit);
