@@ -55,14 +55,18 @@ bool mixed_enabled();
 hipError_t launch_expert_gemm(int mode, int role, int bm, const GemmArgs& a, int max_tiles,
                               hipStream_t st);
 
-// Where the prefill kernels start their walk over the nch = K / 64 chunks of expert e's weight
-// rows (it wraps around). Workgroups run nearly in step, and weight rows lie a power of two
-// apart: all reading the same columns at once keeps few memory channels busy (a bf16 block of
-// 1111 / 2048 tokens: 379 / 413 us against 410 / 442 with one start for all). The start
-// is the weights' own and the same in every kernel that runs a projection, so that a row's
-// result does not depend on its batch.
-__host__ __device__ inline int prefill_start_chunk(int e, int nch) {
-  return nch % 4 ? 0 : e % (nch / 4) * 4;
+// Where the prefill kernels (bf16: gate_up's; e4m3: both projections') start their walk over the
+// nch = K / 64 chunks of expert e's weight rows of row_bytes (it wraps around). Workgroups run nearly
+// in step, and the rows of the model lie 4 KiB apart: all reading the same columns at once keeps
+// few memory channels busy. Start by expert / one start for all, a block's µs: bf16, K = 2048 at 64 /
+// 128 experts and 700 tokens 144 / 225 against 158 / 246, K = 4096 252 / 398 against 277 / 433; e4m3,
+// K = 4096 206 / 308 against 219 / 336. Shorter rows gain nothing (bf16 K = 1536 182 / 182, e4m3
+// K = 2048 286 / 286) or lose, since the experts then read a token's columns at different times (bf16
+// K = 1024 at 64 / 256 experts 101 / 219 against 98 / 209). The start is the expert's own and, for one
+// weight type, the same in every kernel that runs the projection above 512 tokens, so that a row's result
+// does not depend on its batch there; whole groups of four chunks, the streaming kernel's phases.
+__host__ __device__ inline int prefill_start_chunk(int e, int nch, long long row_bytes) {
+  return row_bytes < 4096 || nch % 4 ? 0 : e % (nch / 4) * 4;
 }
 
 // Prefill batches. launch_prefill_gemm (prefill_gemm.hip) takes tables of prefill_tile_rows()

@@ -183,7 +183,7 @@ __global__ __launch_bounds__(kThreads, 1) void k_prefill_gemm(GemmArgs args) {
   // a last half chunk holds its 32 k twice (so that no load runs past a row) and is multiplied once
   const bool half = TAIL && op.K % DKC != 0;
   const int nd = TAIL ? (op.K + DKC - 1) / DKC : op.K / DKC;
-  const int rot = MODE == kModeSwiglu && routed && !half ? prefill_start_chunk(e, nd) : 0;
+  const int rot = MODE == kModeSwiglu && routed && !half ? prefill_start_chunk(e, nd, op.ldw * 2) : 0;
   auto chunk = [&](int d) { return d + rot < nd ? d + rot : d + rot - nd; };
   auto koff = [&](int d) { return d * DKC - (half && d == nd - 1 && unit >= 4 ? PKC : 0); };
   auto issue_a = [&](int d) {
@@ -320,9 +320,8 @@ __global__ __launch_bounds__(kThreads, 1) void k_prefill_gemm(GemmArgs args) {
 // non-temporal one measured slower here (gate_up / down at 4096 tokens 261 / 189 against
 // 248 / 181 µs). Each weight byte costs LDS traffic and barriers that the streaming form does
 // not have, but serves 256 rows instead of 160: at 32768 tokens (1024 rows per expert) gate_up
-// takes 1146 µs (0.96 PFLOP/s) against 1505. The walk over K starts by expert
-// (prefill_start_chunk), as the streaming form's: gate_up / down at 8192 tokens 346 / 271 µs against
-// 370 / 282 with one start for all.
+// takes 1146 µs (0.96 PFLOP/s) against 1505. With the streaming form's epilogue (silu_fast, packed
+// conversions) gate_up / down at 8192 tokens take 346 / 271 µs against 370 / 282 with siluf_ and rbf.
 //
 // The chunk's k order is permuted the same way in both operands (the same products are
 // summed): lane group kq reads weight unit kq (16 e4m3 bytes, one ds_read_b128) once per
@@ -442,7 +441,7 @@ __global__ __launch_bounds__(kThreads, 1) void k_prefill_gemm_f8(GemmArgs args) 
   char* lds = reinterpret_cast<char*>(smem);
   char* bring_lds = lds + F8StagesA * F8Stage;
   const int nd = op.K / DKC;
-  const int rot = prefill_start_chunk(e, nd);
+  const int rot = prefill_start_chunk(e, nd, op.ldw);
   auto chunk = [&](int d) { return d + rot < nd ? d + rot : d + rot - nd; };
   auto issue_a = [&](int d) {
     char* st = lds + (d % F8StagesA) * F8Stage;

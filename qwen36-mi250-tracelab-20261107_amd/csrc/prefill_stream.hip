@@ -340,7 +340,7 @@ __device__ __forceinline__ void prefill_body(const GemmArgs& args, int e, int r0
   weight_rows(rb0);
   clear();
   const int nph = nch / R;
-  const int rot = prefill_start_chunk(e, nch) / R;  // whole phases: R divides 4
+  const int rot = prefill_start_chunk(e, nch, op.ldw) / R;  // whole phases: R divides 4
   auto phase_of = [&](int p) __attribute__((always_inline)) {  // p < nph
     p += rot;
     return p >= nph ? p - nph : p;
