@@ -349,10 +349,16 @@ bool router_gemm_fits(int H, int n_pack) { return H % (32 * kRouterSplit) == 0 &
 // 400, Zipf(1.1) 347 / 367 / 380 / 388 / 405 / 423 against 351 / 372 / 383 / 388 / 404 / 423, e4m3 230 /
 // 236 / 243 / 248 / 258 / 268 against 235 / 241 / 246 / 248 / 256 / 267. At C3 the router launch
 // takes 4.8 µs against 7.7.
+// A wide router of short rows fills the split kernel by itself: up to 8 tokens one launch fewer is
+// the faster choice there (K quarters / split kernel, a block of 5 and 8 tokens, µs: H = 512 at 256
+// experts 29.0, 31.0 / 28.1, 30.0; 1024 at 256 38.9, 49.1 / 38.0, 48.3; 2048 at 512 99.6, 123.4 / 98.3,
+// 121.8; but 2048 at 256 80.4, 100.1 / 81.1, 101.1; 1024 at 160 52.1, 65.0 / 52.1, 66.8; 512 at 128
+// 32.4, 36.4 / 33.1, 37.6; at 12 tokens K quarters gain in all but the third, which loses 0.7 %).
 bool router_part_takes(int T, int H, int n_pack) {
   const int nst = H / (32 * kRouterSplit);
-  return router_gemm_fits(H, n_pack) && (nst == 4 || nst == 8 || nst == 16) && T > 4 &&
-         T <= 384;
+  const bool wide = n_pack > 176 && H < 7 * n_pack;
+  return router_gemm_fits(H, n_pack) && (nst == 4 || nst == 8 || nst == 16) &&
+         T > (wide ? 8 : 4) && T <= 384;
 }
 
 hipError_t launch_router_part(const void* x, int T, int H, const void* w_pack, int n_pack,

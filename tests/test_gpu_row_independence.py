@@ -59,6 +59,24 @@ def test_leading_rows_match_smaller_batch(pkg, dev, mlp, big, small, decode):
         assert torch.equal(a[:small], b)
 
 
+@pytest.mark.parametrize("H,E", [(512, 256), (1024, 256), (512, 16)])
+def test_leading_rows_match_across_router_kernels(pkg, dev, H, E):
+    """Routers of other widths take the split kernel up to 4 or, wide ones of short rows, 8 tokens and
+    K quarters above: the same logits and outputs, bit for bit, on both sides (decode=True: without
+    it the products' rounding changes above 16 tokens)."""
+    print(f"row independence across router kernels H={H} E={E}", flush=True)
+    import __graft_entry__
+
+    mlp = __graft_entry__._mlp_from_weights(orc.make_weights(H, E, 128, 128, seed=7), dev)
+    x = torch.randn(20, H, generator=torch.Generator().manual_seed(H + E)).to(BF16).to(dev)
+    a, ia, wa, la = pkg.block.moe(x, mlp, 8, decode=True, return_routing=True)
+    for n in (16, 9, 8, 5):
+        b, ib, wb, lb = pkg.block.moe(x[:n].contiguous(), mlp, 8, decode=True, return_routing=True)
+        torch.cuda.synchronize()
+        assert torch.equal(la[:n], lb) and torch.equal(ia[:n], ib) and torch.equal(wa[:n], wb)
+        assert torch.equal(a[:n], b)
+
+
 @pytest.mark.parametrize("big,small", [(1024, 600), (1100, 900), (4096, 2048), (6000, 4096),
                                        (8192, 5000), (132000, 4096)])
 def test_leading_rows_match_smaller_batch_fp8_prefill(pkg, dev, big, small):
