@@ -113,15 +113,17 @@ bool prefill_side_enabled() {
 
 // Block forward: the shared expert on the auxiliary stream where its tiles do not share the
 // routed launches (fp8 routed experts, the tiled ones with MOE_MIXED=0), and beside bf16 prefill
-// tiles, except from 96 to 128 rows per expert on average, where it goes first in the routed
-// launches. In the routed launches / beside them, µs per block at 2048 / 2560 / 3072 / 3584 / 4096 /
-// 5120 / 6144 / 8192 / 16384 tokens: uniform routing 407 / 435 / 452 / 478 / 500 / 571 / 642 / 883 /
-// 1603 against 407 / 434 / 453 / 481 / 506 / 560 / 633 / 865 / 1608; Zipf(1.1) 456 / 490 / 527 / 558 /
-// 594 / 673 / 737 / 908 / 1597 against 451 / 487 / 538 / 561 / 592 / 666 / 729 / 889 / 1589. (Beside them it
-// overlaps the router and fills the gaps of the routed rounds, but costs two hops between queues.)
+// tiles, except with 256 experts and more at 96 to 128 rows per expert on average, where it goes
+// first in the routed launches. In the routed launches / beside them, µs per block, at 2048 / 2560 /
+// 3072 / 3584 / 4096 / 5120 / 6144 / 8192 / 16384 tokens (H = 2048, I = 512, E = 256): uniform routing
+// 407 / 435 / 452 / 478 / 500 / 571 / 642 / 883 / 1603 against 407 / 434 / 453 / 481 / 506 / 560 / 633 /
+// 865 / 1608; Zipf(1.1) 456 / 490 / 527 / 558 / 594 / 673 / 737 / 908 / 1597 against 451 / 487 / 538 / 561 /
+// 592 / 666 / 729 / 889 / 1589. With fewer experts at 112 rows each it loses: H = 2048 at 64 / 128 experts
+// 176 / 266 against 170 / 260; 256 at H = 1024 / 4096 273 / 836 against 281 / 852. (Beside them it overlaps
+// the router and fills the gaps of the routed rounds, but costs two hops between queues.)
 bool block_side_enabled(bool fp8, int bm, long long P, int E) {
   if (bm != prefill_tile_rows()) return fp8 && !mixed_enabled();
-  return fp8 || P <= 96LL * E || P > 128LL * E;
+  return fp8 || E < 256 || P <= 96LL * E || P > 128LL * E;
 }
 
 size_t align256(size_t n) { return (n + 255) & ~size_t(255); }
