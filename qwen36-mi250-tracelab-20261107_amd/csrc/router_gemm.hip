@@ -353,10 +353,12 @@ bool router_gemm_fits(int H, int n_pack) { return H % (32 * kRouterSplit) == 0 &
 // the faster choice there (K quarters / split kernel, a block of 5 and 8 tokens, µs: H = 512 at 256
 // experts 29.0, 31.0 / 28.1, 30.0; 1024 at 256 38.9, 49.1 / 38.0, 48.3; 2048 at 512 99.6, 123.4 / 98.3,
 // 121.8; but 2048 at 256 80.4, 100.1 / 81.1, 101.1; 1024 at 160 52.1, 65.0 / 52.1, 66.8; 512 at 128
-// 32.4, 36.4 / 33.1, 37.6; at 12 tokens K quarters gain in all but the third, which loses 0.7 %).
+// 32.4, 36.4 / 33.1, 37.6; at 12 tokens K quarters gain in all but the third, which loses 0.7 %.
+// A replayed layer with add + RMSNorm: 2048 at 256 78.1, 100.6 / 79.0, 101.7 bf16, 63.2, 77.3 / 64.6,
+// 78.9 e4m3; 1024 at 160 55.4, 67.7 / 55.7, 70.6; 512 at 256 45.9, 52.8 / 44.8, 51.3).
 bool router_part_takes(int T, int H, int n_pack) {
   const int nst = H / (32 * kRouterSplit);
-  const bool wide = n_pack > 176 && H < 7 * n_pack;
+  const bool wide = n_pack > 192 && H < 4 * n_pack;  // rows are packed to a multiple of 64
   return router_gemm_fits(H, n_pack) && (nst == 4 || nst == 8 || nst == 16) &&
          T > (wide ? 8 : 4) && T <= 384;
 }
