@@ -120,6 +120,39 @@ def test_decode_experts_forward(pkg, dev, n, mode, shape):
     assert max_abs(got, tiled) <= 8e-3 * scale
 
 
+@pytest.mark.parametrize("k", [15, 16, 17, 31, 32])
+@pytest.mark.parametrize("I,fp8", [(512, False), (1024, False), (1024, True)])
+def test_decode_down_many_experts(pkg, dev, k, I, fp8):
+    """One token of many experts (down's wave counts, its one-token kernel up to k = 15) and two
+    tokens of them: the same dot products in the same order, so the same bits."""
+    _say("decode down", k, I, fp8)
+    E, H = 64, 512
+    g = torch.Generator().manual_seed(k + I)
+    dn = (torch.randn(E, H, I, generator=g) * 0.05).to(BF16).to(dev)
+    dn, scale = pkg.fp8.quantize_rows(dn) if fp8 else (dn, None)
+
+    def rows(*shape):
+        return torch.randn(1, *shape, generator=g).to(BF16).to(dev)
+
+    act, wts, act_sh, logits, res = rows(k, I), rows(k), rows(1024), rows(128), rows(H)
+    sh = rows(H, 1024)[0]
+    idx = torch.randperm(E, generator=g)[:k][None].to(dev)
+    out = [pkg.ops.decode_down(torch.cat([act] * T).reshape(T * k, I), T, k, dn,
+                               idx.repeat(T, 1), wts.repeat(T, 1), scale=scale,
+                               shared=(sh, act_sh.repeat(T, 1)), logits=logits.repeat(T, 1),
+                               experts=E, residual=res.repeat(T, 1)) for T in (1, 2)]
+    torch.cuda.synchronize()
+    assert torch.equal(out[1][:1], out[0]) and torch.equal(out[1][1:], out[0])
+    ref = orc.dequantize_rows(dn.cpu(), scale.cpu()) if fp8 else dn.cpu()
+    y = torch.einsum("jhi,ji->jh", ref.double()[idx[0].cpu()], act[0].double().cpu())
+    ysh = act_sh.double().cpu() @ sh.double().cpu().T
+    gate = torch.sigmoid(logits[:, E:E + 1].double().cpu())
+    want = (wts.double().cpu() @ y + gate * ysh + res.double().cpu())
+    # per term: bf16 roundings of y and w y (2^-8 each), then of the sum, gate, gated term, sums
+    terms = (wts.double().cpu().abs() @ y.abs() + gate * ysh.abs() + res.double().cpu().abs())
+    assert ((out[0].double().cpu() - want).abs() <= 6 * 2.0**-8 * terms).all()
+
+
 @pytest.mark.parametrize("T", [1, 2, 3, 4])
 def test_decode_fp8_block(pkg, dev, layer, T):
     """fp8-e4m3 routed experts on the decode path against the dequantised fp32 oracle and
