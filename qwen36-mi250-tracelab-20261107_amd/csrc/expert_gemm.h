@@ -65,8 +65,11 @@ hipError_t launch_expert_gemm(int mode, int role, int bm, const GemmArgs& a, int
 // K = 1024 at 64 / 256 experts 101 / 219 against 98 / 209). The start is the expert's own and, for one
 // weight type, the same in every kernel that runs the projection above 512 tokens, so that a row's result
 // does not depend on its batch there; whole groups of four chunks, the streaming kernel's phases.
+__host__ __device__ inline bool prefill_starts_by_expert(int nch, long long row_bytes) {
+  return row_bytes >= 4096 && nch % 4 == 0;
+}
 __host__ __device__ inline int prefill_start_chunk(int e, int nch, long long row_bytes) {
-  return row_bytes < 4096 || nch % 4 ? 0 : e % (nch / 4) * 4;
+  return prefill_starts_by_expert(nch, row_bytes) ? e % (nch / 4) * 4 : 0;
 }
 
 // Prefill batches. launch_prefill_gemm (prefill_gemm.hip) takes tables of prefill_tile_rows()
