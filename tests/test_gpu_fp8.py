@@ -74,9 +74,9 @@ def test_fp8_experts_match_dequantised_oracle(pkg, dev, n):
 @pytest.mark.parametrize("mode", ["uniform", "skewed", "one"])
 @pytest.mark.parametrize("shape", [(32, 256, 128, 8), (16, 2048, 1024, 4)])
 def test_fp8_prefill_tiles_match_dequantised_oracle(pkg, dev, n, mode, shape):
-    """More than 512 tokens with e4m3 experts: the prefill kernel's fp8 form (64-k DMA
-    chunks, 256-row table tiles; experts of more than 256 rows span several tiles in the
-    skewed and one-expert modes) against the fp32 oracle on the dequantised weights, at a
+    """More than 512 tokens with e4m3 experts and more than 128 rows per expert on average: the
+    staged prefill kernel's e4m3 form (64-k DMA chunks, 256-row table tiles; experts of more than
+    256 rows span several tiles in the skewed and one-expert modes) against the fp32 oracle on the dequantised weights, at a
     small shape and at the model's hidden size with a doubled intermediate; run twice,
     bit-identical."""
     e, h, i, k = shape
