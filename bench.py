@@ -545,7 +545,10 @@ KERNEL_STATS_FILES = {"c2": ("moe_layer_c2_decode_b1_kernels",
                               "C5: 40-layer stack, fp8-e4m3 routed experts, batch 32"),
                        "c4f8": ("moe_layer_c4f8_prefill_4096_fp8_kernels",
                                 "C4's 4096-token prefill chunk with fp8-e4m3 routed experts "
-                                "(not a BASELINE config), 4 layers cycled")}
+                                "(not a BASELINE config), 4 layers cycled"),
+                       "c2,batches": ("moe_layer_batches_kernels",
+                                      "C2 and decode steps of 2, 4, 8 and 16 tokens, bf16 and "
+                                      "fp8-e4m3 experts, 8 layers cycled")}
 
 
 def kernel_stats_summary(prof_dir, config):
