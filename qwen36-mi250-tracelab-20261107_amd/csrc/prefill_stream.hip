@@ -59,6 +59,7 @@ constexpr int kPBlkBytes = 16 * kPRowBytes;      // a 16-token block of a stage:
 template <int MODE>
 constexpr int kStorePolicy = MODE == kModeSwiglu ? 16 : 0;
 constexpr int kXcds = 8;            // XCDs of an MI355X (round-robin dispatch)
+constexpr int kCus = 256;
 constexpr int kWaves = 8;
 constexpr int kMaxBlocks = 10;                   // 16-token blocks of a part of a tile
 constexpr int kPartRows = 16 * kMaxBlocks;
@@ -461,7 +462,16 @@ hipError_t launch_one(GemmArgs a, int tiles, int which, hipStream_t st) {
   // block's weights stream through the epilogue of one (T = 777 / 1111 / 2048 / 4096, e4m3: 75 /
   // 81 / 93 / 146 µs with 4, 77 / 82 / 96 / 132 with 2, 81 / 87 / 102 / 139 with 1). gate_up
   // gains nothing that the coarser work units do not cost (144 / 206 against 138 / 223 with 2).
-  a.nblk = MODE == kModePlain ? 2 : 1;
+  // One block per workgroup where two, at a tile per expert, would leave the last of their
+  // rounds over the chip a fifth or more idle (16 experts of 2048 x 1408, 88 rows each, 45 µs with 2
+  // and 26 with 1; 64 of 3072 x 1536 at 48 rows 1.10 and 1.03 of the staged kernel's time). Not so
+  // with a short K where one round of two fills half the chip and more: a block's other launches use
+  // the rest (2 / 1 blocks, 520 and 1000 tokens: 32 experts of 2048 x 512, top-4, 105, 121 / 115, 127 µs;
+  // 16 of 4096 x 512, top-2, 153, 159 / 158, 173; 85 of 768 x 512 89, 96 / 91, 97; but 128 of 512 x 512
+  // 91, 100 / 89, 96).
+  const long long two = (long long)a.E * ((a.nrb + 1) / 2), one = (long long)a.E * a.nrb;
+  const bool idle = 8 * ((two + kCus - 1) / kCus) > 5 * ((one + kCus - 1) / kCus);
+  a.nblk = MODE == kModePlain && (!idle || (RES && two >= kCus / 2 && two <= kCus)) ? 2 : 1;
   const long long ng = (a.nrb + a.nblk - 1) / a.nblk;
   const long long grid = (long long)((tiles + kXcds - 1) / kXcds) * kXcds * ng;
   if (grid > 0x7fffffffLL) return hipErrorInvalidValue;

@@ -2,7 +2,8 @@
 tiles: every 16-token block count they are compiled for with the rows one below, at and one
 above a block boundary, parts of a larger table tile, each ring depth of the streaming kernel (K
 of 256, 384, 512, 768 and 1024), the K that the staged e4m3 kernel takes instead (64, 128, 192) and
-experts without rows; above 128 rows per expert on average the staged e4m3 kernel alone.
+experts without rows; above 128 rows per expert on average the staged e4m3 kernel alone; down with
+one and with two row blocks per workgroup.
 
 Tolerance: the results are bf16 roundings of fp32 sums of K bf16 products; the reference sums
 in float64 and rounds at the same points, so a rounded value differs by one bf16 ulp (at most
@@ -67,7 +68,7 @@ MANY = [0, 255, 256, 257, 511, 512, 513, 1, 272, 290]
 
 
 SHAPES = [(256, 128, True), (256, 384, True), (768, 128, True), (1024, 256, True), (512, 512, True),
-          (512, 128, False), (768, 256, False), (256, 128, False)]
+          (256, 1024, True), (512, 128, False), (768, 256, False), (256, 128, False)]
 # hidden sizes that the whole call takes on 64-row tiles
 GROUPED_ONLY = [(64, 128, True), (192, 128, True)]
 
@@ -114,6 +115,35 @@ def test_prefill_stream_tiles(pkg, H, I, fp8, counts, bm):
     got_y = pkg.ops.grouped_down(act[order].to(BF16).to(dev), T, 1, dn, sp, dns)
     torch.cuda.synchronize()
     _close(got_y, _bf(y), 2.0**-7)
+
+
+@pytest.mark.parametrize("K", [256, 512, 640, 1024])
+@pytest.mark.parametrize("E,H", [(130, 512), (100, 768), (64, 1056)])
+def test_prefill_stream_down_row_blocks(pkg, E, H, K):
+    """e4m3 down with enough experts for two row blocks per workgroup, whole pairs of blocks, an odd
+    block (H = 768) and a partial last one (1056), for each form of the walk over K (two phases in
+    LDS: 512)."""
+    print(f"prefill stream down row blocks E={E} H={H} K={K}", flush=True)
+    dev = torch.device("cuda")
+    counts = [(SMALL + LARGE)[e % 32] for e in range(E)]
+    T = sum(counts)
+    assert 32 * E <= T <= 128 * E
+    g = torch.Generator(device=dev).manual_seed(E + K)
+    w = (torch.randn(E, H, K, generator=g, device=dev) * 100).clamp(-448, 448).to(torch.float8_e4m3fn)
+    scale = torch.rand(E, H, generator=g, device=dev) * 4e-4
+    act = torch.randn(T, K, generator=g, device=dev).to(BF16)
+    idx = _routing(counts, 1).to(dev)
+    sp = pkg.ops.sort_pairs(idx, E, bm=256)
+    got = pkg.ops.grouped_down(act, T, 1, w, sp, scale)
+    order = sp.order.long()
+    want = torch.empty(T, H, dtype=torch.float64, device=dev)
+    r = 0
+    for e in range(E):
+        rows = slice(r, r + counts[e])
+        want[order[rows]] = act[rows].double() @ (w[e].double() * scale[e].double()[:, None]).T
+        r += counts[e]
+    torch.cuda.synchronize()
+    _close(got, _bf(want).cpu(), 2.0**-7)
 
 
 @pytest.mark.parametrize("K", [32, 96, 160, 224])
