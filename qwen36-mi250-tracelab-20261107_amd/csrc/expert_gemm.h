@@ -84,8 +84,21 @@ hipError_t launch_prefill_gemm(int mode, const GemmArgs& a, int max_tiles, hipSt
 // E = 256, top-8) of 3072 / 3584 / 4096 / 4608 / 5120 tokens, streaming against staged, µs: uniform
 // routing 369 / 397 / 440 / 498 / 591 against 403 / 435 / 464 / 491 / 519; Zipf(1.1) routing
 // 462 / 489 / 547 / 600 / 631 against 467 / 488 / 518 / 563 / 591.
+// With few rows per expert the staged kernel is the faster one again, except for down with K up to 512.
+// The line is 16 to 24 rows (N / 32) for gate_up where K is a power of two, else K / 32 (at most 96), and
+// K / 32 for down:
+// streaming / staged, µs, uniform routing, 256 experts at 8 / 16 / 24 / 32 / 48 rows each. gate_up of hidden x
+// intermediate 2048 x 512 133 / 134 / 135 / 135 / 138 against 121 / 127 / 137 / 140 / 154, 4096 x 1024 452 / 456 /
+// 457 / 462 / 475 against 403 / 424 / 448 / 467 / 506, 3072 x 512 191 / 193 / 196 / 198 / 203 against 172 / 177 / 183 /
+// 187 / 206 (64 / 100 rows 212 / 239 against 217 / 259); down of 2048 x 512 76 / 82 / 87 / 89 / 89 against 88 / 91 /
+// 99 / 104 / 120, 2048 x 1024 139 / 140 / 145 / 148 / 146 against 136 / 142 / 152 / 160 / 171, 4096 x 1024 282 / 303 /
+// 311 / 317 / 323 against 257 / 270 / 290 / 307 / 334, 2048 x 1536 200 / 208 / 203 / 222 / 227 against 184 / 191 / 201 /
+// 211 / 226. Over 1359 shapes and batches (hidden 256 to 7168, intermediate 256 to 2048, 16 to 512 experts, 8 to
+// 100 rows) the projections so chosen take 0.958 and 0.906 of the staged kernel's time. (16, not 20: at 18 and 20
+// rows a block of the model takes 271 / 272 against 272 / 276 beside its other launches, with Zipf(1.1)
+// routing 289 / 291 against 291 / 298.)
 constexpr int kStreamRowsPerExpert = 128;
-bool prefill_stream_takes(const GemmArgs& a);
+bool prefill_stream_takes(int mode, const GemmArgs& a);
 hipError_t launch_prefill_stream(int mode, const GemmArgs& a, int max_tiles, hipStream_t st);
 
 }  // namespace moe

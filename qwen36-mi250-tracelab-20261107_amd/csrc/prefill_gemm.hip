@@ -619,7 +619,7 @@ hipError_t launch_prefill_gemm(int mode, const GemmArgs& a_in, int max_tiles, hi
   if (f8) {
     // e4m3 weights are the routed experts' only
     if (has1 || !a.table) return hipErrorInvalidValue;
-    if (prefill_stream_takes(a)) return launch_prefill_stream(mode, a, max_tiles, st);
+    if (prefill_stream_takes(mode, a)) return launch_prefill_stream(mode, a, max_tiles, st);
   }
   a.shared_first = 0;
   if (a.table && has0 && has1) {

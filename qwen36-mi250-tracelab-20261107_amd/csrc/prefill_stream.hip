@@ -488,18 +488,25 @@ long long out_bytes(const GemmArgs& a) { return a.P * a.op[0].ld_out * 2; }
 
 }  // namespace
 
-// K in whole phases, at least two per block; 32-bit offsets into the tensors; and few enough rows.
+// K in whole phases, at least two per block; 32-bit offsets into the tensors; and a number of rows
+// per expert between the lines at which the staged kernel is the faster one.
 // For other K (64, 128 and odd multiples of 64) and tensors past 4 GiB (down's from 131072 tokens
 // of the model) a form of this kernel with one chunk in flight measured slower than the staged
 // kernel: down at 777 tokens, K = 320 / 576, 85 / 138 against 75 / 103 µs; gate_up at 4096 tokens,
 // K = 128, 45 against 42; the experts at 140000 tokens 12.8 against 9.6 ms.
-bool prefill_stream_takes(const GemmArgs& a) {
+bool prefill_stream_takes(int mode, const GemmArgs& a) {
   const GemmOperand& o = a.op[0];
   if (o.K % (2 * kPKC) || o.K < 4 * kPKC) return false;
   if (in_bytes(a) > 0xffffff00LL || out_bytes(a) > 0xffffff00LL ||
       (long long)o.N * o.ldw * 2 > 0x7fffffffLL)
     return false;
-  return a.P <= (long long)kStreamRowsPerExpert * a.E;
+  const auto at_most = [](int v, int most) { return v < most ? v : most; };
+  long long least;
+  if (mode == kModeSwiglu)
+    least = o.K & (o.K - 1) ? at_most(o.K / 32, 96) : o.N <= 512 ? 16 : at_most(o.N / 32, 24);
+  else
+    least = o.K <= 512 ? 0 : o.K / 32;
+  return a.P >= least * a.E && a.P <= (long long)kStreamRowsPerExpert * a.E;
 }
 
 hipError_t launch_prefill_stream(int mode, const GemmArgs& a_in, int max_tiles, hipStream_t st) {

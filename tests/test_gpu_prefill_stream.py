@@ -2,8 +2,9 @@
 tiles: every 16-token block count they are compiled for with the rows one below, at and one
 above a block boundary, parts of a larger table tile, each ring depth of the streaming kernel (K
 of 256, 384, 512, 768 and 1024), the K that the staged e4m3 kernel takes instead (64, 128, 192) and
-experts without rows; above 128 rows per expert on average the staged e4m3 kernel alone; down with
-one and with two row blocks per workgroup.
+experts without rows; above 128 rows per expert on average, and for gate_up below 16 to 24 (K / 32
+where K is no power of two) and down below K / 32 (K above 512), the staged e4m3 kernel; down with one and
+with two row blocks per workgroup.
 
 Tolerance: the results are bf16 roundings of fp32 sums of K bf16 products; the reference sums
 in float64 and rounds at the same points, so a rounded value differs by one bf16 ulp (at most
@@ -65,6 +66,8 @@ LARGE = [0, 79, 80, 81, 95, 96, 97, 127, 128, 129, 159, 160, 161, 3, 320, 63]
 
 # more than 128 rows per expert on average: edges of whole 256-row tiles and of the last one
 MANY = [0, 255, 256, 257, 511, 512, 513, 1, 272, 290]
+# fewer than 16 rows per expert on average
+FEW = [0, 1, 2, 5, 15, 16, 17, 31, 3, 33, 0, 0, 7, 1, 0, 0]
 
 
 SHAPES = [(256, 128, True), (256, 384, True), (768, 128, True), (1024, 256, True), (512, 512, True),
@@ -75,7 +78,7 @@ GROUPED_ONLY = [(64, 128, True), (192, 128, True)]
 
 @pytest.mark.parametrize("H,I,fp8,counts,bm", [
     (*shape, counts, bm) for bm in (256, None) for shape in SHAPES + (GROUPED_ONLY if bm else [])
-    for counts in (SMALL, LARGE, MANY)])
+    for counts in (SMALL, LARGE, MANY) + ((FEW,) if bm else ())])
 def test_prefill_stream_tiles(pkg, H, I, fp8, counts, bm):
     """bm None: the whole routed-experts call with its own tile size (more than 512 tokens);
     256: the grouped operations on a table of 256-row tiles."""

@@ -78,15 +78,16 @@ def test_leading_rows_match_across_router_kernels(pkg, dev, H, E):
         assert torch.equal(a[:n], b)
 
 
-@pytest.mark.parametrize("big,small", [(1024, 600), (1100, 900), (4096, 2048), (6000, 4096),
-                                       (8192, 5000), (132000, 4096)])
-def test_leading_rows_match_smaller_batch_fp8_prefill(pkg, dev, big, small):
+@pytest.mark.parametrize("big,small,I", [(1024, 600, 512), (1100, 900, 512), (4096, 2048, 512),
+                                         (6000, 4096, 512), (8192, 5000, 512), (132000, 4096, 512),
+                                         (1100, 900, 1024), (1024, 600, 1024)])
+def test_leading_rows_match_smaller_batch_fp8_prefill(pkg, dev, big, small, I):
     """The e4m3 prefill kernels: a row's bits do not depend on the batch either where its rows
     fall into another part or block count of a tile, where the batch takes the other kernel (above
-    128 rows per expert on average: 4096 tokens), or where the outputs of the experts are past
-    4 GiB (131072 tokens)."""
-    print(f"fp8 row independence {big} -> {small}", flush=True)
-    E, H, I, k = 256, 2048, 512, 8
+    128 rows per expert on average: 4096 tokens; with an intermediate of 1024 down below 32, 1024
+    tokens, and gate_up below 24), or where the outputs of the experts are past 4 GiB (131072 tokens)."""
+    print(f"fp8 row independence {big} -> {small} I={I}", flush=True)
+    E, H, k = 256, 2048, 8
     g = torch.Generator(device=dev).manual_seed(big + small)
 
     def weight(*shape):
