@@ -94,7 +94,7 @@ hipError_t launch_prefill_gemm(int mode, const GemmArgs& a, int max_tiles, hipSt
 // 99 / 104 / 120, 2048 x 1024 139 / 140 / 145 / 148 / 146 against 136 / 142 / 152 / 160 / 171, 4096 x 1024 282 / 303 /
 // 311 / 317 / 323 against 257 / 270 / 290 / 307 / 334, 2048 x 1536 200 / 208 / 203 / 222 / 227 against 184 / 191 / 201 /
 // 211 / 226. Over 1359 shapes and batches (hidden 256 to 7168, intermediate 256 to 2048, 16 to 512 experts, 8 to
-// 100 rows) the projections so chosen take 0.958 and 0.906 of the staged kernel's time. (16, not 20: at 18 and 20
+// 100 rows) the projections so chosen take 0.957 and 0.906 of the staged kernel's time. (16, not 20: at 18 and 20
 // rows a block of the model takes 271 / 272 against 272 / 276 beside its other launches, with Zipf(1.1)
 // routing 289 / 291 against 291 / 298.)
 constexpr int kStreamRowsPerExpert = 128;
